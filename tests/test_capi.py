@@ -87,3 +87,39 @@ def test_ndfield_roundtrip(tmp_path):
     b, meta = ndfield.read(p)
     assert np.array_equal(a, b) and meta["dims"] == [6, 5, 4]
     assert meta["comment"] == "1 1 0 1 2 0"
+
+
+def test_two_operation_pivot_division_is_correctly_rounded():
+    """The line solves divide by a pivot d as fma(a, rh, RN(a rl)) with
+    rh = RN(1/d), rl = RN(1/d - rh).  Exact rational arithmetic: the value
+    before the fma's rounding is off by less than three of the smallest
+    distances of a quotient from a midpoint, and the numerators at the first
+    distance (the only ones that could round wrongly) round to a/d."""
+    from fractions import Fraction as F
+
+    pivots = sorted(set(thomas(201, 31.4)[1][1:202]) | set(thomas(5, 3.0)[1][1:6]))
+    solved = 0  # pivots whose numerators at the first distance were sought
+    for d in pivots:
+        d = float(d)
+        D = int(F(d) * F(2) ** (53 - int(np.frexp(d)[1])))
+        t = (D & -D).bit_length() - 1
+        rh = 1.0 / d
+        rl = float((1 - F(rh) * F(d)) / F(d))  # float() rounds to nearest
+        bound = 4 * abs(F(rl) * F(d)) * D
+        assert bound < 3 * 2 ** t
+        rng = np.random.default_rng(3)
+        tests = [int(a) for a in rng.integers(2 ** 52, 2 ** 53, 200)]
+        if bound >= 2 ** t:
+            solved += 1
+            odd = D >> t
+            for k in (53, 54):
+                inv = pow(2, -(k - t), odd)
+                for a0 in (inv, odd - inv):
+                    lo = a0 + -(-(2 ** 52 - a0) // odd) * odd
+                    found = list(range(lo, 2 ** 53, odd))
+                    assert len(found) <= 2 ** (t + 1)
+                    tests += found
+        for A in tests:
+            a = float(A)
+            assert float(F(a) * F(rh) + F(a * rl)) == a / d, (d, A)
+    assert len(pivots) >= 16 and solved >= 2

@@ -280,7 +280,7 @@ namespace vls {
 // Runs the elimination of create_1D (src/localSpline.hxx:968-1153) on the
 // data-independent coefficients and records what the data path needs.
 void thomas_table(int dim, double hinv, ThomasAxis &ax, std::vector<double> &u,
-                  std::vector<double> &d, std::vector<double> &rd) {
+                  std::vector<double> &d, std::vector<double> &rd, std::vector<double> &rl) {
   const int M = dim + 2;
   std::vector<double> A(4 * (size_t)M);
   const double hi2 = hinv * hinv;
@@ -323,15 +323,21 @@ void thomas_table(int dim, double hinv, ThomasAxis &ax, std::vector<double> &u,
   ax.q = q;
   ax.rq = 1.0 / q;
   rd.assign(M, 0.0);
-  for (int k = 1; k <= M - 2; k++) rd[k] = 1.0 / d[k];
+  rl.assign(M, 0.0);
+  for (int k = 1; k <= M - 2; k++) {
+    rd[k] = 1.0 / d[k];
+    rl[k] = pivot_remainder(d[k], rd[k]);
+    if ((k == 1 || d[k] != d[k - 1]) && !pivot_division_exact(d[k], rd[k], rl[k]))
+      throw Error(VLS_ERR_ARG, "a spline pivot's division is not correctly rounded");
+  }
   // first row of the constant regime (the table is used before it)
   int K0 = M - 2;
   while (K0 > 1 && d[K0 - 1] == d[M - 2] && u[K0 - 1] == u[M - 2] && rd[K0 - 1] == rd[M - 2]) K0--;
   if (K0 - 1 > 16)  // kHead of the kernels
     throw Error(VLS_ERR_ARG, "spline pivots do not settle within 16 rows");
   ax.K0 = K0;
-  ax.dS = d[M - 2];
   ax.rdS = rd[M - 2];
+  ax.rlS = rl[M - 2];
   ax.uS = u[M - 2];
 }
 
@@ -387,8 +393,8 @@ int vls_thomas_table(int dim, double hinv, double *u, double *d, double *rd, dou
   return guarded([&] {
     if (dim < 2 || !u || !d || !rd || !consts) throw vls::Error(VLS_ERR_ARG, "bad arguments");
     vls::ThomasAxis ax{};
-    std::vector<double> U, D, RD;
-    vls::thomas_table(dim, hinv, ax, U, D, RD);
+    std::vector<double> U, D, RD, RL;
+    vls::thomas_table(dim, hinv, ax, U, D, RD, RL);
     std::copy(U.begin(), U.end(), u);
     std::copy(D.begin(), D.end(), d);
     std::copy(RD.begin(), RD.end(), rd);
@@ -531,17 +537,17 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
       h2d(r.Ct1, Ct1.data(), r.nJ, s);
       h2d(r.gfac, gfac.data(), r.nR, s);
       for (int axis = 0; axis < 2; axis++) {
-        std::vector<double> u, d, rd;
+        std::vector<double> u, d, rd, rl;
         vls::ThomasAxis &ax = axis == 0 ? r.tr : r.tv;
-        vls::thomas_table(axis == 0 ? r.nR : r.nU, G.spline_hinv[axis], ax, u, d, rd);
+        vls::thomas_table(axis == 0 ? r.nR : r.nU, G.spline_hinv[axis], ax, u, d, rd, rl);
         double *dev = dalloc<double>(r, 3 * (size_t)ax.M);
         h2d(dev, u.data(), ax.M, s);
-        h2d(dev + ax.M, d.data(), ax.M, s);
-        h2d(dev + 2 * ax.M, rd.data(), ax.M, s);
+        h2d(dev + ax.M, rd.data(), ax.M, s);
+        h2d(dev + 2 * ax.M, rl.data(), ax.M, s);
         ax.u = dev;
-        ax.d = dev + ax.M;
-        ax.rd = dev + 2 * ax.M;
-        VLS_HIP_CHECK(hipStreamSynchronize(s));  // u, d, rd go out of scope
+        ax.rd = dev + ax.M;
+        ax.rl = dev + 2 * ax.M;
+        VLS_HIP_CHECK(hipStreamSynchronize(s));  // u, rd, rl go out of scope
       }
     }
   });

@@ -29,17 +29,17 @@ struct ThomasAxis {
   double rq;    // RN(1/q)
   // The pivot recurrence d_k = 4/6 - u_{k-1}/6, u_k = (1/6)/d_k does not
   // depend on the data or the knot spacing and reaches an exact fixed point:
-  // from row K0 on, d_k = dS, RN(1/d_k) = rdS and u_k = uS.
+  // from row K0 on, RN(1/d_k) = rdS, its remainder is rlS and u_k = uS.
   int K0;
-  double dS, rdS, uS;
+  double rlS, rdS, uS;
   const double *u;   // device [M]: super-diagonal after division, rows 1..M-2
-  const double *d;   // device [M]: divisor of row k before normalisation
-  const double *rd;  // device [M]: RN(1/d[k])
+  const double *rl;  // device [M]: RN(1/d[k] - rd[k]) (div_pivot)
+  const double *rd;  // device [M]: RN(1/d[k]), d[k] the divisor of row k
 };
 
-// Build the table on the host: u[k], d[k], rd[k] for k=1..M-2 and the constants.
+// Build the table on the host: u[k], d[k], rd[k], rl[k] for k=1..M-2 and the constants.
 void thomas_table(int dim, double hinv, ThomasAxis &ax, std::vector<double> &u,
-                  std::vector<double> &d, std::vector<double> &rd);
+                  std::vector<double> &d, std::vector<double> &rd, std::vector<double> &rl);
 
 // Per-kernel timing with HIP events on the stream of the launches.  Every
 // kernel: an event after each launch (consecutive differences).  One kernel

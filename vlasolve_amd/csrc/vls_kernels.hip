@@ -507,7 +507,7 @@ k_moment_fused(const double *__restrict__ f, int nR, int nU, int nJ, MomentArgs 
 // head whose pivots and right-hand sides are all loaded up front (the table
 // through per-lane vector loads, index + lz with lz a zero the compiler
 // cannot see, so that no scalar-memory wait enters the loops).  From row K0
-// on the pivots are the scalars dS, rdS, uS: the steady loops load nothing
+// on the pivots' reciprocals are the scalars rdS, rlS (and uS): the steady loops load nothing
 // but the data stream, kPF rows ahead.
 constexpr int kHead = 16;
 
@@ -520,21 +520,21 @@ constexpr int kHead = 16;
 // loads; head_store writes them to LDS once they are in, and the block's
 // barrier orders them before the loops' reads.
 struct HeadTab {
-  double u[kHead + 1], d[kHead + 1], rd[kHead + 1];
+  double u[kHead + 1], rd[kHead + 1], rl[kHead + 1];
 };
 struct HeadRegs {
-  double u, d, rd;
+  double u, rd, rl;
 };
 __device__ __forceinline__ HeadRegs head_load(const ThomasAxis &ax, int lane, int lz) {
   const int last = kHead < ax.M - 2 ? kHead : ax.M - 2;
   const int k = lane < 1 ? 1 : (lane > last ? last : lane);
-  return {ax.u[k + lz], ax.d[k + lz], ax.rd[k + lz]};
+  return {ax.u[k + lz], ax.rd[k + lz], ax.rl[k + lz]};
 }
 __device__ __forceinline__ void head_store(HeadTab &t, const HeadRegs &h, int lane) {
   if (lane >= 1 && lane <= kHead) {
     t.u[lane] = h.u;
-    t.d[lane] = h.d;
     t.rd[lane] = h.rd;
+    t.rl[lane] = h.rl;
   }
 }
 
@@ -552,21 +552,21 @@ __device__ __forceinline__ void thomas_forward(const ThomasAxis &ax, int lz, RHS
 #pragma unroll
   for (int q = 0; q < kHead; q++) {
     hr[q] = rhs(kc(1 + q));
-    hd[q] = ax.d[kc(1 + q) + lz];
-    he[q] = ax.rd[kc(1 + q) + lz];
+    hd[q] = ax.rd[kc(1 + q) + lz];
+    he[q] = ax.rl[kc(1 + q) + lz];
   }
 #pragma unroll
   for (int q = 0; q < kPF; q++) rb[q] = rhs(kc(P + 1 + q));
   // loop constants as per-lane values (x + lz == x): their scalar loads are
   // waited for here, once, instead of inside every guarded loop body
-  const double c16 = ax.c16 + (double)lz, dS = ax.dS + (double)lz, rdS = ax.rdS + (double)lz;
+  const double c16 = ax.c16 + (double)lz, rdS = ax.rdS + (double)lz, rlS = ax.rlS + (double)lz;
   ym2 = 0.0;
   ym1 = ax.A03;
 #pragma unroll
   for (int q = 0; q < kHead; q++) {
     if (q < P) {
       consume(1 + q, hr[q]);
-      double yk = div_known(hr[q] - c16 * ym1, hd[q], he[q]);
+      double yk = div_pivot(hr[q] - c16 * ym1, hd[q], he[q]);
       store(1 + q, yk);
       ym2 = ym1;
       ym1 = yk;
@@ -578,7 +578,7 @@ __device__ __forceinline__ void thomas_forward(const ThomasAxis &ax, int lz, RHS
       const int kk = k + q;
       if (kk <= M - 2) {
         consume(kk, rb[q]);
-        double yk = div_known(rb[q] - c16 * ym1, dS, rdS);
+        double yk = div_pivot(rb[q] - c16 * ym1, rdS, rlS);
         store(kk, yk);
         ym2 = ym1;
         ym1 = yk;
@@ -823,7 +823,7 @@ k_spline_r_stream(const double *__restrict__ f, double *__restrict__ c, int nR, 
     }
     __syncthreads();
   };
-  const double c16 = ax.c16 + (double)lz, dS = ax.dS + (double)lz, rdS = ax.rdS + (double)lz;
+  const double c16 = ax.c16 + (double)lz, rdS = ax.rdS + (double)lz, rlS = ax.rlS + (double)lz;
   double ym1 = ax.A03, ym2 = 0.0;
   // forward elimination: rhs_k = f[k-1], y_k to padded column k
   for (int e0 = 0; e0 < nR; e0 += kC) {
@@ -832,12 +832,12 @@ k_spline_r_stream(const double *__restrict__ f, double *__restrict__ c, int nR, 
     for (int i = 0; i < kC; i++) {
       const int k = e0 + i + 1;
       if (k <= M - 2) {
-        double dv = dS, ev = rdS;
+        double dv = rdS, ev = rlS;
         if (k <= kHead) {
-          dv = ax.d[k + lz];
-          ev = ax.rd[k + lz];
+          dv = ax.rd[k + lz];
+          ev = ax.rl[k + lz];
         }
-        const double yk = div_known(v[i] - c16 * ym1, dv, ev);
+        const double yk = div_pivot(v[i] - c16 * ym1, dv, ev);
         v[i] = yk;
         ym2 = ym1;
         ym1 = yk;
@@ -881,8 +881,8 @@ k_spline_r_stream(const double *__restrict__ f, double *__restrict__ c, int nR, 
 // are stored as they are produced.  Every line of the grid is in flight at
 // once (one wave per SIMD at ~2M VGPRs), which is what a latency-bound
 // recurrence needs.  Rows 1..kHead use the pivot table (whose entries from
-// K0 <= kHead+1 on equal the fixed point), later rows the fixed point dS,
-// rdS, uS.
+// K0 <= kHead+1 on equal the fixed point), later rows the fixed point rdS,
+// rlS, uS.
 //   KICK = false: the nR+2 = S padded columns (j, col); rhs_k = c[j][k][col],
 //                 c_k -> c[j][k][col]      (create_2D second loop); with src
 //                 non-null the right-hand sides come from src (same layout)
@@ -934,17 +934,17 @@ k_line(const double *__restrict__ src, double *__restrict__ c, int nR, int nU, i
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const double c16 = ax.c16 + (double)lz, dS = ax.dS + (double)lz, rdS = ax.rdS + (double)lz;
+  const double c16 = ax.c16 + (double)lz, rdS = ax.rdS + (double)lz, rlS = ax.rlS + (double)lz;
   double prev = ax.A03;
 #pragma unroll
   for (int k = 1; k <= M - 2; k++) {
     if (k + kLA <= M - 2) y[k + kLA] = in[(k + kLA) * is];
-    double dv = dS, ev = rdS;
+    double dv = rdS, ev = rlS;
     if (k <= kHead) {
-      dv = htab.d[k];
-      ev = htab.rd[k];
+      dv = htab.rd[k];
+      ev = htab.rl[k];
     }
-    y[k] = div_known(y[k] - c16 * prev, dv, ev);
+    y[k] = div_pivot(y[k] - c16 * prev, dv, ev);
     prev = y[k];
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -1022,7 +1022,7 @@ k_kick_solve_moment(const double *__restrict__ f, double *__restrict__ c, int nR
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const double c16 = ax.c16 + (double)lz, dS = ax.dS + (double)lz, rdS = ax.rdS + (double)lz;
+  const double c16 = ax.c16 + (double)lz, rdS = ax.rdS + (double)lz, rlS = ax.rlS + (double)lz;
   double prev = ax.A03;
   // moment state: the previous raw row (own and next column), the group sum,
   // the groups of the current block, the partial over finished blocks
@@ -1059,12 +1059,12 @@ k_kick_solve_moment(const double *__restrict__ f, double *__restrict__ c, int nR
     }
     aOwn = b;
     aN = bN;
-    double dv = dS, ev = rdS;
+    double dv = rdS, ev = rlS;
     if (k <= kHead) {
-      dv = htab.d[k];
-      ev = htab.rd[k];
+      dv = htab.rd[k];
+      ev = htab.rl[k];
     }
-    y[k] = div_known(b - c16 * prev, dv, ev);
+    y[k] = div_pivot(b - c16 * prev, dv, ev);
     prev = y[k];
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -1247,7 +1247,7 @@ k_kick_line(double *f, const double *__restrict__ U_Val, const double *__restric
   // the time (its U value read from LDS one step ahead)
   int dlo = 1 << 30, dhi = -(1 << 30);
   double usNext = Us[0];
-  const double c16 = ax.c16 + (double)lz, dS = ax.dS + (double)lz, rdS = ax.rdS + (double)lz;
+  const double c16 = ax.c16 + (double)lz, rdS = ax.rdS + (double)lz, rlS = ax.rlS + (double)lz;
   double prev = ax.A03;
 #pragma unroll
   for (int m = 1; m <= Mv - 2; m++) {
@@ -1261,12 +1261,12 @@ k_kick_line(double *f, const double *__restrict__ U_Val, const double *__restric
         dhi = max(dhi, n - (m - 1));
       }
     }
-    double dv = dS, ev = rdS;
+    double dv = rdS, ev = rlS;
     if (m <= kHead) {
-      dv = htab.d[m];
-      ev = htab.rd[m];
+      dv = htab.rd[m];
+      ev = htab.rl[m];
     }
-    const double yk = div_known(y[m] - c16 * prev, dv, ev);
+    const double yk = div_pivot(y[m] - c16 * prev, dv, ev);
     if (m <= kYL)
       ylds[(m - 1) * 64 + lane] = yk;
     else
@@ -2075,7 +2075,7 @@ k_line_rows(const double *__restrict__ f, double *__restrict__ c, int nR, int nU
       t[q] = src[row * nIn + e];
     }
   };
-  const double c16 = ax.c16 + (double)lz, dS = ax.dS + (double)lz, rdS = ax.rdS + (double)lz;
+  const double c16 = ax.c16 + (double)lz, rdS = ax.rdS + (double)lz, rlS = ax.rlS + (double)lz;
   double prev = ax.A03;
 #pragma unroll
   for (int ch = 0; ch < kAh; ch++)
@@ -2096,12 +2096,12 @@ k_line_rows(const double *__restrict__ f, double *__restrict__ c, int nR, int nU
     for (int i = 0; i < kC; i++) {
       const int k = 1 + ch * kC + i;
       if (k <= M - 2) {
-        double dv = dS, ev = rdS;
+        double dv = rdS, ev = rlS;
         if (k <= kHead) {
-          dv = htab.d[k];
-          ev = htab.rd[k];
+          dv = htab.rd[k];
+          ev = htab.rl[k];
         }
-        y[k] = div_known(y[k] - c16 * prev, dv, ev);
+        y[k] = div_pivot(y[k] - c16 * prev, dv, ev);
         prev = y[k];
       }
     }
@@ -2310,7 +2310,7 @@ k_line_rows_kick(const double *__restrict__ d, double *__restrict__ c,
   }
   wave_sync();
   double y[M];
-  const double c16 = ax.c16 + (double)lz, dS = ax.dS + (double)lz, rdS = ax.rdS + (double)lz;
+  const double c16 = ax.c16 + (double)lz, rdS = ax.rdS + (double)lz, rlS = ax.rlS + (double)lz;
   double prev = ax.A03;
   // Software pipeline: the evaluation of chunk ch + 1 (VALU-heavy, from the
   // window in LDS into the chunk transpose) shares a step with the
@@ -2346,12 +2346,12 @@ k_line_rows_kick(const double *__restrict__ d, double *__restrict__ c,
     for (int i = 0; i < kC; i++) {
       const int k = 1 + ch * kC + i;
       if (k <= M - 2) {
-        double dv = dS, ev = rdS;
+        double dv = rdS, ev = rlS;
         if (k <= kHead) {
-          dv = htab.d[k];
-          ev = htab.rd[k];
+          dv = htab.rd[k];
+          ev = htab.rl[k];
         }
-        const double yk = div_known(y[k] - c16 * prev, dv, ev);
+        const double yk = div_pivot(y[k] - c16 * prev, dv, ev);
         if (k <= kYL)
           ylds[(k - 1) * 64 + lane] = yk;
         else
