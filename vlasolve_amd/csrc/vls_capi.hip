@@ -162,12 +162,35 @@ void step_once(vls::Run &r, hipStream_t s, vls::Timing *t) {
   r.stepped = true;
 }
 
+// nSteps steps of a run
+void step_many(vls::Run &r, hipStream_t s, int nSteps, vls::Timing *t) {
+  if (!vls::slice_on(r)) {
+    for (int n = 0; n < nSteps; n++) step_once(r, s, t);
+    return;
+  }
+  if (nSteps < 1) return;
+  vls::time_begin(t, s, "slice_start");
+  vls::launch_slice_start(r, s);
+  vls::time_mark(t, s, "slice_start");
+  for (int n = 0; n < nSteps; n++) {
+    vls::time_begin(t, s, "slice_kick");
+    vls::launch_slice_kick(r, s, nullptr);
+    vls::time_mark(t, s, "slice_kick");
+    vls::time_begin(t, s, "slice_drift");
+    vls::launch_slice_drift(r, s, n + 1 == nSteps);
+    vls::time_mark(t, s, "slice_drift");
+  }
+  r.stepped = true;
+}
+
 // One step that also keeps what the adjoint of the step needs: the kick's
 // acceleration (accOut, [nR]) and the v-spline coefficients of the columns
 // of f (cK, [j][m][r] with slice stride cs), which the kick leaves there.
 // Without advance the step stops after the kick (the state after it is not
 // needed: the last step of a recomputed segment).
-void step_keep(vls::Run &r, hipStream_t s, double *cK, double *accOut, bool advance = true) {
+// slice: by the slice step, last: the last one of the recording.
+void step_keep(vls::Run &r, hipStream_t s, double *cK, double *accOut, bool advance, bool slice,
+               bool last) {
   // the moment writes the acceleration straight into accOut (the step's
   // kernels take r.acc when launched); r.acc is left as it was
   struct AccSwap {
@@ -176,6 +199,11 @@ void step_keep(vls::Run &r, hipStream_t s, double *cK, double *accOut, bool adva
     ~AccSwap() { r.acc = own; }
   } swap{r, r.acc};
   r.acc = accOut;
+  if (slice) {
+    vls::launch_slice_kick(r, s, cK);
+    if (advance) vls::launch_slice_drift(r, s, last);
+    return;
+  }
   vls::launch_spline_kick(r, s, nullptr, true, cK);
   r.acc = swap.own;
   if (!advance) return;
@@ -199,7 +227,7 @@ void ensure_run_streams(vls::Context &C) {
   }
 }
 
-void build_ensemble_graph(vls::Context &C) {
+void build_ensemble_graph(vls::Context &C, int which) {
   const int n = (int)C.runs.size();
   ensure_run_streams(C);
   if (!C.forkEv) VLS_HIP_CHECK(hipEventCreateWithFlags(&C.forkEv, hipEventDisableTiming));
@@ -209,7 +237,11 @@ void build_ensemble_graph(vls::Context &C) {
     VLS_HIP_CHECK(hipEventRecord(C.forkEv, C.stream));
     for (int k = 0; k < n; k++) {
       VLS_HIP_CHECK(hipStreamWaitEvent(C.runStreams[k], C.forkEv, 0));
-      step_once(C.runs[k], C.runStreams[k], nullptr);
+      if (vls::slice_on(C.runs[k])) {
+        vls::launch_slice_kick(C.runs[k], C.runStreams[k], nullptr);
+        vls::launch_slice_drift(C.runs[k], C.runStreams[k], which == 1);
+      } else
+        step_once(C.runs[k], C.runStreams[k], nullptr);
       VLS_HIP_CHECK(hipEventRecord(C.joinEv[k], C.runStreams[k]));
       VLS_HIP_CHECK(hipStreamWaitEvent(C.stream, C.joinEv[k], 0));
     }
@@ -219,17 +251,19 @@ void build_ensemble_graph(vls::Context &C) {
     throw;
   }
   VLS_HIP_CHECK(hipStreamEndCapture(C.stream, &g));
-  hipError_t e = hipGraphInstantiate(&C.graph, g, nullptr, nullptr, 0);
+  hipError_t e = hipGraphInstantiate(&C.graph[which], g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   if (e != hipSuccess) {
-    C.graph = nullptr;
+    C.graph[which] = nullptr;
     throw vls::Error(VLS_ERR_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
   }
 }
 
 void drop_graph(vls::Context &C) {
-  if (C.graph) (void)hipGraphExecDestroy(C.graph);
-  C.graph = nullptr;
+  for (hipGraphExec_t &g : C.graph) {
+    if (g) (void)hipGraphExecDestroy(g);
+    g = nullptr;
+  }
 }
 }  // namespace
 
@@ -471,6 +505,8 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
     VLS_HIP_CHECK(hipStreamCreateWithFlags(&ctx->c.stream, hipStreamNonBlocking));
     hipStream_t s = ctx->c.stream;
     ctx->c.runs.resize(nRuns);
+    int64_t slices = 0;
+    for (int k = 0; k < nRuns; k++) slices += std::max(1, g[k].nJ);
     for (int k = 0; k < nRuns; k++) {
       const vls_geometry &G = g[k];
       vls::Run &r = ctx->c.runs[k];
@@ -492,6 +528,7 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
       r.hU.assign(G.U_Val, G.U_Val + r.nU);
       r.Ulo = G.U_Val[0];
       r.Uhi = G.U_Val[r.nU - 1];
+      r.cus = (int)(256 * (int64_t)r.nJ / slices);
       vls::configure_tiles(r, maxLds);
       // the kick folded into the r-solve leaves the solved rows (c's layout) in
       // f's buffer between the kick and the drift
@@ -536,10 +573,12 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
       h2d(r.dU, G.dU, r.nU, s);
       h2d(r.Ct1, Ct1.data(), r.nJ, s);
       h2d(r.gfac, gfac.data(), r.nR, s);
+      bool pivots = true;
       for (int axis = 0; axis < 2; axis++) {
         std::vector<double> u, d, rd, rl;
         vls::ThomasAxis &ax = axis == 0 ? r.tr : r.tv;
         vls::thomas_table(axis == 0 ? r.nR : r.nU, G.spline_hinv[axis], ax, u, d, rd, rl);
+        pivots = pivots && vls::slice_pivots(ax, u.data(), rd.data(), rl.data());
         double *dev = dalloc<double>(r, 3 * (size_t)ax.M);
         h2d(dev, u.data(), ax.M, s);
         h2d(dev + ax.M, rd.data(), ax.M, s);
@@ -548,6 +587,13 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
         ax.rd = dev + ax.M;
         ax.rl = dev + 2 * ax.M;
         VLS_HIP_CHECK(hipStreamSynchronize(s));  // u, rd, rl go out of scope
+      }
+      if (pivots && vls::slice_shape(r, maxLds)) {
+        vls::configure_slice(maxLds);
+        r.sliceG = dalloc<double>(r, vls::slice_group_doubles(r));
+        r.sliceCnt = dalloc<unsigned>(r, r.nJ);
+        VLS_HIP_CHECK(hipMemsetAsync(r.sliceCnt, 0, r.nJ * sizeof(unsigned), s));
+        if (vls::slice_shared(r)) r.sliceF = dalloc<double>(r, r.nVal);
       }
     }
   });
@@ -638,6 +684,7 @@ int vls_set_drift(vls_ctx *ctx, int run, const double *xr, const double *xu, con
       if (flag[i] == VLS_FOOT_CHAIN) xf[i] = -2.0, uf[i] = -1.0;
     }
     r.hflag.assign(flag, flag + r.nVal);
+    r.nChainFlags = std::count(flag, flag + r.nVal, (uint8_t)VLS_FOOT_CHAIN);
     hipStream_t s = ctx->c.stream;
     std::vector<double> ft(2 * r.nVal);
     for (int64_t i = 0; i < r.nVal; i++) ft[2 * i] = xf[i], ft[2 * i + 1] = uf[i];
@@ -690,6 +737,8 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
     dfree(r, r.ch_xu);
     dfree(r, r.ch_out);
     dfree(r, r.ch_vals);
+    dfree(r, r.ch_order);
+    dfree(r, r.ch_start);
     r.adj.recorded = false;
     r.adj.tilesValid = false;  // the transposed foot table lists the back cells
     r.nChains = nChains;
@@ -713,6 +762,19 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
     h2d(r.ch_xr, back_xr, nChains, s);
     h2d(r.ch_xu, back_xu, nChains, s);
     h2d(r.ch_out, back_out, nChains, s);
+    // the delay lines by slice
+    const int64_t nSlice = (int64_t)r.nU * r.nR;
+    std::vector<int32_t> start(r.nJ + 1, 0), order(nChains);
+    for (int64_t k = 0; k < nChains; k++) start[point[k] / nSlice + 1]++;
+    r.maxLines = *std::max_element(start.begin(), start.end());
+    for (int j = 0; j < r.nJ; j++) start[j + 1] += start[j];
+    std::vector<int32_t> at(start.begin(), start.end() - 1);
+    for (int64_t k = 0; k < nChains; k++) order[at[point[k] / nSlice]++] = (int32_t)k;
+    r.ch_order = dalloc<int32_t>(r, nChains);
+    r.ch_start = dalloc<int32_t>(r, r.nJ + 1);
+    h2d(r.ch_order, order.data(), nChains, s);
+    h2d(r.ch_start, start.data(), r.nJ + 1, s);
+    VLS_HIP_CHECK(hipStreamSynchronize(s));  // start, order go out of scope
     if (r.nS > 1) {
       std::vector<double> planes = to_planes(vals, cells, r.nS);
       h2d(r.ch_vals, planes.data(), planes.size(), s);
@@ -769,12 +831,20 @@ int vls_step(vls_ctx *ctx, int nSteps) {
     vls::Context &C = ctx->c;
     if (C.runs.size() > 1 && C.graphOn && !t->on) {
       // an ensemble: the runs advance concurrently, one graph launch a step
-      if (!C.graph) build_ensemble_graph(C);
-      for (int n = 0; n < nSteps; n++) VLS_HIP_CHECK(hipGraphLaunch(C.graph, s));
+      bool slices = false;
+      for (auto &r : C.runs)
+        if (nSteps > 0 && vls::slice_on(r)) {
+          vls::launch_slice_start(r, s);
+          slices = true;
+        }
+      for (int n = 0; n < nSteps; n++) {
+        const int which = slices && n + 1 == nSteps;
+        if (!C.graph[which]) build_ensemble_graph(C, which);
+        VLS_HIP_CHECK(hipGraphLaunch(C.graph[which], s));
+      }
       for (auto &r : C.runs) r.stepped = true;
     } else {
-      for (int n = 0; n < nSteps; n++)
-        for (auto &r : C.runs) step_once(r, s, t);
+      for (auto &r : C.runs) step_many(r, s, nSteps, t);
     }
     VLS_HIP_CHECK(hipGetLastError());
   });
@@ -1108,9 +1178,16 @@ void record_step(vls::Run &r, hipStream_t s, int n) {
     d2d(A.ckVals + nc * k, r.ch_vals, nc, s);
     d2d(A.ckHead + nch * k, r.ch_head, nch, s);
   }
+  const bool slice = vls::slice_on(r), last = n + 1 == A.nSteps;
+  if (slice && n == 0) vls::launch_slice_start(r, s);
   if (n >= A.keptFrom)
-    step_keep(r, s, A.keepC + coef * (n - A.keptFrom), A.keepAcc + (size_t)r.nR * (n - A.keptFrom));
-  else
+    step_keep(r, s, A.keepC + coef * (n - A.keptFrom), A.keepAcc + (size_t)r.nR * (n - A.keptFrom),
+              true, slice, last);
+  else if (slice) {
+    vls::launch_slice_kick(r, s, nullptr);
+    vls::launch_slice_drift(r, s, last);
+    r.stepped = true;
+  } else
     step_once(r, s, nullptr);
 }
 
@@ -1161,8 +1238,11 @@ void adjoint_segment(vls::Run &r, hipStream_t s, int sg) {
     d2d(r.f, A.ckF + nv * sg, nv, s);
     d2d(r.ch_vals, A.ckVals + nc * sg, nc, s);
     d2d(r.ch_head, A.ckHead + nch * sg, nch, s);
+    const bool slice = vls::slice_on(r);
+    if (slice) vls::launch_slice_start(r, s);
     for (int n = n0; n < n1; n++)
-      step_keep(r, s, A.segC + coef * (n - n0), A.segAcc + (size_t)r.nR * (n - n0), n + 1 < n1);
+      step_keep(r, s, A.segC + coef * (n - n0), A.segAcc + (size_t)r.nR * (n - n0), n + 1 < n1,
+                slice, false);
   }
   for (int n = n1 - 1; n >= n0; n--) {
     const double *cK = kept ? A.keepC + coef * (n - A.keptFrom) : A.segC + coef * (n - n0);

@@ -70,6 +70,9 @@ struct Run {
   // moment fused into the kick's column splines / that, and the kick's
   // evaluation folded into the drift's r-solve
   int lineMode = -1, kickMode = -1;
+  // a step in two launches (vls_slice.hip), for the shapes that have sliceG: -1
+  // unless the environment forces one of the other schedules, 0 / 1 tuned
+  int sliceMode = -1;
   vls_solver_params sp{};
   double start_v = 0, hinv_v = 0, Ulo = 0, Uhi = 0;
 
@@ -84,9 +87,15 @@ struct Run {
   // (xr <= -1 marks points outside the grid or on delay lines)
   double *feet = nullptr;  // [nVal][2]
   std::vector<uint8_t> hflag;  // host copy of the VLS_FOOT_* kinds
+  int64_t nChainFlags = 0;     // points of kind VLS_FOOT_CHAIN
   // moment
   double *P = nullptr;      // [nJ][nR] per-slice partials
   double *dM = nullptr, *Mx = nullptr, *acc = nullptr, *mTot = nullptr;
+  int cus = 256;  // the compute units the run may count on (an ensemble's runs share them)
+  // slice step: the kicked f where several blocks share a slice, their group
+  // sums of the moment and their counters (zero between launches)
+  double *sliceF = nullptr, *sliceG = nullptr;
+  unsigned *sliceCnt = nullptr;
   unsigned *mCnt = nullptr;  // counters of the one-launch moment (zero between launches)
   double *rhoPhi = nullptr;  // [2][nR]: shell density and potential (vls_density_potential)
   // tables
@@ -95,8 +104,10 @@ struct Run {
   ThomasAxis tr{}, tv{};
   // delay lines
   int64_t nChains = 0, nCells = 0;
+  int maxLines = 0;  // delay lines of a slice, at most
   int64_t *ch_point = nullptr, *ch_off = nullptr;
   int32_t *ch_len = nullptr, *ch_head = nullptr;
+  int32_t *ch_order = nullptr, *ch_start = nullptr;  // [nChains] by slice, [nJ+1]
   double *ch_xr = nullptr, *ch_xu = nullptr, *ch_vals = nullptr;
   uint8_t *ch_out = nullptr;
   // statistics
@@ -150,7 +161,9 @@ struct Context {
   std::vector<hipStream_t> runStreams;
   hipEvent_t forkEv = nullptr;
   std::vector<hipEvent_t> joinEv;
-  hipGraphExec_t graph = nullptr;
+  // one step of the ensemble, and the last of a call, which differs for the
+  // runs with the slice step (without such runs the first serves for all)
+  hipGraphExec_t graph[2] = {};
   bool graphOn = true;
 };
 
@@ -195,6 +208,23 @@ void launch_spline_kick(Run &r, hipStream_t s, Timing *t, bool moment = true,
                         double *dKeep = nullptr);
 size_t kick_scratch_doubles(const Run &r);
 void launch_drift(Run &r, hipStream_t s);
+// the slice step (vls_slice.hip): shapes whose slices fit in a CU's LDS (and
+// have the standard pivots), whether this run takes it, what precedes the
+// first step of a call (the moment partials of f, and without linking the
+// first half drift), and a step's two halves.  The kick advances the delay
+// lines' heads by the step's drifts; dKeep receives its column splines
+// ([j][m][r], slice stride cs).  The drift forms the partials that the next
+// kick takes; the last of a call leaves its coefficients in c instead.
+bool slice_shape(const Run &r, int maxLdsPerBlock);
+bool slice_pivots(const ThomasAxis &ax, const double *u, const double *rd, const double *rl);
+bool slice_shared(const Run &r);  // several blocks take a slice
+size_t slice_group_doubles(const Run &r);
+void configure_slice(int maxLdsPerBlock);
+bool slice_fits(const Run &r);    // the run's buffers are there and its delay lines fit too
+bool slice_on(const Run &r);
+void launch_slice_start(Run &r, hipStream_t s);
+void launch_slice_kick(Run &r, hipStream_t s, double *dKeep);
+void launch_slice_drift(Run &r, hipStream_t s, bool last);
 void mark_chains(Run &r, hipStream_t s);  // attach the delay lines to their points
 void launch_stats(Run &r, hipStream_t s);
 // rho[nR], phi[nR] (device) from the moment and enclosed mass of the last launch_moment

@@ -17,6 +17,7 @@
 #include <string>
 #include <tuple>
 
+#include "vls_device.hpp"
 #include "vls_div.hpp"
 #include "vls_internal.hpp"
 #include "vls_tile.hpp"
@@ -27,21 +28,6 @@ namespace {
 
 constexpr int kBlock = 256;
 
-__device__ __forceinline__ double BV2(double x) { return x * x * x; }
-__device__ __forceinline__ double BV1(double x) {
-  return 1.0 + 3.0 * x + 3.0 * x * x - 3.0 * x * x * x;
-}
-
-// modf for the finite, non-negative coordinates used here: integer part by
-// truncation, exact fractional remainder (localSpline::pos2Coord,
-// src/localSpline.hxx:352-358).
-__device__ __forceinline__ void split(double x, int &n, double &t) {
-  double ip = trunc(x);
-  t = x - ip;
-  n = (int)ip;
-}
-
-
 // ---------------------------------------------------------------- moment
 // Per (j, r) partial of quadrature21::integrate1D (src/quadrature21.hxx:104-133):
 // the terms ((Ct1_j*dU_u)*dR_r) * avg4 over u < nU-1, summed in a fixed tree:
@@ -51,12 +37,6 @@ __device__ __forceinline__ void split(double x, int &n, double &t) {
 // block; column r + 1 arrives by a lane shift) and a wave per block of 64
 // rows (loaded in two halves of 32 rows and the row after each); the blocks'
 // partials meet in LDS.
-__device__ __forceinline__ double lane_next(double x) {  // lane i gets lane i+1's x
-  int lo = __double2loint(x), hi = __double2hiint(x);
-  lo = __builtin_amdgcn_mov_dpp(lo, 0x130 /* wave_shl:1 */, 0xf, 0xf, true);
-  hi = __builtin_amdgcn_mov_dpp(hi, 0x130, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
-}
 // Stores and loads that other XCDs see without cache maintenance: system
 // scope, so they go through the (per-XCD, non-coherent) L2 to memory; the
 // counters below are agent-scope atomics, which the device keeps coherent.
@@ -286,7 +266,7 @@ __device__ __forceinline__ void scan_prefix_out(double *sdm, const double *sgf,
 // the S_c with a block per chunk (the partials are read by many CUs at
 // once) and leaves S_c in place of the chunk's first slice of P (read by the
 // same thread only); k_moment_scan adds the chunks and runs the prefix.
-constexpr int kScanThreads = 1024, kJC = 20, kChunkThreads = 256;
+constexpr int kScanThreads = 1024, kChunkThreads = 256;
 __global__ void __launch_bounds__(kChunkThreads)
 k_moment_chunks(double *__restrict__ P, int nR, int nJ) {
   const int r = blockIdx.y * kChunkThreads + threadIdx.x;
@@ -349,12 +329,6 @@ k_moment_scan(const double *__restrict__ P, const double *__restrict__ gfac, dou
 // the count, read with coherent_load after it; agent-scope fences would
 // instead write back and invalidate each XCD's whole L2 in every block.
 // Every thread of the block calls it; sdm holds 2 nR doubles of LDS.
-struct MomentArgs {
-  const double *Ct1, *dU, *dR, *gfac;
-  double *P, *dM, *Mx, *acc, *mTot;
-  unsigned *cnt;
-};
-
 // The block's count in its (chunk, column tile) counter, issued once its
 // partials are acknowledged; the returned value o completes the chunk when
 // moment_chunk_done(o, ...) holds.  lz: a zero in a VGPR that the compiler
@@ -509,7 +483,6 @@ k_moment_fused(const double *__restrict__ f, int nR, int nU, int nJ, MomentArgs 
 // cannot see, so that no scalar-memory wait enters the loops).  From row K0
 // on the pivots' reciprocals are the scalars rdS, rlS (and uS): the steady loops load nothing
 // but the data stream, kPF rows ahead.
-constexpr int kHead = 16;
 
 // The head's pivots staged in LDS, for the register line kernels whose loops
 // stream their line: a global load of a table entry inside such a loop makes
@@ -519,9 +492,6 @@ constexpr int kHead = 16;
 // k, clamped to the rows a line of M entries has) before the line's own
 // loads; head_store writes them to LDS once they are in, and the block's
 // barrier orders them before the loops' reads.
-struct HeadTab {
-  double u[kHead + 1], rd[kHead + 1], rl[kHead + 1];
-};
 struct HeadRegs {
   double u, rd, rl;
 };
@@ -1470,15 +1440,6 @@ k_kick_vsolve(const double *__restrict__ f, double *__restrict__ d, int nR, int 
       [&](int k, double v) { dc[(int64_t)k * nR] = v; });
 }
 
-// The kick's value of a point from the four column-spline coefficients of
-// its target rows n..n+3 and its offset y in the cell (evaluateNxPy,
-// src/localSpline.hxx:423-441, in the column form)
-__device__ __forceinline__ double kick_value(double y, double d0, double d1, double d2, double d3) {
-  double result = 1.0 / 6.0;
-  result *= BV2(1. - y) * d0 + BV1(1. - y) * d1 + BV1(y) * d2 + BV2(y) * d3;
-  return result;
-}
-
 // k_kick_vsolve with the moment of the same f (as k_kick_solve_moment does
 // for the register lines): tiles of 63 columns, lane 63 solving the next
 // tile's first column for its values only; the moment's terms are taken as
@@ -1604,65 +1565,6 @@ k_kick_cols(double *__restrict__ f, const double *__restrict__ d, const double *
 }
 
 // ---------------------------------------------------------------- drift
-// localSpline::evaluateC(Nx,x,Ny,y), src/localSpline.hxx:381-398
-__device__ __forceinline__ double eval_c(const double *d, int64_t st, double xr, double xu) {
-  int Nx, Ny;
-  double x, y;
-  split(xr, Nx, x);
-  split(xu, Ny, y);
-  Nx++;
-  Ny++;
-  const double *p0 = d + Nx + (int64_t)(Ny - 1) * st;
-  const double *p1 = p0 + st;
-  const double *p2 = p1 + st;
-  const double *p3 = p2 + st;
-  const double b2xI = BV2(1. - x);
-  const double b1xI = BV1(1. - x);
-  const double b2x = BV2(x);
-  const double b1x = BV1(x);
-  double result = 1.0 / 36.0;
-  result *= BV2(1. - y) * (p0[-1] * b2xI + p0[0] * b1xI + p0[1] * b1x + p0[2] * b2x) +
-            BV1(1. - y) * (p1[-1] * b2xI + p1[0] * b1xI + p1[1] * b1x + p1[2] * b2x) +
-            BV1(y) * (p2[-1] * b2xI + p2[0] * b1xI + p2[1] * b1x + p2[2] * b2x) +
-            BV2(y) * (p3[-1] * b2xI + p3[0] * b1xI + p3[1] * b1x + p3[2] * b2x);
-  return result;
-}
-
-// eval_c in two parts, so that several points' loads can leave together:
-// the 4x4 coefficients and the offsets in the cell, then the same sum in the
-// same order as eval_c.
-struct CStencil {
-  double v[16];  // rows Ny-1..Ny+2, columns Nx-1..Nx+2 (v[4 a + b])
-  double x, y;
-};
-__device__ __forceinline__ void eval_c_fetch(const double *d, int64_t st, double xr, double xu,
-                                             CStencil &s) {
-  int Nx, Ny;
-  split(xr, Nx, s.x);
-  split(xu, Ny, s.y);
-  Nx++;
-  Ny++;
-  const double *p0 = d + Nx + (int64_t)(Ny - 1) * st;
-#pragma unroll
-  for (int a = 0; a < 4; a++)
-#pragma unroll
-    for (int b = 0; b < 4; b++) s.v[4 * a + b] = p0[(int64_t)a * st + b - 1];
-}
-__device__ __forceinline__ double eval_c_sum(const CStencil &s) {
-  const double x = s.x, y = s.y;
-  const double *v = s.v;
-  const double b2xI = BV2(1. - x);
-  const double b1xI = BV1(1. - x);
-  const double b2x = BV2(x);
-  const double b1x = BV1(x);
-  double result = 1.0 / 36.0;
-  result *= BV2(1. - y) * (v[0] * b2xI + v[1] * b1xI + v[2] * b1x + v[3] * b2x) +
-            BV1(1. - y) * (v[4] * b2xI + v[5] * b1xI + v[6] * b1x + v[7] * b2x) +
-            BV1(y) * (v[8] * b2xI + v[9] * b1xI + v[10] * b1x + v[11] * b2x) +
-            BV2(y) * (v[12] * b2xI + v[13] * b1xI + v[14] * b1x + v[15] * b2x);
-  return result;
-}
-
 // drift loop, src/vlasovSolver21_spline.hxx:788-796, with the delayed central
 // kernel.  The foot table carries the point's kind in xr: an evaluated foot
 // has xr > -1 (trunc(xr) >= 0), kFootOut (-1) is a foot outside the grid
@@ -1676,19 +1578,6 @@ __device__ __forceinline__ double eval_c_sum(const CStencil &s) {
 // XCD (block id mod 8) walks a contiguous range of points: the 4x4 stencils
 // of neighbouring points share coefficient rows, which then stay in that
 // XCD's L2.
-constexpr double kFootOut = -1.0, kFootChain = -2.0;
-
-struct ChainTables {
-  const int64_t *off;
-  const int32_t *len;
-  int32_t *head;
-  const double *bxr, *bxu;
-  const uint8_t *bout;
-  double *vals;  // the values of the species being drifted
-  int64_t n;
-  int roll;      // turn the rings (the last species of the step)
-};
-
 // Two points per thread (i and i + kBlock of a block's 2 kBlock points):
 // both points' feet, then both stencils' loads, go out together, so that a
 // wave keeps twice the loads in flight (a stencil's reads wait on its foot's
@@ -2647,6 +2536,8 @@ struct Sched {
   int lineMode, kickMode, TR, LS, TC;
   bool streamR, streamV;
   double splineUs, kickUs;
+  bool slice = false;              // a step in two launches
+  double stepUs = 0, sliceUs = 0;  // a step of the kernels per phase, and of the slice step
 };
 std::mutex g_tuneMu;
 std::map<std::tuple<int, int, int, int>, Sched> g_tuned;
@@ -2659,6 +2550,7 @@ void apply_sched(Run &r, const Sched &c) {
   r.TC = c.TC;
   r.streamR = c.streamR;
   r.streamV = c.streamV;
+  r.sliceMode = c.slice ? 1 : 0;
 }
 
 // mean duration in microseconds of fn() on stream s over reps launches,
@@ -2684,6 +2576,11 @@ double time_us(hipStream_t s, F &&fn, int reps = 5) {
 std::string describe(const Run &r, const Sched &c, bool cached) {
   char buf[256];
   std::string sp;
+  if (c.slice) {
+    snprintf(buf, sizeof buf, "%dx%dx%d: slice step (%.1f us a step, kernels per phase %.1f us%s)",
+             r.nR, r.nU, r.nJ, c.sliceUs, c.stepUs, cached ? ", cached" : "");
+    return buf;
+  }
   if (c.lineMode == 1) {
     sp = "register lines";
   } else {
@@ -2760,6 +2657,7 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
   const size_t fDoubles = r.fRows ? std::max<size_t>(r.nVal, (size_t)r.nJ * r.cs) : r.nVal;
   VLS_HIP_CHECK(hipMalloc(&tmp, fDoubles * sizeof(double)));
   r.f = tmp;
+  const int64_t chains = r.nChains;
   try {
     auto time_kick = [&](int mode) {
       r.kickMode = mode;
@@ -2802,7 +2700,42 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
         best.kickUs = us;
       }
     }
+    if (slice_fits(r) && r.nS > 1) {
+      best.slice = true;
+    } else if (slice_fits(r)) {
+      // whole steps on the copy of f, the delay lines left out of the drift
+      r.nChains = 0;
+      apply_sched(r, best);
+      auto copy_f = [&] {
+        VLS_HIP_CHECK(hipMemcpyAsync(tmp, f0, (size_t)r.nVal * sizeof(double),
+                                     hipMemcpyDeviceToDevice, s));
+      };
+      copy_f();
+      best.stepUs = time_us(s, [&] {
+        if (r.sp.no_linking) {
+          launch_spline(r, r.f, s, nullptr);
+          launch_drift(r, s);
+        }
+        if (kick_in_rsolve(r)) {
+          launch_kick_rsolve(r, s, nullptr);
+          launch_spline_v_timed(r, s, nullptr);
+        } else {
+          launch_spline_kick(r, s, nullptr);
+          launch_spline(r, r.f, s, nullptr);
+        }
+        launch_drift(r, s);
+      });
+      copy_f();
+      launch_slice_start(r, s);
+      best.sliceUs = time_us(s, [&] {
+        launch_slice_kick(r, s, nullptr);
+        launch_slice_drift(r, s, false);
+      });
+      best.slice = best.sliceUs < best.stepUs;
+      r.nChains = chains;
+    }
   } catch (...) {
+    r.nChains = chains;
     r.f = f0;
     (void)hipStreamSynchronize(s);
     (void)hipFree(tmp);

@@ -1,0 +1,950 @@
+// A step in two launches for grids whose padded slice of coefficients fits in
+// the LDS of a CU (gfx950, FP64).
+//
+// Everything of a step but the moment is local to a slice (fixed j), and the
+// kick to a column (fixed j, r).  With a kernel per phase a small grid spends
+// its step on launches and on the first loads of each kernel, with a few lines
+// per CU in flight.  Here
+//   k_kick_tile    takes a tile of a slice's columns through the column
+//                  splines and the kick in LDS; meanwhile each block sums the
+//                  moment partials of all slices for itself (they come from
+//                  L2) into the acceleration, so that no launch and no block
+//                  waits for the reduction;
+//   k_slice_drift  takes a slice through the r- and v-solves in LDS, then
+//                  drifts its points and forms the slice's moment partials of
+//                  the new f.  Where the slices are fewer than the CUs several
+//                  blocks share a slice: each solves it for itself (the CUs
+//                  would idle) and drifts a part of its rows.
+// What bounds both: the serial chains of the solves (a lane per line: at
+// 129x129x64 5.5 us each of three) and the first loads (3 and 5 us); then the
+// drift's points (8 evaluations a wave and block, 0.3 us each) and the way of
+// the group sums to the partials (4 us).  The operations and their order are
+// those of the kernels per phase (vls_kernels.hip): same bits.  Against those,
+// a step of 65x65x32 takes 26 us for 32, 91x81x80 36 for 92, 181x81x80 50 for
+// 122, 129x129x64 47 for 60 and 69 for 100 without linking, two species of
+// 97x97x48 82 for 150.  One launch for the whole step, a block per slice, was
+// 29 us at 65x65x32 but 69 at 129x129x64: its evaluations had 64 of the CUs.
+#pragma clang fp contract(off)
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdlib>
+
+#include "vls_device.hpp"
+#include "vls_div.hpp"
+#include "vls_internal.hpp"
+#include "vls_tile.hpp"
+
+namespace vls {
+
+namespace {
+
+constexpr int kMaxLds = 163840;  // LDS of one, all of which a block may take
+
+// i / d == __umulhi(i, magic(d)) for i d < 2^32
+inline unsigned magic(int d) { return (unsigned)(((1ull << 32) + d - 1) / d); }
+
+// The pivots of the natural spline solve, rows 1..kHead and (last) all later
+// ones: super-diagonal u, RN(1/d) and its remainder.  They are the same for
+// every grid (the first row is c_0 - 2 c_1 + c_2 = 0 whatever the spacing);
+// literals cost a row nothing, where an LDS table is read behind the row
+// before's write (its address could be the table's): 250 cycles a head row.
+// The set-up compares them with the run's table (slice_pivots).
+constexpr double kPivU[kHead + 2] = {0.0, 0x0.0p+0, 0x1.0000000000000p-2, 0x1.1111111111111p-2,
+    0x1.1249249249249p-2, 0x1.125f8a6956f76p-2, 0x1.1261261261262p-2, 0x1.126143a0aba9dp-2,
+    0x1.126145bfe7dedp-2, 0x1.126145e6e884bp-2, 0x1.126145e9b5624p-2, 0x1.126145e9e8da4p-2,
+    0x1.126145e9ec8c4p-2, 0x1.126145e9ecd02p-2, 0x1.126145e9ecd50p-2, 0x1.126145e9ecd56p-2,
+    0x1.126145e9ecd57p-2, 0x1.126145e9ecd57p-2};
+constexpr double kPivRd[kHead + 2] = {0.0, 0x1.0000000000000p+0, 0x1.8000000000000p+0,
+    0x1.999999999999ap+0, 0x1.9b6db6db6db6ep+0, 0x1.9b8f4f9e02732p+0, 0x1.9b91b91b91b93p+0,
+    0x1.9b91e571017ebp+0, 0x1.9b91e89fdbce4p+0, 0x1.9b91e8da5cc71p+0, 0x1.9b91e8de90137p+0,
+    0x1.9b91e8dedd476p+0, 0x1.9b91e8dee2d26p+0, 0x1.9b91e8dee3384p+0, 0x1.9b91e8dee33f8p+0,
+    0x1.9b91e8dee3401p+0, 0x1.9b91e8dee3402p+0, 0x1.9b91e8dee3402p+0};
+constexpr double kPivRl[kHead + 2] = {0.0, 0x0.0p+0, 0x1.8000000000000p-54,
+    -0x1.999999999999ap-54, -0x1.9a1f58d0fac68p-54, 0x1.8d66824e61708p-56, -0x1.2679ca12c88eep-54,
+    0x1.e50bd0f2693f2p-54, 0x1.e146a6c0ff79cp-54, -0x1.d42b2b514981bp-54, 0x1.fa760ee70d1c5p-57,
+    0x1.85c55fb87d6e8p-55, 0x1.aa34d354ae79bp-57, -0x1.38360a9a30f98p-54, 0x1.80e9a827b6badp-60,
+    0x1.ac2a59571744bp-57, 0x1.60e0f4f57eecap-54, 0x1.60e0f4f57eecap-54};
+constexpr double kC16 = 1.0 / 6.0;
+
+// The constants of an axis's last row.
+struct LineTab {
+  double hi2, p, q, rq;
+};
+__device__ __forceinline__ void line_tab(LineTab *l, const ThomasAxis &ax) {
+  l->hi2 = ax.hi2, l->p = ax.p, l->q = ax.q, l->rq = ax.rq;
+}
+// The natural spline solve of a line in LDS, in place (thomas_forward and
+// thomas_backward of the kernels per phase): p[k st] holds the right-hand
+// side of row k = 1..L and receives the L + 2 coefficients.  The rows go by
+// in chunks of kPF whose reads are issued a chunk ahead.  The forward values
+// of the head and of the last rows (whole chunks, kNY rows at most) wait in
+// registers for the way down, the others in place.  A row takes about 36
+// cycles up and 34 down in registers (a chain of 4 and 2 dependent FP64
+// operations of 5 cycles, a DS read of 15 or a write of 20), 60 and 50 in
+// place.
+constexpr int kPF = 8, kNY = 80;
+static_assert(kHead == 2 * kPF, "the head is two chunks");
+
+__device__ __forceinline__ void lds_line(double *p, int st, int L, const LineTab &ax) {
+  // uniform, and unknown before this point: what is formed from them would
+  // otherwise be kept in scalar registers across the kernel's loops (and
+  // spilled to vector lanes)
+  st = __builtin_amdgcn_readfirstlane(st);
+  L = __builtin_amdgcn_readfirstlane(L);
+  asm volatile("" : "+s"(st), "+s"(L));
+  const double hi2 = ax.hi2, last1 = ax.p, lastQ = ax.q, lastRq = ax.rq;
+  const double rdS = kPivRd[kHead + 1], rlS = kPivRl[kHead + 1], uS = kPivU[kHead + 1];
+  double prev = 0.0, prev2 = 0.0;     // y_k, y_{k-1} of the last row done (y_0 = 0)
+  double *lp = p + st, *sp = p + st;  // next row to read, next to write
+  auto up = [&](double rhs, double rd, double rl) {
+    const double y = div_pivot(rhs - kC16 * prev, rd, rl);
+    prev2 = prev;
+    prev = y;
+    return y;
+  };
+  auto put = [&](double y, int step) {
+    *sp = y;
+    sp += step;
+  };
+  auto load = [&](double (&v)[kPF], int step) {  // kPF rows in the direction of step
+#pragma unroll
+    for (int q = 0; q < kPF; q++) {
+      v[q] = *lp;
+      lp += step;
+    }
+  };
+  double yh[kHead], y[kNY];
+  // chunks in registers, and rows between the head and them
+  int nc = L > kHead ? min((L - kHead) / kPF, kNY / kPF) : 0;
+  const int nl = L - kHead - nc * kPF;
+  if (nc == 0) {
+    // short lines: the head's rows that exist, then fewer than kPF others
+#pragma unroll
+    for (int k = 1; k <= kHead; k++)
+      if (k <= L) yh[k - 1] = up(p[k * st], kPivRd[k], kPivRl[k]);
+#pragma unroll
+    for (int k = 0; k < kPF - 1; k++)
+      if (k < nl) y[k] = up(p[(kHead + 1 + k) * st], rdS, rlS);
+    sp = p + (L + 1) * st;
+  } else {
+    double a[kPF], b[kPF];
+    load(a, st);
+    load(b, st);
+#pragma unroll
+    for (int q = 0; q < kPF; q++) yh[q] = up(a[q], kPivRd[1 + q], kPivRl[1 + q]);
+    load(a, st);
+#pragma unroll
+    for (int q = 0; q < kPF; q++)
+      yh[kPF + q] = up(b[q], kPivRd[1 + kPF + q], kPivRl[1 + kPF + q]);
+    // a: the next kPF rows (there are that many: nc >= 1); whole chunks in
+    // place, then the rest of them
+    sp += kHead * st;
+    int k = nl;
+#pragma unroll 1
+    for (; k >= kPF; k -= kPF) {
+#pragma unroll
+      for (int q = 0; q < kPF; q++) b[q] = a[q];
+      load(a, st);
+#pragma unroll
+      for (int q = 0; q < kPF; q++) put(up(b[q], rdS, rlS), st);
+    }
+    if (k > 0) {
+#pragma unroll
+      for (int q = 0; q < kPF - 1; q++)
+        if (q < k) put(up(a[q], rdS, rlS), st);
+      lp = sp;
+      load(a, st);
+    }
+#pragma unroll
+    for (int c = 0; c < kNY / kPF; c++) {
+      if (c < nc) {
+        if (c + 1 < nc) load(b, st);
+#pragma unroll
+        for (int q = 0; q < kPF; q++) y[c * kPF + q] = up(a[q], rdS, rlS);
+#pragma unroll
+        for (int q = 0; q < kPF; q++) a[q] = b[q];
+      }
+    }
+    sp += nc * kPF * st;
+  }
+  double tt = 0.0 - hi2 * prev2;
+  tt = tt - last1 * prev;
+  double cn = div_known(tt, lastQ, lastRq), c2 = cn;
+  put(cn, -st);  // row L + 1
+  auto down = [&](double yk, double u) {
+    const double c = yk - u * cn;
+    put(c, -st);
+    c2 = cn;
+    cn = c;
+  };
+  if (nc == 0) {
+#pragma unroll
+    for (int k = kPF - 2; k >= 0; k--)
+      if (k < nl) down(y[k], uS);
+#pragma unroll
+    for (int k = kHead; k >= 1; k--)
+      if (k <= L) down(yh[k - 1], kPivU[k]);
+  } else {
+    asm volatile("" : "+s"(nc));  // compared again on the way down
+    double a[kPF], b[kPF];
+    // the rows in place after the registers'
+    lp = p + (nl + kHead) * st;
+    int k = nl;
+    const int rest = k % kPF;
+#pragma unroll
+    for (int q = 0; q < kPF - 1; q++) b[q] = lp[-min(q, rest) * st];
+#pragma unroll
+    for (int c = kNY / kPF - 1; c >= 0; c--) {
+      if (c < nc) {
+#pragma unroll
+        for (int q = kPF - 1; q >= 0; q--) down(y[c * kPF + q], uS);
+      }
+    }
+    lp -= rest * st;
+    load(a, -st);  // (the head's rows if no whole chunk is left: not used)
+#pragma unroll
+    for (int q = 0; q < kPF - 1; q++)
+      if (q < rest) down(b[q], uS);
+    k -= rest;
+#pragma unroll 1
+    for (; k >= kPF; k -= kPF) {
+#pragma unroll
+      for (int q = 0; q < kPF; q++) b[q] = a[q];
+      load(a, -st);
+#pragma unroll
+      for (int q = 0; q < kPF; q++) down(b[q], uS);
+    }
+#pragma unroll
+    for (int q = kHead - 1; q >= 0; q--) down(yh[q], kPivU[q + 1]);
+  }
+  // c_0 = (A03 - A01 c_1) - A02 c_2 with A03 = 0, A01 = -2, A02 = 1
+  *sp = (0.0 - -2.0 * cn) - 1.0 * c2;
+}
+
+// ---------------------------------------------------------------- kick
+struct KickArgs {
+  const double *src;   // f [nS][nJ][nU][nR]
+  double *dst;         // the kicked f (may be src)
+  const double *P;     // moment partials [nJ][nR] of f
+  double *dKeep;       // the column splines [j][m][r], slice stride cs (null: not kept)
+  const double *gfac, *U_Val;
+  double *dM, *Mx, *acc, *mTot;
+  int32_t *head;       // the delay lines' heads, advanced by roll (null: none)
+  const int32_t *len;
+  int64_t nChains, nVal, cs;
+  double Ulo, Uhi, start_v, hinv_v;
+  ThomasAxis tv;
+  int nR, nU, nJ, nS;
+  int W, nT;           // columns of a tile, tiles of a slice
+  unsigned mulW, mulR;  // i / W == __umulhi(i, mulW), i / nR == __umulhi(i, mulR)
+  int roll;
+};
+
+// kTK threads: one wave solves, the others sum the moment.  512 where every
+// block has a CU for itself (twice the waves in the evaluation), else 256 (two
+// blocks on a CU, two solves side by side).
+
+inline size_t kick_lds(int nR, int nU, int nJ, int W) {
+  const size_t nC = (nJ + kJC - 1) / kJC;
+  return ((size_t)W * (nU + 3) + nU + nR + nC * nR + 1) * sizeof(double) + sizeof(LineTab);
+}
+
+// The acceleration in LDS by one wave: dM[r] from the chunk sums Sc [nC][nR],
+// the serial prefix, times the factors that accs holds (out: with the global
+// outputs).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ __forceinline__ void wave_accel(double *Sc, double *accs, int nC, int nR, int lane,
+                                           bool out, const KickArgs &a) {
+  for (int r = lane; r < nR; r += 64) {
+    double m = 0.0;
+    for (int c = 0; c < nC; c++) m += Sc[c * nR + r];
+    Sc[r] = m;
+    if (out) a.dM[r] = m;
+  }
+  wave_sync();
+  if (lane == 0) {
+    // 16 entries a batch
+    double prev = 0.0;
+    int r = 0;
+#pragma unroll 1
+    for (; r + 16 <= nR; r += 16) {
+      double x[16];
+#pragma unroll
+      for (int k = 0; k < 16; k++) x[k] = Sc[r + k];
+#pragma unroll
+      for (int k = 0; k < 16; k++) {
+        const double y = x[k];
+        x[k] = prev;
+        prev += y;
+      }
+#pragma unroll
+      for (int k = 0; k < 16; k++) Sc[r + k] = x[k];
+    }
+#pragma unroll 1
+    for (; r < nR; r++) {
+      const double y = Sc[r];
+      Sc[r] = prev;
+      prev += y;
+    }
+    if (out) *a.mTot = prev;
+  }
+  wave_sync();
+  for (int r = lane; r < nR; r += 64) {
+    const double m = Sc[r], x = m * accs[r];
+    accs[r] = x;
+    if (out) {
+      a.Mx[r] = m;
+      a.acc[r] = x;
+    }
+  }
+}
+
+template <int kTK>
+__global__ void __launch_bounds__(kTK) k_kick_tile(KickArgs a) {
+  extern __shared__ double lds[];
+  const int nR = a.nR, nU = a.nU, nJ = a.nJ, W = a.W;
+  const int nC = (nJ + kJC - 1) / kJC;
+  double *D = lds, *Us = D + W * (nU + 3), *accs = Us + nU;
+  double *Sc = accs + nR;
+  LineTab *hv = (LineTab *)(Sc + nC * nR);
+  unsigned *ready = (unsigned *)(hv + 1);  // waves whose chunk sums are in Sc
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int j = tile / a.nT, c0 = (tile - j * a.nT) * W;
+  const int wid = min(W, nR - c0);  // columns of this tile
+
+  if (a.head)
+    for (int64_t k = (int64_t)blockIdx.x * kTK + t; k < a.nChains; k += (int64_t)gridDim.x * kTK) {
+      const int h = a.head[k] + a.roll, len = a.len[k];
+      a.head[k] = h >= len ? h - len : h;
+    }
+  if (t == 0) {
+    line_tab(hv, a.tv);
+    *ready = 0;
+  }
+  for (int u = t; u < nU; u += kTK) Us[u] = a.U_Val[u];
+  for (int r = t; r < nR; r += kTK) accs[r] = a.gfac[r];
+  for (int i = t; i < W; i += kTK) D[(nU + 2) * W + i] = 0.0;  // read with weight 0
+
+  for (int s = 0; s < a.nS; s++) {
+    const size_t at = (size_t)s * a.nVal + (size_t)j * nU * nR + c0;
+    const double *fj = a.src + at;
+    double *fo = a.dst + at;
+    // the tile's columns, 16 values of each thread in flight
+    constexpr int kB = 16;
+    const int n = nU * W;
+#pragma unroll 1
+    for (int b = t; b < n; b += kB * kTK) {
+      double v[kB];
+#pragma unroll
+      for (int q = 0; q < kB; q++) {
+        const int i = min(b + q * kTK, n - 1);
+        const int u = __umulhi((unsigned)i, a.mulW), c = i - u * W;
+        v[q] = fj[(size_t)u * nR + min(c, wid - 1)];
+      }
+#pragma unroll
+      for (int q = 0; q < kB; q++)
+        if (b + q * kTK < n) D[W + b + q * kTK] = v[q];
+    }
+    __syncthreads();
+    if (w == 0) {
+      if (lane < W) lds_line(D + lane, W, nU, *hv);
+    } else if (s == 0) {
+      // chunk sums of the partials (k_moment_chunks), a thread per (chunk, r)
+#pragma unroll 1
+      for (int i = t - 64; i < nC * nR; i += kTK - 64) {
+        const int c = __umulhi((unsigned)i, a.mulR), r = i - c * nR, jb = c * kJC;
+        const int je = min(nJ, jb + kJC);
+        double x[kJC];
+#pragma unroll
+        for (int k = 0; k < kJC; k++) x[k] = a.P[(size_t)min(jb + k, nJ - 1) * nR + r];
+        double sum = 0.0;
+#pragma unroll
+        for (int k = 0; k < kJC; k++)
+          if (jb + k < je) sum += x[k];
+        Sc[i] = sum;
+      }
+      // the last wave goes on to the acceleration once the others' chunk sums
+      // are in (they run beside it: the wait ends), while wave 0 still solves
+      constexpr int kOthers = kTK / 64 - 2;
+      if (w < kTK / 64 - 1) {
+        wave_sync();
+        if (lane == 0)
+          __hip_atomic_fetch_add(ready, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      } else {
+        while (__hip_atomic_load(ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < kOthers)
+          __builtin_amdgcn_s_sleep(1);
+        wave_sync();
+        wave_accel(Sc, accs, nC, nR, lane, tile == 0, a);
+      }
+    }
+    __syncthreads();
+    // the kick's evaluation (k_kick_cols)
+    if (a.dKeep) {
+      double *dk = a.dKeep + (size_t)j * a.cs + c0;
+      const int nk = (nU + 2) * W;
+      for (int i = t; i < nk; i += kTK) {
+        const int m = __umulhi((unsigned)i, a.mulW), c = i - m * W;
+        if (c < wid) dk[(size_t)m * nR + c] = D[i];
+      }
+    }
+    // four points' reads together, then their sums
+    constexpr int kE = 4;
+#pragma unroll 1
+    for (int b = t; b < n; b += kE * kTK) {
+      double d[kE][4], yy[kE];
+      bool in[kE];
+      int o[kE];
+#pragma unroll
+      for (int q = 0; q < kE; q++) {
+        const int i = min(b + q * kTK, n - 1);
+        const int u = __umulhi((unsigned)i, a.mulW), c = i - __umul24(u, W);
+        const double newU = Us[u] + accs[min(c0 + c, nR - 1)];
+        in[q] = !(newU <= a.Ulo) && !(newU >= a.Uhi);
+        double y = in[q] ? (newU - a.start_v) * a.hinv_v : 0.0;
+        int m;
+        split(y, m, y);
+        yy[q] = y;
+        // row m + 3 is past the column only at y == 0, with weight 0 (zeroed)
+        const double *p = D + __umul24(m, W) + c;
+#pragma unroll
+        for (int k = 0; k < 4; k++) d[q][k] = p[k * W];
+        o[q] = c < wid && b + q * kTK < n ? (int)(__umul24(u, nR) + c) : -1;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < kE; q++) {
+        const double x = kick_value(yy[q], d[q][0], d[q][1], d[q][2], d[q][3]);
+        if (o[q] >= 0) fo[o[q]] = in[q] ? x : 0.0;
+      }
+    }
+    if (s + 1 < a.nS) __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------- drift
+struct SliceArgs {
+  const double *src;  // the values to drift [nS][nJ][nU][nR]
+  double *f;      // the drifted ones (src itself with one block per slice: the blocks of a
+                  // slice all read all of it)
+  double *P;      // moment partials [nJ][nR] of the new f (null: none)
+  double *G;      // [nJ][nG][nR] group sums where several blocks share a slice
+  unsigned *cnt;  // [nJ] counters of those blocks (zero between launches)
+  double *cOut;   // the drift's coefficients of the last species (null: not kept)
+  const double *Ct1, *dU, *dR;
+  const double2 *feet;
+  ChainTables ch;                       // vals: the first species' plane; roll not used
+  const int64_t *chPoint;               // the delay lines' points
+  const int32_t *chOrder, *chStart;     // the delay lines by slice: chOrder[chStart[j]..]
+  int64_t nVal, nCells, cs;
+  ThomasAxis tr, tv;
+  int nR, nU, nJ, nS;
+  unsigned mulR;   // i / nR == __umulhi(i, mulR) for the slice's point indices
+  int hOff;        // ring position of this drift relative to the heads: 0 or -1
+  int parts;       // blocks per slice
+  int gPart;       // groups of 16 rows of a block
+  int maxLines;    // delay lines of a slice, at most
+  int loose;       // some delay-line points have no line
+};
+
+// Threads: 8 waves, 2 on each SIMD, with 256 VGPRs each, so that a line keeps
+// 96 rows in registers.
+constexpr int kT = 512;
+
+// LDS of k_slice_drift: the coefficients (rows of odd pitch, one row more than
+// the padded slice for stencils on the last knot), dU, the row after the
+// block's rows, the axes' constants and the slice's delay lines.
+__host__ __device__ inline int slice_pitch(int nR) { return (nR + 2) | 1; }
+__host__ __device__ inline int slice_coef(int nR, int nU) { return slice_pitch(nR) * (nU + 3) + 8; }
+struct LineRec;
+size_t slice_lds(int nR, int nU, int maxLines);
+
+// The thread's index as a value the compiler cannot connect with its other
+// uses (each phase then forms its addresses for itself instead of keeping them
+// in registers from the phase before).
+__device__ __forceinline__ int fresh(int t) {
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// Stores and loads between blocks of a launch: through memory (system scope),
+// acknowledged before the count that tells of them (as moment_tail).
+__device__ __forceinline__ void coherent_store(double *p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ double coherent_load(const double *p) {
+  return __hip_atomic_load(const_cast<double *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void wait_stores() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// The moment's group sums of slice j over the groups [g0, g1) of 16 rows, in
+// the order of moment_cols_block and k_moment_partial_sp: a wave takes a group
+// (its 16 rows and the row after them) of 63 columns.  Row uH comes from halo
+// (LDS; the block that owns it may not have written it).  put(g, r, sum).
+template <class PUT>
+__device__ __forceinline__ void group_sums(const SliceArgs &a, int j, int g0, int g1,
+                                           const double *dUs, const double *halo, int uH, PUT put) {
+  const int nR = a.nR, nU = a.nU;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nX = (nR + 62) / 63;
+  const double ct = a.Ct1[j];
+  const double *fj = a.f + (size_t)j * nU * nR;
+  for (int task = w; task < (g1 - g0) * nX; task += kT / 64) {
+    const int gi = task / nX, g = g0 + gi, x = task - gi * nX;
+    const int u0 = 16 * g, r = x * 63 + lane, rc = min(r, nR - 1);
+    const bool term = lane < 63 && r < nR - 1;
+    const double *col = fj + rc;
+    const double dr = term ? a.dR[r] : 0.0;
+    double s = 0.0;
+    if (a.nS == 1) {
+      double row[17];
+#pragma unroll
+      for (int q = 0; q < 17; q++) row[q] = col[(size_t)min(u0 + q, nU - 1) * nR];
+      if (u0 + 16 == uH) row[16] = halo[rc];
+      double own = row[0], next = lane_next(own);
+#pragma unroll
+      for (int q = 0; q < 16; q++) {
+        const double b = row[q + 1], bN = lane_next(b);
+        if (u0 + q < nU - 1) {
+          const double sum4 = ((own + next) + b) + bN;
+          s += (((ct * dUs[u0 + q]) * 0.25) * dr) * sum4;
+        }
+        own = b;
+        next = bN;
+      }
+    } else {
+      // a few rows at a time: every species' values of a cell meet in its
+      // average (one block per slice: no halo)
+      for (int q0 = 0; q0 < 16; q0 += 4) {
+        double avg[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int k = 0; k < a.nS; k++) {
+          double row[5];
+#pragma unroll
+          for (int q = 0; q < 5; q++)
+            row[q] = col[(size_t)k * a.nVal + (size_t)min(u0 + q0 + q, nU - 1) * nR];
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const double own = row[q], b = row[q + 1];
+            avg[q] += (((own + lane_next(own)) + b) + lane_next(b)) * 0.25;
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          if (u0 + q0 + q < nU - 1) s += ((ct * dUs[u0 + q0 + q]) * dr) * avg[q];
+      }
+    }
+    if (lane < 63 && r < nR) put(g, r, s);
+  }
+}
+
+// P[j][r] from the group sums get(g, r): ((G0 + G1) + G2) + G3 per block of 64
+// rows, the blocks left to right.
+template <class GET>
+__device__ __forceinline__ void group_combine(const SliceArgs &a, int j, GET get) {
+  const int nR = a.nR, nU = a.nU, nG = (nU - 1 + 15) / 16, nW = (nU + 63) / 64;
+  for (int r = threadIdx.x; r < nR; r += kT) {
+    double Pj = 0.0;
+    for (int b = 0; b < nW; b++) {
+      double v[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) v[q] = 4 * b + q < nG ? get(4 * b + q, r) : 0.0;
+      const double W = ((v[0] + v[1]) + v[2]) + v[3];
+      Pj = b == 0 ? W : Pj + W;
+    }
+    a.P[(size_t)j * nR + r] = r < nR - 1 ? Pj : 0.0;
+  }
+}
+
+// The partials alone (before the first step of a call).
+__global__ void __launch_bounds__(kT) k_slice_moment(SliceArgs a) {
+  extern __shared__ double lds[];
+  double *dUs = lds, *G = lds + a.nU;
+  const int nR = a.nR;
+  for (int u = threadIdx.x; u < a.nU; u += kT) dUs[u] = a.dU[u];
+  __syncthreads();
+  group_sums(a, blockIdx.x, 0, (a.nU - 1 + 15) / 16, dUs, nullptr, -1,
+             [&](int g, int r, double s) { G[g * nR + r] = s; });
+  __syncthreads();
+  group_combine(a, blockIdx.x, [&](int g, int r) { return G[g * nR + r]; });
+}
+
+// The n values of a slice into columns 1..nR of rows 1..nU of the coefficients,
+// kB of each thread in flight (n <= kB kT): one round trip to memory.
+template <int kB>
+__device__ __forceinline__ void load_slice(const double *sj, double *C, int n, int nR, int ps,
+                                           unsigned mulR) {
+  double v[kB];
+  const int i0 = fresh(threadIdx.x);
+#pragma unroll
+  for (int q = 0; q < kB; q++) v[q] = sj[min(i0 + q * kT, n - 1)];
+  __builtin_amdgcn_sched_barrier(0);
+  const int i1 = fresh(threadIdx.x);
+#pragma unroll
+  for (int q = 0; q < kB; q++) {
+    const int i = i1 + q * kT;
+    if (i < n) C[ps + 1 + i + __umulhi((unsigned)i, mulR) * (unsigned)(ps - nR)] = v[q];
+  }
+}
+static_assert(40 * kT * sizeof(double) >= 163840, "a slice that fits in LDS fits in load_slice<40>");
+
+// A delay line of the slice while its block waits for the solves.
+struct LineRec {
+  double bxr, bxu, front;  // back foot (bxr < 0: outside), value at the front
+  int64_t back;            // index of the slot behind the front in vals
+  int il;                  // point in the slice (-1: of another block's rows)
+  int pad;
+};
+
+__global__ void __launch_bounds__(kT) k_slice_drift(SliceArgs a) {
+  extern __shared__ double lds[];
+  const int nR = a.nR, nU = a.nU;
+  const int n = nR * nU, ps = slice_pitch(nR), S = nR + 2, nG = (nU - 1 + 15) / 16;
+  double *C = lds, *halo = C + slice_coef(nR, nU), *dUs = halo + nR;
+  LineTab *hr = (LineTab *)(dUs + nU), *hv = hr + 1;
+  LineRec *rec = (LineRec *)(hv + 1);  // [maxLines]
+  int *lastBlock = (int *)(rec + a.maxLines);
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  // the parts of a slice on one XCD (its f in one L2)
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int j = tile / a.parts, part = tile - j * a.parts;
+  // this block's groups of 16 rows, and its rows
+  const int g0 = part * a.gPart, g1 = min(nG, g0 + a.gPart);
+  const int uA = 16 * g0, uB = part == a.parts - 1 ? nU : 16 * g1;
+
+  if (t == 0) {
+    line_tab(hr, a.tr);
+    line_tab(hv, a.tv);
+  }
+  for (int u = t; u < nU; u += kT) dUs[u] = a.dU[u];
+  // what a stencil on the last knot reads with weight 0: the row after the
+  // padded slice, and the column after each row
+  for (int i = t; i < ps + 8; i += kT) C[(nU + 2) * ps + i] = 0.0;
+  if (ps > S)
+    for (int m = t; m < nU + 2; m += kT) C[m * ps + S] = 0.0;
+
+  const bool hasHalo = a.P && uB < nU;
+  const int lines0 = a.ch.n ? a.chStart[j] : 0;
+  const int nLines = a.ch.n ? a.chStart[j + 1] - lines0 : 0;
+#pragma unroll 1
+  for (int s = 0; s < a.nS; s++) {
+    const size_t at = (size_t)s * a.nVal + (size_t)j * n;
+    const double *sj = a.src + at;
+    double *fj = a.f + at;
+    double *vals = a.ch.vals + (size_t)s * a.nCells;
+    // the slice's values, the right-hand sides of the r-solve
+    if (n <= 10 * kT)
+      load_slice<10>(sj, C, n, nR, ps, a.mulR);
+    else if (n <= 20 * kT)
+      load_slice<20>(sj, C, n, nR, ps, a.mulR);
+    else
+      load_slice<40>(sj, C, n, nR, ps, a.mulR);
+    __syncthreads();
+    // the solves of the rows, then of the padded columns.  One loop, so that
+    // the solver, unrolled over its registers, is in the kernel once.
+#pragma unroll 1
+    for (int ph = 0; ph < 2; ph++) {
+      const int lines = ph == 0 ? nU : S, step = ph == 0 ? ps : 1;
+      double *first = C + (ph == 0 ? ps : 0);
+      const LineTab *ax = ph == 0 ? hr : hv;
+#pragma unroll 1
+      for (int i = t; i < lines; i += kT)
+        lds_line(first + i * step, ph == 0 ? 1 : ps, ph == 0 ? nR : nU, *ax);
+      if (ph == 0) {
+        // meanwhile the waves without a row bring the first lines of the feet
+        // into L2, and the last one collects the delay lines (three dependent
+        // loads that the drift would otherwise wait for)
+        const int free0 = (lines + 63) / 64 * 64;
+        if (t >= free0) {
+          const double2 *fp = a.feet + (size_t)j * n;
+          double x[4];
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+            x[q] = fp[min(uA * nR + (t - free0 + q * (kT - free0)) * 8, n - 1)].x;
+          asm volatile("" ::"v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
+        }
+        if (w == kT / 64 - 1)
+          for (int q = lane; q < nLines; q += 64) {
+            const int k = a.chOrder[lines0 + q], len = a.ch.len[k];
+            const int il = (int)(a.chPoint[k] - (int64_t)j * n);
+            const int u = __umulhi((unsigned)il, a.mulR);
+            int h = a.ch.head[k] + a.hOff;
+            if (h < 0) h += len;
+            const int64_t off = a.ch.off[k];
+            LineRec l;
+            l.bxr = a.ch.bout[k] ? -1.0 : a.ch.bxr[k];
+            l.bxu = a.ch.bxu[k];
+            l.front = vals[off + h];
+            l.back = off + (h == 0 ? len - 1 : h - 1);
+            l.il = (u >= uA && u < uB) || (hasHalo && u == uB) ? il : -1;
+            rec[q] = l;
+          }
+      }
+      __syncthreads();
+    }
+    if (a.cOut && part == 0 && s == a.nS - 1) {
+      double *co = a.cOut + (size_t)j * a.cs;
+      for (int m = w; m < nU + 2; m += kT / 64)
+        for (int k = lane; k < S; k += 64) co[m * S + k] = C[m * ps + k];
+    }
+    // the delay lines (drift_chain), a thread each, from the last one down
+    for (int q = kT - 1 - t; q < nLines; q += kT) {
+      const LineRec l = rec[q];
+      if (l.il < 0) continue;
+      if (l.il >= uB * nR) {
+        halo[l.il - uB * nR] = l.front;
+      } else {
+        vals[l.back] = l.bxr < 0.0 ? 0.0 : eval_c(C, ps, l.bxr, l.bxu);
+        fj[l.il] = l.front;
+      }
+    }
+    // the drift (k_drift) of this block's rows, the feet of the next kA points
+    // loaded ahead; with the row after them for the moment
+    const double2 *ft = a.feet + (size_t)j * n;
+    const int iB = uB * nR, iE = iB + (hasHalo ? nR : 0);
+    constexpr int kA = 4;
+    double2 nx[kA];
+    const int iW = uA * nR + w * 64;  // the wave's first point
+#pragma unroll
+    for (int q = 0; q < kA; q++) nx[q] = ft[min(iW + lane + q * kT, n - 1)];
+#pragma unroll 1
+    for (int b = iW; b < iE; b += kA * kT) {
+#pragma unroll
+      for (int q = 0; q < kA; q++) {
+        if (b + q * kT >= iE) break;
+        const int i = b + q * kT + lane;
+        const double2 cu = nx[q];
+        nx[q] = ft[min(i + kA * kT, n - 1)];
+        const bool e = cu.x > kFootOut;
+        // the 16 reads together, before the sums
+        CStencil st;
+        eval_c_fetch(C, ps, e ? cu.x : 0.0, e ? cu.y : 0.0, st);
+        __builtin_amdgcn_sched_barrier(0);
+        double x = eval_c_sum(st);
+        x = e ? x : 0.0;
+        if (cu.x >= kFootOut) {  // (delay lines: above)
+          if (i < iB)
+            fj[i] = x;
+          else if (i < iE)
+            halo[i - iB] = x;
+        }
+      }
+    }
+    if (a.loose) {
+      // delay-line points without a line: f keeps its value
+      for (int i = uA * nR + t; i < iE; i += kT) {
+        const double2 cu = ft[i];
+        if (cu.x < kFootOut && cu.y < 0.0) {
+          const double x = sj[i];
+          if (i < iB)
+            fj[i] = x;
+          else
+            halo[i - iB] = x;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (!a.P) return;
+  if (a.parts == 1) {
+    double *G = C;
+    group_sums(a, j, 0, nG, dUs, halo, -1, [&](int g, int r, double s) { G[g * nR + r] = s; });
+    __syncthreads();
+    group_combine(a, j, [&](int g, int r) { return G[g * nR + r]; });
+    return;
+  }
+  // the block that is the last of its slice to leave its group sums combines
+  // them (no block waits for another); it resets the count for the next launch
+  double *G = a.G + (size_t)j * nG * nR;
+  group_sums(a, j, g0, g1, dUs, halo, uB < nU ? uB : -1,
+             [&](int g, int r, double s) { coherent_store(&G[(size_t)g * nR + r], s); });
+  wait_stores();
+  __syncthreads();
+  if (t == 0) {
+    const unsigned o =
+        __hip_atomic_fetch_add(&a.cnt[j], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *lastBlock = o == (unsigned)(a.parts - 1);
+    if (*lastBlock) __hip_atomic_store(&a.cnt[j], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (*lastBlock)
+    group_combine(a, j, [&](int g, int r) { return coherent_load(&G[(size_t)g * nR + r]); });
+}
+
+size_t slice_lds(int nR, int nU, int maxLines) {
+  return (slice_coef(nR, nU) + nR + (size_t)nU + 1) * sizeof(double) + 2 * sizeof(LineTab) +
+         maxLines * sizeof(LineRec);
+}
+
+// Blocks per slice of the drift: as many as keep the grid within one block per
+// CU (of the run's share of them in an ensemble, whose runs execute side by
+// side), each with at least one group of 16 rows (several species: the moment
+// needs all of a slice's planes in one block).
+int slice_parts(const Run &r) {
+  const int nG = (r.nU - 1 + 15) / 16;
+  return r.nS > 1 ? 1 : std::max(1, std::min(nG, r.cus / r.nJ));
+}
+
+SliceArgs slice_args(Run &r) {
+  SliceArgs a{};
+  a.src = a.f = r.f;
+  a.Ct1 = r.Ct1;
+  a.dU = r.dU;
+  a.dR = r.dR;
+  a.feet = (const double2 *)r.feet;
+  a.ch = ChainTables{r.ch_off, r.ch_len, r.ch_head, r.ch_xr, r.ch_xu, r.ch_out, r.ch_vals, r.nChains, 0};
+  a.chPoint = r.ch_point;
+  a.chOrder = r.ch_order;
+  a.chStart = r.ch_start;
+  a.nVal = r.nVal;
+  a.nCells = r.nCells;
+  a.cs = r.cs;
+  a.tr = r.tr;
+  a.tv = r.tv;
+  a.nR = r.nR;
+  a.nU = r.nU;
+  a.nJ = r.nJ;
+  a.nS = r.nS;
+  a.mulR = magic(r.nR);
+  a.G = r.sliceG;
+  a.cnt = r.sliceCnt;
+  const int nG = (r.nU - 1 + 15) / 16, parts = slice_parts(r);
+  a.maxLines = r.maxLines;
+  a.loose = r.nChainFlags > r.nChains;
+  a.gPart = (nG + parts - 1) / parts;
+  a.parts = (nG + a.gPart - 1) / a.gPart;
+  return a;
+}
+
+void launch_drift(Run &r, SliceArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL(k_slice_drift, dim3(a.nJ * a.parts), dim3(kT), slice_lds(a.nR, a.nU, a.maxLines), s, a);
+}
+
+// where the kick leaves f for the drift
+double *kicked(Run &r) { return r.sliceF ? r.sliceF : r.f; }
+
+// columns of a tile of the kick: the fewest tiles of at most 64 columns, or
+// more of them while they still find idle CUs (down to 16 columns)
+int kick_width(const Run &r) {
+  int nT = (r.nR + 63) / 64;
+  while (r.nJ * (nT + 1) <= r.cus && (r.nR + nT) / (nT + 1) >= 16) nT++;
+  return (r.nR + nT - 1) / nT;
+}
+
+}  // namespace
+
+// Whether the set-up's table holds the pivots that lds_line has as literals.
+bool slice_pivots(const ThomasAxis &ax, const double *u, const double *rd, const double *rl) {
+  if (ax.c16 != kC16 || ax.A01 != -2.0 || ax.A02 != 1.0 || ax.A03 != 0.0) return false;
+  for (int k = 1; k <= ax.M - 2; k++) {
+    const int h = k <= kHead ? k : kHead + 1;
+    if (u[k] != kPivU[h] || rd[k] != kPivRd[h] || rl[k] != kPivRl[h]) return false;
+  }
+  return true;
+}
+
+bool slice_shape(const Run &r, int maxLdsPerBlock) {
+  return maxLdsPerBlock >= kMaxLds && slice_lds(r.nR, r.nU, r.maxLines) <= (size_t)kMaxLds &&
+         kick_lds(r.nR, r.nU, r.nJ, kick_width(r)) <= (size_t)kMaxLds;
+}
+
+size_t slice_group_doubles(const Run &r) { return (size_t)r.nJ * ((r.nU + 14) / 16) * r.nR; }
+bool slice_shared(const Run &r) { return slice_parts(r) > 1; }
+
+void configure_slice(int maxLdsPerBlock) {
+  for (const void *fn : {(const void *)k_kick_tile<256>, (const void *)k_kick_tile<512>,
+                         (const void *)k_slice_drift, (const void *)k_slice_moment})
+    VLS_HIP_CHECK(
+        hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxLdsPerBlock));
+}
+
+bool slice_fits(const Run &r) {
+  return r.sliceG && slice_lds(r.nR, r.nU, r.maxLines) <= (size_t)kMaxLds;
+}
+
+bool slice_on(const Run &r) {
+  if (!slice_fits(r)) return false;
+  if (r.sliceMode >= 0) return r.sliceMode == 1;
+  if (r.lineMode >= 0 || r.kickMode >= 0) return false;
+  for (const char *e : {"VLS_NO_SLICE_STEP", "VLS_NO_REGISTER_LINES", "VLS_FUSED_KICK",
+                        "VLS_NO_FUSED_KICK", "VLS_KICK_SCRATCH", "VLS_KICK_RSOLVE",
+                        "VLS_NO_KICK_MOMENT", "VLS_MOMENT_3K", "VLS_SPLINE_STREAM", "VLS_TILE_R",
+                        "VLS_TILE_V"})
+    if (getenv(e)) return false;
+  return true;
+}
+
+void launch_slice_start(Run &r, hipStream_t s) {
+  SliceArgs a = slice_args(r);
+  a.P = r.P;
+  if (r.sp.no_linking) {  // the first half step
+    a.f = kicked(r);
+    launch_drift(r, a, s);
+    return;
+  }
+  hipLaunchKernelGGL(k_slice_moment, dim3(r.nJ), dim3(kT),
+                     ((size_t)r.nU + (size_t)(r.nU + 14) / 16 * r.nR) * sizeof(double), s, a);
+}
+
+void launch_slice_kick(Run &r, hipStream_t s, double *dKeep) {
+  KickArgs k{};
+  k.src = r.sp.no_linking ? kicked(r) : r.f;
+  k.dst = kicked(r);
+  k.P = r.P;
+  k.dKeep = dKeep;
+  k.gfac = r.gfac;
+  k.U_Val = r.U_Val;
+  k.dM = r.dM;
+  k.Mx = r.Mx;
+  k.acc = r.acc;
+  k.mTot = r.mTot;
+  k.head = r.nChains ? r.ch_head : nullptr;
+  k.len = r.ch_len;
+  k.nChains = r.nChains;
+  k.nVal = r.nVal;
+  k.cs = r.cs;
+  k.Ulo = r.Ulo;
+  k.Uhi = r.Uhi;
+  k.start_v = r.start_v;
+  k.hinv_v = r.hinv_v;
+  k.tv = r.tv;
+  k.nR = r.nR;
+  k.nU = r.nU;
+  k.nJ = r.nJ;
+  k.nS = r.nS;
+  k.W = kick_width(r);
+  k.nT = (r.nR + k.W - 1) / k.W;
+  k.mulW = magic(k.W);
+  k.mulR = magic(r.nR);
+  k.roll = r.sp.no_linking ? 2 : 1;
+  const bool wide = r.nJ * k.nT <= r.cus;
+  hipLaunchKernelGGL(wide ? k_kick_tile<512> : k_kick_tile<256>, dim3(r.nJ * k.nT),
+                     dim3(wide ? 512 : 256), kick_lds(r.nR, r.nU, r.nJ, k.W), s, k);
+}
+
+void launch_slice_drift(Run &r, hipStream_t s, bool last) {
+  SliceArgs a = slice_args(r);
+  // the kick has advanced the heads by the step's drifts: this is its last
+  a.src = kicked(r);
+  a.hOff = -1;
+  if (r.sp.no_linking && !last) {
+    launch_drift(r, a, s);  // and the first half of the next step
+    a.src = r.f;
+    a.f = kicked(r);
+    a.hOff = 0;
+  }
+  a.P = last ? nullptr : r.P;
+  a.cOut = last ? r.c : nullptr;
+  launch_drift(r, a, s);
+}
+
+}  // namespace vls
