@@ -42,6 +42,12 @@ def _run(cfg, label):
         assert np.array_equal(gpu.f(), orc.f()), label
     for a, b in zip(gpu.moments(), orc.last_moments()):
         assert np.array_equal(a, b), label
+    # the statistics' sums (their groups of 16 rows and radii) at the same edges;
+    # the entropy goes through the device's logarithm
+    sg, so = gpu.stats_total(), orc.stats_total()
+    for key in ("M", "E", "Ek", "Ep", "L1", "L2"):
+        assert sg[key] == so[key], (label, key)
+    assert abs(sg["S"] - so["S"]) <= 1e-14 * abs(so["S"])
 
 
 def test_slice_step_against_kernels_per_phase(monkeypatch):

@@ -16,6 +16,7 @@
 #include <mutex>
 #include <string>
 #include <tuple>
+#include <type_traits>
 
 #include "vls_device.hpp"
 #include "vls_div.hpp"
@@ -1652,148 +1653,257 @@ k_mark_chains(double2 *__restrict__ feet, const int64_t *__restrict__ point, int
 // the statistics.txt line, take the sum of the species' cell averages
 // (int21::f / entropy / L2Norm(0, nS)); the other integrands read species 0,
 // as the reference's default integrands do (src/slice21Iterator.hxx:90-94).
-__global__ void __launch_bounds__(kBlock)
+//
+// A block takes 64 columns of a slice.  The terms (a logarithm among them, about
+// 100 operations a point) are what costs, so the four waves form them for four
+// rows each of a group of 16 and leave them in LDS; then each wave adds up one
+// integrand (the last the mass too) over the group's rows in order.  It is bound
+// by the issue of the terms: 62 us at 201x201x200, 327 at 513x513x256, 10 at
+// 65x65x32.  A thread per column for the whole sum kept less than a wave per
+// SIMD in flight: 123, 425 and 42 us.  (The next group's rows loaded ahead
+// change nothing.)
+constexpr int kStatRows = 16;
+template <bool kSpecies>
+__global__ void __launch_bounds__(256)
 k_stats_partial(const double *__restrict__ f, const double *__restrict__ Ct1,
                 const double *__restrict__ dU, const double *__restrict__ dR,
                 const double *__restrict__ R_Val, const double *__restrict__ U_Val,
                 const double *__restrict__ J_Val, double *__restrict__ part, int nR, int nU,
                 int nJ, int nS, int64_t nVal) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  int j = blockIdx.y;
-  if (r >= nR) return;
-  double m = 0.0, ek = 0.0, s = 0.0, l1 = 0.0, l2 = 0.0, sAll = 0.0, l2All = 0.0;
-  if (r < nR - 1) {
-    const double ct = Ct1[j];
-    const double dr = dR[r];
-    const double rc = R_Val[r] + 0.5 * dr;
-    const double J = J_Val[j];
-    const double *p = f + (int64_t)j * nU * nR + r;
-    double a0 = p[0], a1 = p[1];
-    // the mass in the moment's tree order (groups of 16 rows, waves of 64),
-    // the other integrands serial in u
-    const int nW = (nU + 63) / 64;
-    for (int wv = 0; wv < nW; wv++) {
-      double G[4];
-      for (int q4 = 0; q4 < 4; q4++) {
-        double g = 0.0;
-        for (int t = 0; t < 16; t++) {
-          const int u = 64 * wv + 16 * q4 + t;
-          if (u >= nU - 1) break;
-          const double *q = p + (int64_t)(u + 1) * nR;
-          double b0 = q[0], b1 = q[1];
-          double v = (((a0 + a1) + b0) + b1) * 0.25;
-          double vm = v;  // the sum over the species
-          if (nS > 1) {
-            vm = 0.0 + v;
-            for (int k = 1; k < nS; k++) {
-              const double *pk = p + (int64_t)k * nVal + (int64_t)u * nR;
-              vm += (((pk[0] + pk[1]) + pk[nR]) + pk[nR + 1]) * 0.25;
-            }
-          }
-          double du = dU[u];
-          double w = (ct * du) * dr;
-          double uc = U_Val[u] + 0.5 * du;
-          g += w * vm;
-          ek += w * (0.5 * v * (uc * uc + J * J / (rc * rc)));
-          s += w * ((v <= 0) ? 0.0 : -v * log(v));
-          l1 += w * fabs(v);
-          l2 += w * (v * v);
-          if (nS > 1) {
-            sAll += w * ((vm <= 0) ? 0.0 : -vm * log(vm));
-            l2All += w * (vm * vm);
-          }
-          a0 = b0;
-          a1 = b1;
-        }
-        G[q4] = g;
-      }
-      const double Wm = ((G[0] + G[1]) + G[2]) + G[3];
-      m = wv == 0 ? Wm : m + Wm;
+  constexpr int kTerms = kSpecies ? 7 : 5;  // m, ek, s, l1, l2 (and all species' s, l2)
+  __shared__ double T[kTerms][kStatRows][64];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nX = (nR + 63) / 64;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int j = tile / nX, r = (tile - j * nX) * 64 + lane;
+  const bool term = r < nR - 1;
+  const int rc0 = min(r, nR - 2);  // columns past the last cell repeat it, not stored
+  const double ct = Ct1[j], dr = dR[rc0], J = J_Val[j];
+  const double rc = R_Val[rc0] + 0.5 * dr;
+  const double jr2 = J * J / (rc * rc);
+  const double *p = f + (int64_t)j * nU * nR + rc0;
+  double sum[2] = {0.0, 0.0};  // this wave's integrands: 1 + w, and 5 + w (w < 2, species)
+  double m = 0.0, G[4];
+  for (int u0 = 0; u0 < nU - 1; u0 += kStatRows) {
+    constexpr int kQ = kStatRows / 4;
+    double a0[kQ + 1], a1[kQ + 1];
+#pragma unroll
+    for (int q = 0; q <= kQ; q++) {
+      const double *pu = p + (int64_t)min(u0 + kQ * w + q, nU - 1) * nR;
+      a0[q] = pu[0];
+      a1[q] = pu[1];
     }
+#pragma unroll
+    for (int q = 0; q < kQ; q++) {
+      const int row = kQ * w + q, u = min(u0 + row, nU - 2);  // rows past the last: not added
+      const double v = (((a0[q] + a1[q]) + a0[q + 1]) + a1[q + 1]) * 0.25;
+      double vm = v;  // the sum over the species
+      if (kSpecies) {
+        vm = 0.0 + v;
+        for (int k = 1; k < nS; k++) {
+          const double *pk = p + (int64_t)k * nVal + (int64_t)u * nR;
+          vm += (((pk[0] + pk[1]) + pk[nR]) + pk[nR + 1]) * 0.25;
+        }
+      }
+      const double du = dU[u], wt = (ct * du) * dr, uc = U_Val[u] + 0.5 * du;
+      T[0][row][lane] = wt * vm;
+      T[1][row][lane] = wt * (0.5 * v * (uc * uc + jr2));
+      T[2][row][lane] = wt * ((v <= 0) ? 0.0 : -v * log(v));
+      T[3][row][lane] = wt * fabs(v);
+      T[4][row][lane] = wt * (v * v);
+      if (kSpecies) {
+        T[5][row][lane] = wt * ((vm <= 0) ? 0.0 : -vm * log(vm));
+        T[6][row][lane] = wt * (vm * vm);
+      }
+    }
+    __syncthreads();
+    // rows past the last one are left out, not added as 0
+    const int rows = min(kStatRows, nU - 1 - u0);
+    auto add = [&](const double (*t)[64], double s) {
+      double x[kStatRows];
+#pragma unroll
+      for (int q = 0; q < kStatRows; q++) x[q] = t[q][lane];
+#pragma unroll
+      for (int q = 0; q < kStatRows; q++)
+        if (q < rows) s += x[q];
+      return s;
+    };
+    sum[0] = add(T[1 + w], sum[0]);
+    if (kSpecies && w < 2) sum[1] = add(T[5 + w], sum[1]);
+    if (w == 3) {
+      // the mass: groups of 16 rows, ((G0 + G1) + G2) + G3 per block of 64, the
+      // blocks left to right
+      const int g = (u0 / kStatRows) & 3;
+      const double x = add(T[0], 0.0);
+      if (g == 0) G[0] = x, G[1] = 0.0, G[2] = 0.0, G[3] = 0.0;
+      if (g == 1) G[1] = x;
+      if (g == 2) G[2] = x;
+      if (g == 3) G[3] = x;
+      if (g == 3 || u0 + kStatRows >= nU - 1) {
+        const double W = ((G[0] + G[1]) + G[2]) + G[3];
+        m = u0 < 64 ? W : m + W;
+      }
+    }
+    __syncthreads();
   }
+  // blocks of 64 rows past the last term
+  if (w == 3)
+    for (int b = (nU - 2) / 64 + 1; b < (nU + 63) / 64; b++) m = m + 0.0;
+  if (r >= nR) return;
   const int64_t o = (int64_t)j * nR + r, n = (int64_t)nJ * nR;
-  part[o] = m;
-  part[n + o] = ek;
-  part[2 * n + o] = s;
-  part[3 * n + o] = l1;
-  part[4 * n + o] = l2;
-  part[5 * n + o] = sAll;
-  part[6 * n + o] = l2All;
+  part[(1 + w) * n + o] = term ? sum[0] : 0.0;
+  if (w == 3) part[o] = term ? m : 0.0;
+  if (w < 2) part[(5 + w) * n + o] = kSpecies && term ? sum[1] : 0.0;
 }
 
-// Serial sums over j (moment) and over r (integrands), then over j; the
-// potential energy of vlasovSolver21::potentialEnergy
+// The sums of the partials: q[k][j], serial over r, of the integrands k, and
+// the radial mass dM[r] in the order of the moment scan (chunks of kJC slices).
+// One block did all of them with a thread per sum, each waiting for its loads
+// one after another: with the line below 452 us at 201x201x200, 1172 at
+// 513x513x256, 46 at 65x65x32.  Here the first nQ blocks take 64 sums each,
+// whose rows come through LDS 16 radii at a time with the next 16 in flight,
+// and the others 64 radii each, a wave per chunk: 24, 57 and 10 us.
+constexpr int kSumC = 16;
+__global__ void __launch_bounds__(256)
+k_stats_sums(const double *__restrict__ part, double *__restrict__ dM, double *__restrict__ q,
+             int nR, int nJ, int nQ) {
+  const int64_t n = (int64_t)nJ * nR;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  __shared__ double L[64][kSumC + 1];
+  if ((int)blockIdx.x < nQ) {
+    const int s0 = blockIdx.x * 64, nSum = 6 * nJ;
+    // thread t loads rows t / 16 + 16 i of column t % 16
+    const int cs = t % kSumC, rs = t / kSumC;
+    double v[4];
+    auto load = [&](int c0) {
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        v[i] = part[n + (int64_t)min(s0 + rs + 16 * i, nSum - 1) * nR + min(c0 + cs, nR - 1)];
+    };
+    double s = 0.0;
+    load(0);
+    for (int c0 = 0; c0 < nR - 1; c0 += kSumC) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) L[rs + 16 * i][cs] = v[i];
+      __syncthreads();
+      if (c0 + kSumC < nR - 1) load(c0 + kSumC);
+      if (w == 0) {
+        double x[kSumC];
+#pragma unroll
+        for (int k = 0; k < kSumC; k++) x[k] = L[lane][k];
+#pragma unroll
+        for (int k = 0; k < kSumC; k++)
+          if (c0 + k < nR - 1) s += x[k];
+      }
+      __syncthreads();
+    }
+    if (w == 0 && s0 + lane < nSum) q[s0 + lane] = s;
+    return;
+  }
+  // the chunks' sums, up to 64 chunks at a time, then their serial sum
+  const int r = (blockIdx.x - nQ) * 64 + lane, rc = min(r, nR - 1);
+  const int nC = (nJ + kJC - 1) / kJC;
+  double *S = &L[0][0];  // [16][64]
+  double s = 0.0;
+  for (int cb = 0; cb < nC; cb += 16) {
+    for (int c = cb + w; c < min(nC, cb + 16); c += 4) {
+      double v[kJC];
+#pragma unroll
+      for (int k = 0; k < kJC; k++) v[k] = part[(int64_t)min(c * kJC + k, nJ - 1) * nR + rc];
+      double x = 0.0;
+#pragma unroll
+      for (int k = 0; k < kJC; k++)
+        if (c * kJC + k < nJ) x += v[k];
+      S[(c - cb) * 64 + lane] = x;
+    }
+    __syncthreads();
+    if (w == 0)
+      for (int c = cb; c < min(nC, cb + 16); c++) s += S[(c - cb) * 64 + lane];
+    __syncthreads();
+  }
+  if (w == 0 && r < nR) dM[r] = s;
+}
+
+// The sums over j and the potential energy of vlasovSolver21::potentialEnergy
 // (src/vlasovSolver21.hxx:627-642, with the gathered array shifted by one,
 // src/quadrature21.hxx:36).  out = {M, E, Ek, Ep, S, L1, L2} (the species
 // files' line), then the statistics.txt line: with nS species the species
 // loop of vlasovSolver21::statistics (:656-688) adds that line nS times, and
 // S and L2 are those of the summed species (:690-699); with one species the
-// same line again.
-__global__ void __launch_bounds__(kBlock)
-k_stats_final(const double *__restrict__ part, const double *__restrict__ R_Val, double G,
-              double *__restrict__ dM, double *__restrict__ q, double *__restrict__ out, int nR,
-              int nJ, int nS) {
-  const int64_t n = (int64_t)nJ * nR;
-  // the radial mass in the order of the moment scan: chunks of kJC slices
-  for (int r = threadIdx.x; r < nR; r += blockDim.x) {
-    double s = 0.0;
-    for (int j0 = 0; j0 < nJ; j0 += kJC) {
-      double S = 0.0;
-      for (int j = j0; j < nJ && j < j0 + kJC; j++) S += part[(int64_t)j * nR + r];
-      s += S;
+// same line again.  The serial sums run on values that the block has brought
+// into LDS (x: nR doubles, and 6 nJ where staged), and the shells' terms of the potential
+// energy, a division each, are formed by all threads between its two chains.
+__global__ void __launch_bounds__(256)
+k_stats_line(const double *__restrict__ dM, const double *__restrict__ q,
+             const double *__restrict__ R_Val, double G, double *__restrict__ out, int nR, int nJ,
+             int nS, int staged) {
+  extern __shared__ double x[];
+  __shared__ double tot[6], mass, pot;
+  const int t = threadIdx.x;
+  double *xq = x + nR;
+  for (int r = t; r < nR; r += 256) x[r] = dM[r];
+  if (staged)
+    for (int i = t; i < 6 * nJ; i += 256) xq[i] = q[i];
+  __syncthreads();
+  // sums of n entries in order, 16 of them read at a time; pre: the prefix
+  // before each entry takes its place
+  auto chain = [&](auto *v, int n, double s, auto pre) {
+    constexpr int kS = 16;
+    for (int i0 = 0; i0 < n; i0 += kS) {
+      double y[kS];
+#pragma unroll
+      for (int k = 0; k < kS; k++) y[k] = v[min(i0 + k, n - 1)];
+#pragma unroll
+      for (int k = 0; k < kS; k++)
+        if (i0 + k < n) {
+          if constexpr (decltype(pre)::value) v[i0 + k] = s;
+          s += y[k];
+        }
     }
-    dM[r] = s;
-  }
-  for (int t = threadIdx.x; t < 6 * nJ; t += blockDim.x) {
-    int k = t / nJ, j = t % nJ;
-    const double *p = part + (int64_t)(k + 1) * n + (int64_t)j * nR;
-    double s = 0.0;
-    for (int r = 0; r < nR - 1; r++) s += p[r];
-    q[t] = s;
+    return s;
+  };
+  if (t == 0) mass = chain(x, nR, 0.0 + 0.0, std::true_type{});
+  if (t >= 64 && t < 70) {
+    const int k = t - 64;
+    tot[k] = staged ? chain(xq + k * nJ, nJ, 0.0, std::false_type{})
+                    : chain(q + k * nJ, nJ, 0.0, std::false_type{});
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    // shell k (R[k]..R[k+1]) meets M(<R[k]) at its midpoint: the gathered
-    // array of potentialEnergy is shifted by one (addSpare=1)
-    double M = 0.0 + 0.0, Ep = 0.0;
-    for (int i = 1; i < nR; i++) {
-      double rr = 0.5 * (R_Val[i - 1] + R_Val[i]);
-      Ep -= (dM[i - 1] * G * M) / rr;
-      M += dM[i - 1];
+  // shell k (R[k]..R[k+1]) meets M(<R[k]) at its midpoint: the gathered
+  // array of potentialEnergy is shifted by one (addSpare=1)
+  for (int i = t; i < nR - 1; i += 256) {
+    const double rr = 0.5 * (R_Val[i] + R_Val[i + 1]);
+    x[i] = -((dM[i] * G * x[i]) / rr);
+  }
+  __syncthreads();
+  if (t != 0) return;
+  pot = chain(x, nR - 1, 0.0, std::false_type{});
+  const double M = mass, Ep = pot;
+  out[0] = M;
+  out[1] = tot[0] + Ep;
+  out[2] = tot[0];
+  out[3] = Ep;
+  out[4] = tot[1];
+  out[5] = tot[2];
+  out[6] = tot[3];
+  if (nS == 1) {
+    for (int k = 0; k < 7; k++) out[7 + k] = out[k];
+  } else {
+    double Ep_tot = 0, M_tot = 0, Ek_tot = 0, E_tot = 0, L1_tot = 0;
+    for (int k = 0; k < nS; k++) {
+      Ep_tot += Ep;
+      M_tot += M;
+      Ek_tot += tot[0];
+      E_tot += tot[0] + Ep;
+      L1_tot += tot[2];
     }
-    M += dM[nR - 1];
-    double tot[6];
-    for (int k = 0; k < 6; k++) {
-      double s = 0.0;
-      for (int j = 0; j < nJ; j++) s += q[k * nJ + j];
-      tot[k] = s;
-    }
-    out[0] = M;
-    out[1] = tot[0] + Ep;
-    out[2] = tot[0];
-    out[3] = Ep;
-    out[4] = tot[1];
-    out[5] = tot[2];
-    out[6] = tot[3];
-    if (nS == 1) {
-      for (int k = 0; k < 7; k++) out[7 + k] = out[k];
-    } else {
-      double Ep_tot = 0, M_tot = 0, Ek_tot = 0, E_tot = 0, L1_tot = 0;
-      for (int k = 0; k < nS; k++) {
-        Ep_tot += out[3];
-        M_tot += out[0];
-        Ek_tot += out[2];
-        E_tot += out[1];
-        L1_tot += out[5];
-      }
-      out[7] = M_tot;
-      out[8] = E_tot;
-      out[9] = Ek_tot;
-      out[10] = Ep_tot;
-      out[11] = tot[4];
-      out[12] = L1_tot;
-      out[13] = tot[5];
-    }
+    out[7] = M_tot;
+    out[8] = E_tot;
+    out[9] = Ek_tot;
+    out[10] = Ep_tot;
+    out[11] = tot[4];
+    out[12] = L1_tot;
+    out[13] = tot[5];
   }
 }
 
@@ -2801,11 +2911,17 @@ void launch_density_potential_from(Run &r, const double *dM, const double *Mx, d
 }
 
 void launch_stats(Run &r, hipStream_t s) {
-  dim3 g(blocks_for(r.nR), r.nJ);
-  hipLaunchKernelGGL(k_stats_partial, g, dim3(kBlock), 0, s, r.f, r.Ct1, r.dU, r.dR, r.R_Val,
-                     r.U_Val, r.J_Val, r.st_part, r.nR, r.nU, r.nJ, r.nS, r.nVal);
-  hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(kBlock), 0, s, r.st_part, r.R_Val, r.sp.G,
-                     r.st_q + 6 * (int64_t)r.nJ, r.st_q, r.st_out, r.nR, r.nJ, r.nS);
+  double *dM = r.st_q + 6 * (int64_t)r.nJ;
+  hipLaunchKernelGGL(r.nS > 1 ? k_stats_partial<true> : k_stats_partial<false>,
+                     dim3((r.nR + 63) / 64 * r.nJ), dim3(256), 0, s, r.f, r.Ct1, r.dU, r.dR,
+                     r.R_Val, r.U_Val, r.J_Val, r.st_part, r.nR, r.nU, r.nJ, r.nS, r.nVal);
+  const int nQ = (6 * r.nJ + 63) / 64;
+  hipLaunchKernelGGL(k_stats_sums, dim3(nQ + (r.nR + 63) / 64), dim3(256), 0, s, r.st_part, dM,
+                     r.st_q, r.nR, r.nJ, nQ);
+  const bool staged = 6 * (size_t)r.nJ * sizeof(double) <= 32768;
+  hipLaunchKernelGGL(k_stats_line, dim3(1), dim3(256),
+                     (r.nR + (staged ? 6 * (size_t)r.nJ : 0)) * sizeof(double), s, dM, r.st_q,
+                     r.R_Val, r.sp.G, r.st_out, r.nR, r.nJ, r.nS, staged ? 1 : 0);
 }
 
 }  // namespace vls
