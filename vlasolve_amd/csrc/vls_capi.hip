@@ -588,8 +588,8 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
         ax.rl = dev + 2 * ax.M;
         VLS_HIP_CHECK(hipStreamSynchronize(s));  // u, rd, rl go out of scope
       }
+      vls::configure_slice(maxLds);
       if (pivots && vls::slice_shape(r, maxLds)) {
-        vls::configure_slice(maxLds);
         r.sliceG = dalloc<double>(r, vls::slice_group_doubles(r));
         r.sliceCnt = dalloc<unsigned>(r, r.nJ);
         VLS_HIP_CHECK(hipMemsetAsync(r.sliceCnt, 0, r.nJ * sizeof(unsigned), s));
@@ -1037,10 +1037,10 @@ int vls_density_potential_noalloc(vls_ctx *ctx, int run, const double *f_dev, do
     double *rho = Mx + r.nR, *phi = rho + r.nR, *mTot = phi + r.nR;
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ctx->c.stream;
     const vls::MomentBufs b{f_dev, P, dM, M_dev ? M_dev : Mx, acc, mTot, nullptr};
-    vls::launch_moment_into(r, b, s);
     if (rho_dev || phi_dev)
-      vls::launch_density_potential_from(r, dM, b.Mx, rho_dev ? rho_dev : rho,
-                                         phi_dev ? phi_dev : phi, s);
+      vls::launch_profile_into(r, b, rho_dev ? rho_dev : rho, phi_dev ? phi_dev : phi, s);
+    else
+      vls::launch_moment_into(r, b, s);
     VLS_HIP_CHECK(hipGetLastError());
   });
 }

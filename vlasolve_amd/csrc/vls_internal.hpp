@@ -222,6 +222,9 @@ size_t slice_group_doubles(const Run &r);
 void configure_slice(int maxLdsPerBlock);
 bool slice_fits(const Run &r);    // the run's buffers are there and its delay lines fit too
 bool slice_on(const Run &r);
+// the moment partials P [nJ][nR] of f (the run's shape and species), a block
+// per slice; false if a slice's group sums don't fit in LDS
+bool launch_slice_partials(Run &r, const double *f, double *P, hipStream_t s);
 void launch_slice_start(Run &r, hipStream_t s);
 void launch_slice_kick(Run &r, hipStream_t s, double *dKeep);
 void launch_slice_drift(Run &r, hipStream_t s, bool last);
@@ -229,6 +232,8 @@ void mark_chains(Run &r, hipStream_t s);  // attach the delay lines to their poi
 void launch_stats(Run &r, hipStream_t s);
 // rho[nR], phi[nR] (device) from the moment and enclosed mass of the last launch_moment
 void launch_density_potential(Run &r, double *rho, double *phi, hipStream_t s);
+// launch_moment_into and the density and potential from it (rho, phi: [nR])
+void launch_profile_into(Run &r, const MomentBufs &b, double *rho, double *phi, hipStream_t s);
 void launch_density_potential_from(Run &r, const double *dM, const double *Mx, double *rho,
                                    double *phi, hipStream_t s);
 

@@ -1908,25 +1908,88 @@ k_stats_line(const double *__restrict__ dM, const double *__restrict__ q,
 }
 
 // Shell density and potential from the moment (the definitions of
-// vls_density_potential): rho[k] = dM[k] / (vol (R[k+1]^3 - R[k]^3)) with
-// vol = 4 pi / 3, and phi[i] = -G (Mx[i] / R[i] + S[i]), S the suffix sum of
-// dM[k] / rbar[k] over the shells k >= i, rbar[k] = (R[k] + R[k+1]) / 2,
-// added from the outermost shell inwards by one thread.
+// vls_density_potential), by one block: rho[k] = dM[k] / (vol (R[k+1]^3 -
+// R[k]^3)) with vol = 4 pi / 3, and phi[i] = -G (Mx[i] / R[i] + S[i]), S the
+// suffix sum of dM[k] / rbar[k] over the shells k >= i, rbar[k] = (R[k] +
+// R[k+1]) / 2, added from the outermost shell inwards by one thread on the
+// quotients that the block has left in LDS (x: nR doubles).
+__device__ __forceinline__ void density_potential(const double *__restrict__ R, const double *dM,
+                                                  const double *Mx, double G, double vol,
+                                                  double *__restrict__ rho,
+                                                  double *__restrict__ phi, int nR, double *x) {
+  const int t = threadIdx.x, T = blockDim.x;
+  for (int k = t; k < nR; k += T) {
+    rho[k] = k < nR - 1
+                 ? dM[k] / (vol * (R[k + 1] * R[k + 1] * R[k + 1] - R[k] * R[k] * R[k]))
+                 : 0.0;
+    x[k] = k < nR - 1 ? dM[k] / (0.5 * (R[k] + R[k + 1])) : 0.0;
+  }
+  __syncthreads();
+  if (t == 0) {
+    constexpr int kS = 16;
+    double S = 0.0;
+    for (int i0 = nR - 2; i0 >= 0; i0 -= kS) {
+      double v[kS];
+#pragma unroll
+      for (int k = 0; k < kS; k++) v[k] = x[max(i0 - k, 0)];
+#pragma unroll
+      for (int k = 0; k < kS; k++)
+        if (i0 - k >= 0) {
+          S = v[k] + S;
+          x[i0 - k] = S;
+        }
+    }
+  }
+  __syncthreads();
+  for (int i = t; i < nR; i += T) phi[i] = -(G * (Mx[i] / R[i] + x[i]));
+}
+
 __global__ void __launch_bounds__(kBlock)
 k_density_potential(const double *__restrict__ R, const double *__restrict__ dM,
                     const double *__restrict__ Mx, double G, double vol, double *__restrict__ rho,
                     double *__restrict__ phi, int nR) {
-  for (int k = threadIdx.x; k < nR; k += blockDim.x)
-    rho[k] = k < nR - 1
-                 ? dM[k] / (vol * (R[k + 1] * R[k + 1] * R[k + 1] - R[k] * R[k] * R[k]))
-                 : 0.0;
-  if (threadIdx.x == 0) {
-    double S = 0.0;
-    for (int i = nR - 1; i >= 0; i--) {
-      if (i < nR - 1) S = dM[i] / (0.5 * (R[i] + R[i + 1])) + S;
-      phi[i] = -(G * (Mx[i] / R[i] + S));
-    }
+  extern __shared__ double x[];
+  density_potential(R, dM, Mx, G, vol, rho, phi, nR, x);
+}
+
+// k_moment_chunks and k_moment_scan in one launch of one block, for grids
+// whose chunk sums [nC][nR] fit in its LDS with the scan, and where rho is
+// given the density and potential too: the calls that end in these few radii
+// are launches and round trips and nothing else.  At 65x65x32 the profile call
+// took 26.6 us in four launches (the last, a thread dividing shell by shell,
+// 16), now 11 in two.
+__global__ void __launch_bounds__(kScanThreads)
+k_moment_reduce(const double *__restrict__ P, const double *__restrict__ gfac,
+                double *__restrict__ dM, double *__restrict__ Mx, double *__restrict__ acc,
+                double *__restrict__ mTot, int nR, int nJ, const double *__restrict__ R, double G,
+                double vol, double *__restrict__ rho, double *__restrict__ phi) {
+  extern __shared__ double sdm[];  // [nR] the scan, [nR] the factors, [nC][nR] chunk sums
+  double *sgf = sdm + nR, *S = sgf + nR;
+  const int t = threadIdx.x, nC = (nJ + kJC - 1) / kJC;
+  for (int i = t; i < nC * nR; i += kScanThreads) {
+    const int c = i / nR, r = i - c * nR, jb = c * kJC;
+    double v[kJC];
+    // clamped rows are loaded, not added
+#pragma unroll
+    for (int k = 0; k < kJC; k++) v[k] = P[(size_t)min(jb + k, nJ - 1) * nR + r];
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < kJC; k++)
+      if (jb + k < nJ) s += v[k];
+    S[i] = s;
   }
+  for (int r = t; r < nR; r += kScanThreads) sgf[r] = gfac[r];
+  __syncthreads();
+  for (int r = t; r < nR; r += kScanThreads) {
+    double a = 0.0;
+    for (int c = 0; c < nC; c++) a += S[c * nR + r];
+    dM[r] = a;
+    sdm[r] = a;
+  }
+  scan_prefix_out(sdm, sgf, Mx, acc, mTot, nR);
+  if (!rho) return;
+  __syncthreads();
+  density_potential(R, dM, Mx, G, vol, rho, phi, nR, S);
 }
 
 inline unsigned blocks_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -1959,15 +2022,11 @@ void launch_moment(Run &r, hipStream_t s) {
   launch_moment_into(r, MomentBufs{r.f, r.P, r.dM, r.Mx, r.acc, r.mTot, r.mCnt}, s);
 }
 
-void launch_moment_into(Run &r, const MomentBufs &b, hipStream_t s) {
+// The partials of b.f into b.P: a block per slice, or where its group sums
+// don't fit in LDS a thread or lane per column.
+static void launch_partials(Run &r, const MomentBufs &b, hipStream_t s) {
+  if (!getenv("VLS_MOMENT_3K") && launch_slice_partials(r, b.f, b.P, s)) return;
   dim3 g(blocks_for(r.nR), r.nJ);
-  if (r.nS == 1 && b.cnt && !getenv("VLS_MOMENT_3K")) {
-    const size_t lds = std::max<size_t>(64 * ((r.nU + 63) / 64), 2 * r.nR) * sizeof(double);
-    const MomentArgs ma{r.Ct1, r.dU, r.dR, r.gfac, b.P, b.dM, b.Mx, b.acc, b.mTot, b.cnt};
-    hipLaunchKernelGGL(k_moment_fused, dim3((r.nR + 62) / 63 * r.nJ), dim3(256), lds, s, b.f,
-                       r.nR, r.nU, r.nJ, ma);
-    return;
-  }
   if (r.nS > 1)
     hipLaunchKernelGGL(k_moment_partial_sp, g, dim3(kBlock), 0, s, b.f, r.Ct1, r.dU, r.dR, b.P,
                        r.nR, r.nU, r.nJ, r.nS, r.nVal);
@@ -1975,6 +2034,23 @@ void launch_moment_into(Run &r, const MomentBufs &b, hipStream_t s) {
     hipLaunchKernelGGL(k_moment_cols, dim3((r.nR + 62) / 63 * r.nJ), dim3(256),
                        64 * ((r.nU + 63) / 64) * sizeof(double), s, b.f, r.Ct1, r.dU,
                        r.dR, b.P, r.nR, r.nU);
+}
+
+// k_moment_reduce's LDS
+static size_t reduce_lds(const Run &r) {
+  return (2 + (size_t)(r.nJ + kJC - 1) / kJC) * r.nR * sizeof(double);
+}
+constexpr size_t kReduceLds = 65536;
+
+void launch_moment_into(Run &r, const MomentBufs &b, hipStream_t s) {
+  if (r.nS == 1 && b.cnt && !getenv("VLS_MOMENT_3K")) {
+    const size_t lds = std::max<size_t>(64 * ((r.nU + 63) / 64), 2 * r.nR) * sizeof(double);
+    const MomentArgs ma{r.Ct1, r.dU, r.dR, r.gfac, b.P, b.dM, b.Mx, b.acc, b.mTot, b.cnt};
+    hipLaunchKernelGGL(k_moment_fused, dim3((r.nR + 62) / 63 * r.nJ), dim3(256), lds, s, b.f,
+                       r.nR, r.nU, r.nJ, ma);
+    return;
+  }
+  launch_partials(r, b, s);
   launch_moment_scan_into(r, b, s);
 }
 
@@ -1982,7 +2058,27 @@ void launch_moment_scan(Run &r, hipStream_t s) {
   launch_moment_scan_into(r, MomentBufs{r.f, r.P, r.dM, r.Mx, r.acc, r.mTot, nullptr}, s);
 }
 
+static void launch_reduce(Run &r, const MomentBufs &b, double *rho, double *phi, hipStream_t s) {
+  hipLaunchKernelGGL(k_moment_reduce, dim3(1), dim3(kScanThreads), reduce_lds(r), s, b.P, r.gfac,
+                     b.dM, b.Mx, b.acc, b.mTot, r.nR, r.nJ, r.R_Val, r.sp.G, (4.0 * M_PI) / 3.0,
+                     rho, phi);
+}
+
+void launch_profile_into(Run &r, const MomentBufs &b, double *rho, double *phi, hipStream_t s) {
+  if (reduce_lds(r) > kReduceLds) {
+    launch_moment_into(r, b, s);
+    launch_density_potential_from(r, b.dM, b.Mx, rho, phi, s);
+    return;
+  }
+  launch_partials(r, b, s);
+  launch_reduce(r, b, rho, phi, s);
+}
+
 void launch_moment_scan_into(Run &r, const MomentBufs &b, hipStream_t s) {
+  if (reduce_lds(r) <= kReduceLds && !getenv("VLS_MOMENT_3K")) {
+    launch_reduce(r, b, nullptr, nullptr, s);
+    return;
+  }
   const int nC = (r.nJ + kJC - 1) / kJC;
   hipLaunchKernelGGL(k_moment_chunks, dim3(nC, (r.nR + kChunkThreads - 1) / kChunkThreads),
                      dim3(kChunkThreads), 0, s, b.P, r.nR, r.nJ);
@@ -2906,7 +3002,7 @@ void launch_density_potential(Run &r, double *rho, double *phi, hipStream_t s) {
 
 void launch_density_potential_from(Run &r, const double *dM, const double *Mx, double *rho,
                                    double *phi, hipStream_t s) {
-  hipLaunchKernelGGL(k_density_potential, dim3(1), dim3(kBlock), 0, s, r.R_Val, dM, Mx, r.sp.G,
+  hipLaunchKernelGGL(k_density_potential, dim3(1), dim3(kBlock), r.nR * sizeof(double), s, r.R_Val, dM, Mx, r.sp.G,
                      (4.0 * M_PI) / 3.0, rho, phi, r.nR);
 }
 

@@ -883,6 +883,19 @@ bool slice_on(const Run &r) {
   return true;
 }
 
+size_t partials_lds(const Run &r) {
+  return ((size_t)r.nU + (size_t)(r.nU + 14) / 16 * r.nR) * sizeof(double);
+}
+
+bool launch_slice_partials(Run &r, const double *f, double *P, hipStream_t s) {
+  if (partials_lds(r) > (size_t)kMaxLds) return false;
+  SliceArgs a = slice_args(r);
+  a.f = const_cast<double *>(f);  // read only
+  a.P = P;
+  hipLaunchKernelGGL(k_slice_moment, dim3(r.nJ), dim3(kT), partials_lds(r), s, a);
+  return true;
+}
+
 void launch_slice_start(Run &r, hipStream_t s) {
   SliceArgs a = slice_args(r);
   a.P = r.P;
@@ -891,8 +904,7 @@ void launch_slice_start(Run &r, hipStream_t s) {
     launch_drift(r, a, s);
     return;
   }
-  hipLaunchKernelGGL(k_slice_moment, dim3(r.nJ), dim3(kT),
-                     ((size_t)r.nU + (size_t)(r.nU + 14) / 16 * r.nR) * sizeof(double), s, a);
+  launch_slice_partials(r, r.f, r.P, s);
 }
 
 void launch_slice_kick(Run &r, hipStream_t s, double *dKeep) {
