@@ -279,7 +279,10 @@ void step_once(vls::Run &r, hipStream_t s, vls::Timing *t) {
     vls::launch_drift(r, s);
     vls::time_mark(t, s, "drift");
   }
-  if (vls::kick_in_rsolve(r)) {
+  if (vls::kick_streams(r)) {
+    vls::launch_kick_stream(r, s, t, nullptr);
+    vls::launch_spline_from_kick(r, s, t);
+  } else if (vls::kick_in_rsolve(r)) {
     vls::launch_kick_rsolve(r, s, t);
     vls::launch_spline_v_timed(r, s, t);
   } else {
@@ -334,10 +337,17 @@ void step_keep(vls::Run &r, hipStream_t s, double *cK, double *accOut, bool adva
     if (advance) vls::launch_slice_drift(r, s, last);
     return;
   }
-  vls::launch_spline_kick(r, s, nullptr, true, cK);
+  const bool streams = vls::kick_streams(r);
+  if (streams)
+    vls::launch_kick_stream(r, s, nullptr, cK);
+  else
+    vls::launch_spline_kick(r, s, nullptr, true, cK);
   r.acc = swap.own;
   if (!advance) return;
-  vls::launch_spline(r, r.f, s, nullptr);
+  if (streams)
+    vls::launch_spline_from_kick(r, s, nullptr);
+  else
+    vls::launch_spline(r, r.f, s, nullptr);
   vls::launch_drift(r, s);
 }
 
@@ -661,9 +671,10 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
       r.Uhi = G.U_Val[r.nU - 1];
       r.cus = (int)(256 * (int64_t)r.nJ / slices);
       vls::configure_tiles(r, maxLds);
-      // the kick folded into the r-solve leaves the solved rows (c's layout) in
-      // f's buffer between the kick and the drift
-      r.fRows = vls::kick_rsolve_shape(r);
+      // the kick folded into the r-solve and the streaming kick leave the solved
+      // rows (c's layout) in f's buffer between the kick and the drift
+      const bool streams = vls::kick_stream_shape(r);
+      r.fRows = streams || vls::kick_rsolve_shape(r);
       r.f = dalloc<double>(r, r.fRows ? std::max<size_t>(r.nVal, (size_t)r.nJ * r.cs)
                                       : (size_t)(r.nVal * r.nS));
       // A foot on the last knot (integer part dim-1, fraction 0) makes the
@@ -674,6 +685,7 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
       VLS_HIP_CHECK(hipMemsetAsync(r.c, 0, ((size_t)r.nJ * r.cs + kCoefPad(r)) * sizeof(double), s));
       if (size_t n = vls::kick_scratch_doubles(r)) r.gsc = dalloc<double>(r, n);
       r.kickScratch = getenv("VLS_KICK_SCRATCH") != nullptr;
+      if (streams) r.kept = dalloc<double>(r, vls::kept_doubles(r));
       r.feet = dalloc<double>(r, 2 * r.nVal);
       r.P = dalloc<double>(r, (size_t)r.nJ * r.nR);
       r.dM = dalloc<double>(r, r.nR);
@@ -721,10 +733,12 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
       }
       vls::configure_slice(maxLds);
       if (pivots && vls::slice_shape(r, maxLds)) {
-        r.sliceG = dalloc<double>(r, vls::slice_group_doubles(r));
-        r.sliceCnt = dalloc<unsigned>(r, r.nJ);
+        // one allocation: the group sums, the counters and the kicked f
+        const size_t nG = vls::slice_group_doubles(r);
+        r.sliceG = dalloc<double>(r, nG + r.nJ + (vls::slice_shared(r) ? r.nVal : 0));
+        r.sliceCnt = (unsigned *)(r.sliceG + nG);
         VLS_HIP_CHECK(hipMemsetAsync(r.sliceCnt, 0, r.nJ * sizeof(unsigned), s));
-        if (vls::slice_shared(r)) r.sliceF = dalloc<double>(r, r.nVal);
+        if (vls::slice_shared(r)) r.sliceF = r.sliceG + nG + r.nJ;
       }
     }
   });
@@ -860,7 +874,6 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
     dfree(r, r.ch_xu);
     dfree(r, r.ch_out);
     dfree(r, r.ch_vals);
-    dfree(r, r.ch_order);
     dfree(r, r.ch_start);
     r.adj.recorded = false;
     r.adj.tilesValid = false;  // the transposed foot table lists the back cells
@@ -893,11 +906,11 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
     for (int j = 0; j < r.nJ; j++) start[j + 1] += start[j];
     std::vector<int32_t> at(start.begin(), start.end() - 1);
     for (int64_t k = 0; k < nChains; k++) order[at[point[k] / nSlice]++] = (int32_t)k;
-    r.ch_order = dalloc<int32_t>(r, nChains);
-    r.ch_start = dalloc<int32_t>(r, r.nJ + 1);
-    h2d(r.ch_order, order.data(), nChains, s);
-    h2d(r.ch_start, start.data(), r.nJ + 1, s);
-    VLS_HIP_CHECK(hipStreamSynchronize(s));  // start, order go out of scope
+    r.ch_start = dalloc<int32_t>(r, r.nJ + 1 + nChains);
+    r.ch_order = r.ch_start + r.nJ + 1;
+    start.insert(start.end(), order.begin(), order.end());
+    h2d(r.ch_start, start.data(), start.size(), s);
+    VLS_HIP_CHECK(hipStreamSynchronize(s));  // start goes out of scope
     if (r.nS > 1) {
       std::vector<double> planes = to_planes(vals, cells, r.nS);
       h2d(r.ch_vals, planes.data(), planes.size(), s);

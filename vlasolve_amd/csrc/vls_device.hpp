@@ -11,6 +11,8 @@ namespace vls {
 // Slices per chunk of the moment's sum over j, and head rows of the pivot
 // tables (past them the pivots are at their fixed point).
 constexpr int kJC = 20, kHead = 16;
+// Rows of a segment of the streaming line solves (vls_stream.hip).
+constexpr int kSegRows = 16;
 
 __device__ __forceinline__ double BV2(double x) { return x * x * x; }
 __device__ __forceinline__ double BV1(double x) {

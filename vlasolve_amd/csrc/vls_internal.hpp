@@ -66,9 +66,9 @@ struct Run {
   bool streamR = false, streamV = false;  // streaming solvers for long lines
   // schedule choices (vls_autotune): -1 from the shape and the environment;
   // lineMode 0 / 1: LDS-tiled or streaming solvers / register lines (shapes
-  // that have them); kickMode 0 / 1 / 2 / 3: two-kernel / fused kick / the
+  // that have them); kickMode 0 / 1 / 2 / 3 / 4: two-kernel / fused kick / the
   // moment fused into the kick's column splines / that, and the kick's
-  // evaluation folded into the drift's r-solve
+  // evaluation folded into the drift's r-solve / streaming
   int lineMode = -1, kickMode = -1;
   // a step in two launches (vls_slice.hip), for the shapes that have sliceG: -1
   // unless the environment forces one of the other schedules, 0 / 1 tuned
@@ -79,9 +79,10 @@ struct Run {
   // state
   double *f = nullptr;      // [nS][nJ][nU][nR]
   double *c = nullptr;      // [nJ][nU+2][nR+2] spline coefficients
+  double *kept = nullptr;   // the streaming kick's kept elimination values (vls_stream.hip)
   double *gsc = nullptr;    // fused kick: per-wave scratch for wide kicks
-  bool fRows = false;       // f's buffer holds nJ*cs doubles: the kick folded into the r-solve
-                            // leaves its rows there (f is rewritten by the drift)
+  bool fRows = false;       // f's buffer holds nJ*cs doubles: the r-solve after an out-of-place
+                            // kick leaves its rows there (f is rewritten by the drift)
   bool kickScratch = false; // fused kick: always take the scratch path
   // static feet, interleaved (xr, xu) per point: one 16-byte load each
   // (xr <= -1 marks points outside the grid or on delay lines)
@@ -187,6 +188,20 @@ size_t moment_counters(const Run &r);
 void launch_moment_into(Run &r, const MomentBufs &b, hipStream_t s);
 void launch_moment_scan_into(Run &r, const MomentBufs &b, hipStream_t s);
 void launch_spline(Run &r, const double *src, hipStream_t s, Timing *t);
+// the streaming solves (vls_stream.hip): rows of src (f's layout) to the
+// padded rows dst, the columns of src (c's layout) to c (dst == src allowed)
+void launch_stream_r(const Run &r, const double *src, double *dst, hipStream_t s);
+void launch_stream_v(const Run &r, const double *src, double *dst, hipStream_t s);
+// the kick of r.f into out, after the elimination that kept r.kept
+void launch_kick_up(const Run &r, double *out, double *dKeep, hipStream_t s);
+size_t kept_doubles(const Run &r);
+// the streaming kick: whether a run's arrays are made for it, whether its
+// steps take it now, the moment and the kick of r.f into c (f's layout;
+// dKeep as below), and the drift's spline from there
+bool kick_stream_shape(const Run &r);
+bool kick_streams(const Run &r);
+void launch_kick_stream(Run &r, hipStream_t s, Timing *t, double *dKeep);
+void launch_spline_from_kick(Run &r, hipStream_t s, Timing *t);
 // the kick of the plane r.f in column form: v-spline of each column of f
 // into d (slice stride cs, row stride nR), then the evaluation
 void launch_kick(Run &r, hipStream_t s, double *d);

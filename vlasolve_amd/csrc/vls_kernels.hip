@@ -693,7 +693,7 @@ k_spline_r(const double *__restrict__ f, double *__restrict__ c, int nR, int nU,
 // substitution instead of taking a second trip through memory.  A block
 // covers TC columns (TC <= 64, chosen from the LDS budget).
 __global__ void __launch_bounds__(64)
-k_spline_v(double *__restrict__ c, int nR, int nU, int nJ, int64_t cs, int TC, int lzmask,
+k_spline_v(const double *src, double *c, int nR, int nU, int nJ, int64_t cs, int TC, int lzmask,
            ThomasAxis ax) {
   extern __shared__ double ybuf[];  // [M][TC]
   const int lane = threadIdx.x;
@@ -704,145 +704,18 @@ k_spline_v(double *__restrict__ c, int nR, int nU, int nJ, int64_t cs, int TC, i
   const int64_t st = nR + 2;
   const bool live = col < nR + 2;
   // dead lanes read a valid column and store nothing
-  double *tab = c + (size_t)j * cs + (live ? col : nR + 1);
+  const int64_t at = (int64_t)j * cs + (live ? col : nR + 1);
+  const double *in = src + at;
+  double *tab = c + at;
   double ym2, ym1;
   thomas_forward<24>(
-      ax, lz, [&](int k) { return tab[(int64_t)k * st]; },
+      ax, lz, [&](int k) { return in[(int64_t)k * st]; },
       [&](int k, double y) { ybuf[k * TC + lane] = y; }, ym2, ym1);
   thomas_backward<12>(
       ax, lz, ym2, ym1, [&](int k) { return ybuf[k * TC + lane]; },
       [&](int k, double v) {
         if (live) tab[(int64_t)k * st] = v;
       });
-}
-
-// Streaming line solvers for lines too long for an LDS tile of 64 lines
-// (M > ~100): the forward values y_k take a trip through memory (written
-// over the line, read back by the back substitution) instead of waiting on
-// chip, so that no LDS per line is needed and every line of the grid is in
-// flight at once; they move 4 doubles per coefficient instead of 2.  Same
-// operations in the same order as thomas_forward / thomas_backward.
-//
-// v direction: lane = padded column, 64 per wave, every access a coalesced
-// row segment, kPF rows ahead both ways; in place on c.
-__global__ void __launch_bounds__(64)
-k_spline_v_stream(double *__restrict__ c, int nR, int64_t cs, int lzmask, ThomasAxis ax) {
-  const int lane = threadIdx.x;
-  const int lz = lane & lzmask;  // a zero the compiler treats as per-lane
-  const int S = nR + 2;
-  const Tile2 t = xcd_tile2((S + 63) / 64);
-  const int col = t.x * 64 + lane;
-  if (col >= S) return;  // no barriers below
-  double *tab = c + (size_t)t.j * cs + col;
-  double ym2, ym1;
-  thomas_forward<16>(
-      ax, lz, [&](int k) { return tab[(int64_t)k * S]; },
-      [&](int k, double y) { tab[(int64_t)k * S] = y; }, ym2, ym1);
-  thomas_backward<16>(
-      ax, lz, ym2, ym1, [&](int k) { return tab[(int64_t)k * S]; },
-      [&](int k, double v) { tab[(int64_t)k * S] = v; });
-}
-
-// r direction: lane = row, 64 consecutive rows of a slice per wave; chunks
-// of kC columns through a small LDS transpose (4 rows x kC columns per pass,
-// so that the global accesses are row segments).  The forward sweep reads
-// f and leaves y_k in the padded coefficient rows, the back substitution
-// reads them back a chunk at a time from the last column down.
-__global__ void __launch_bounds__(64)
-k_spline_r_stream(const double *__restrict__ f, double *__restrict__ c, int nR, int nU,
-                  int64_t cs, int lzmask, ThomasAxis ax) {
-  constexpr int kC = 16, kP = kC + 1;
-  __shared__ double chunk[64 * kP];
-  const int M = nR + 2;
-  const int lane = threadIdx.x;
-  const int lz = lane & lzmask;
-  const int j = blockIdx.y;
-  const int u0 = blockIdx.x * 64;
-  const int rows = min(64, nU - u0);
-  const int rsub = lane / kC, ksub = lane % kC;
-  const double *src = f + ((size_t)j * nU + u0) * nR;
-  double *dst = c + (size_t)j * cs + (size_t)(u0 + 1) * M;
-  double v[kC];
-  // columns [e0, e0 + kC) of a (rows x width) array into v[] of the lane's row
-  auto gather = [&](const double *a, int width, int e0) {
-    const int e = e0 + ksub;
-    // every load of the chunk leaves before the first LDS write (the
-    // scheduler would otherwise issue a few, wait for them, and go on)
-    double t[kC];
-#pragma unroll
-    for (int q = 0; q < kC; q++) {
-      const int row = min(q * 4 + rsub, rows - 1);
-      t[q] = a[(size_t)row * width + min(e, width - 1)];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int q = 0; q < kC; q++) chunk[(q * 4 + rsub) * kP + ksub] = e < width ? t[q] : 0.0;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kC; i++) v[i] = chunk[lane * kP + i];
-    __syncthreads();
-  };
-  auto scatter = [&](double *a, int width, int e0) {
-#pragma unroll
-    for (int i = 0; i < kC; i++) chunk[lane * kP + i] = v[i];
-    __syncthreads();
-    const int e = e0 + ksub;
-#pragma unroll
-    for (int q = 0; q < kC; q++) {
-      const int row = q * 4 + rsub;
-      if (row < rows && e < width) a[(size_t)row * width + e] = chunk[row * kP + ksub];
-    }
-    __syncthreads();
-  };
-  const double c16 = ax.c16 + (double)lz, rdS = ax.rdS + (double)lz, rlS = ax.rlS + (double)lz;
-  double ym1 = ax.A03, ym2 = 0.0;
-  // forward elimination: rhs_k = f[k-1], y_k to padded column k
-  for (int e0 = 0; e0 < nR; e0 += kC) {
-    gather(src, nR, e0);
-#pragma unroll
-    for (int i = 0; i < kC; i++) {
-      const int k = e0 + i + 1;
-      if (k <= M - 2) {
-        double dv = rdS, ev = rlS;
-        if (k <= kHead) {
-          dv = ax.rd[k + lz];
-          ev = ax.rl[k + lz];
-        }
-        const double yk = div_pivot(v[i] - c16 * ym1, dv, ev);
-        v[i] = yk;
-        ym2 = ym1;
-        ym1 = yk;
-      }
-    }
-    scatter(dst, M, e0 + 1);
-  }
-  // last row, back substitution and first row, chunks of padded columns
-  double tt = 0.0 - ax.hi2 * ym2;
-  tt = tt - ax.p * ym1;
-  double cn = div_known(tt, ax.q, ax.rq);
-  const double uS = ax.uS + (double)lz;
-  double c1 = 0.0, c2 = cn;
-  for (int e0 = ((M - 1) / kC) * kC; e0 >= 0; e0 -= kC) {
-    gather(dst, M, e0);
-#pragma unroll
-    for (int i = kC - 1; i >= 0; i--) {
-      const int k = e0 + i;
-      if (k == M - 1) {
-        v[i] = cn;
-      } else if (k >= 1 && k <= M - 2) {
-        double uv = uS;
-        if (k <= kHead) uv = ax.u[k + lz];
-        const double ck = v[i] - uv * cn;
-        v[i] = ck;
-        c2 = cn;
-        cn = ck;
-        c1 = ck;
-      } else if (k == 0) {
-        v[i] = (ax.A03 - ax.A01 * c1) - ax.A02 * c2;
-      }
-    }
-    scatter(dst, M, e0);
-  }
 }
 
 // Whole-line solve in registers, for a line length M known at compile time.
@@ -1441,12 +1314,15 @@ k_kick_vsolve(const double *__restrict__ f, double *__restrict__ d, int nR, int 
       [&](int k, double v) { dc[(int64_t)k * nR] = v; });
 }
 
+// kDown: the elimination alone, keeping the y of every kSegRows-th row but
+// the last in d ([j][k / kSegRows - 1][r]) for k_kick_up; else
 // k_kick_vsolve with the moment of the same f (as k_kick_solve_moment does
 // for the register lines): tiles of 63 columns, lane 63 solving the next
 // tile's first column for its values only; the moment's terms are taken as
 // the raw rows are used by the forward sweep, the group and block sums as
 // left folds (((G0 + G1) + G2) + G3 with the groups past the last row as 0),
 // then moment_tail.  Dynamic LDS: nU + 2 nR doubles.
+template <bool kDown>
 __global__ void __launch_bounds__(64)
 k_kick_vsolve_moment(const double *__restrict__ f, double *__restrict__ d, int nR, int nU, int nJ,
                      int64_t ds, int lzmask, ThomasAxis ax, MomentArgs ma) {
@@ -1494,15 +1370,20 @@ k_kick_vsolve_moment(const double *__restrict__ f, double *__restrict__ d, int n
   thomas_forward<16>(
       ax, lz, [&](int k) { return fc[(int64_t)(k - 1) * nR]; },
       [&](int k, double y) {
-        if (owner) dc[(int64_t)k * nR] = y;
+        if constexpr (kDown) {
+          if (k % kSegRows == 0 && k < nU && owner) dc[(int64_t)(k / kSegRows - 1) * nR] = y;
+        } else {
+          if (owner) dc[(int64_t)k * nR] = y;
+        }
       },
       ym2, ym1, consume);
   for (int w = (nU - 2) / 64 + 1; w < nW; w++) Pj = Pj + 0.0;
-  thomas_backward<16>(
-      ax, lz, ym2, ym1, [&](int k) { return dc[(int64_t)k * nR]; },
-      [&](int k, double v) {
-        if (owner) dc[(int64_t)k * nR] = v;
-      });
+  if constexpr (!kDown)
+    thomas_backward<16>(
+        ax, lz, ym2, ym1, [&](int k) { return dc[(int64_t)k * nR]; },
+        [&](int k, double v) {
+          if (owner) dc[(int64_t)k * nR] = v;
+        });
   if (owner) coherent_store(&ma.P[(size_t)j * nR + colRaw], term ? Pj : 0.0);
   moment_tail<1>(ma, j, x, nR, nJ, sdm, &last);
 }
@@ -2590,17 +2471,16 @@ bool kick_rsolve_shape(const Run &r) {
 
 // The drift's r-direction solves (rows of src -> padded rows of c) and its
 // v-direction solves (in place on c), with the run's schedule.
-static void launch_spline_r(Run &r, const double *src, hipStream_t s) {
+static void launch_spline_r(Run &r, const double *src, double *dst, hipStream_t s) {
   if (const LineShape *ls = line_shape(r)) {
-    hipLaunchKernelGGL(ls->rows, dim3((r.nU + 63) / 64, r.nJ), dim3(64), 0, s, src, r.c, r.nR,
+    hipLaunchKernelGGL(ls->rows, dim3((r.nU + 63) / 64, r.nJ), dim3(64), 0, s, src, dst, r.nR,
                        r.nU, r.nJ, r.cs, 0, r.tr);
   } else if (r.streamR) {
-    hipLaunchKernelGGL(k_spline_r_stream, dim3((r.nU + 63) / 64, r.nJ), dim3(64), 0, s, src, r.c,
-                       r.nR, r.nU, r.cs, 0, r.tr);
+    launch_stream_r(r, src, dst, s);
   } else {
     dim3 gr((r.nU + r.TR - 1) / r.TR, r.nJ);
     hipLaunchKernelGGL(k_spline_r, gr, dim3(64), (size_t)r.LS * (r.nR + 2) * sizeof(double), s,
-                       src, r.c, r.nR, r.nU, r.nJ, r.cs, r.TR, r.LS, 0, r.tr);
+                       src, dst, r.nR, r.nU, r.nJ, r.cs, r.TR, r.LS, 0, r.tr);
   }
 }
 
@@ -2611,18 +2491,17 @@ static void launch_spline_v(Run &r, const double *rowsIn, hipStream_t s) {
     hipLaunchKernelGGL(ls->cols, dim3((r.nR + 2 + 63) / 64 * r.nJ), dim3(64), 0, s, rowsIn, r.c,
                        r.nR, r.nU, r.nJ, r.cs, 0, r.tv);
   } else if (r.streamV) {
-    hipLaunchKernelGGL(k_spline_v_stream, dim3((r.nR + 2 + 63) / 64 * r.nJ), dim3(64), 0, s, r.c,
-                       r.nR, r.cs, 0, r.tv);
+    launch_stream_v(r, rowsIn ? rowsIn : r.c, r.c, s);
   } else {
     dim3 gv((r.nR + 2 + r.TC - 1) / r.TC, r.nJ);
     hipLaunchKernelGGL(k_spline_v, gv, dim3(64), (size_t)r.TC * (r.nU + 2) * sizeof(double), s,
-                       r.c, r.nR, r.nU, r.nJ, r.cs, r.TC, 0, r.tv);
+                       rowsIn ? rowsIn : r.c, r.c, r.nR, r.nU, r.nJ, r.cs, r.TC, 0, r.tv);
   }
 }
 
 void launch_spline(Run &r, const double *src, hipStream_t s, Timing *t) {
   time_begin(t, s, "spline_r");
-  launch_spline_r(r, src, s);
+  launch_spline_r(r, src, r.c, s);
   time_mark(t, s, "spline_r");
   time_begin(t, s, "spline_v");
   launch_spline_v(r, nullptr, s);
@@ -2659,7 +2538,7 @@ static bool kick_moment_possible(const Run &r) { return r.nS == 1 && r.mCnt; }
 // buffer instead of c).
 static bool kick_moment(const Run &r) {
   if (!kick_moment_possible(r)) return false;
-  if (r.kickMode >= 0) return r.kickMode == 2;
+  if (r.kickMode >= 0) return r.kickMode == 2 || r.kickMode == 4;
   return getenv("VLS_NO_KICK_MOMENT") == nullptr && !getenv("VLS_FUSED_KICK");
 }
 
@@ -2694,6 +2573,55 @@ void launch_spline_v_timed(Run &r, hipStream_t s, Timing *t) {
   time_mark(t, s, "spline_v");
 }
 
+// The streaming kick (vls_stream.hip; kickMode 4): the elimination of the
+// columns with the moment (it keeps every kSegRows-th row's y), then the back
+// substitution with the evaluation, out of place into c; the r-solves go from
+// there to f's buffer and the v-solves back to c.  5 passes over memory
+// where the column splines written out and read back take 7, against longer
+// chains per column, so it wants columns enough to fill the SIMDs: moment and
+// kick of 513x513x256 take 420 us for 870, of 321x321x200 182 for 249, of
+// 385x385x128 208 for 234, but of 321x321x100 161 for 146 and of 201x201x200,
+// whose lines fit in registers, 111 for 70.  The order of evaluation counts
+// on U_Val rising.
+constexpr int64_t kStreamColumns = 40960;
+
+bool kick_stream_shape(const Run &r) {
+  if (r.nS > 1 || !(r.hinv_v > 0) || r.nU > 8192) return false;
+  // 32-bit byte offsets within a wave's columns
+  if ((64 / r.nR + 2) * r.cs * (int64_t)sizeof(double) >= (int64_t)1 << 32) return false;
+  for (int u = 0; u < r.nU; u++)
+    if (!(r.hU[u] > (u ? r.hU[u - 1] : -HUGE_VAL))) return false;
+  const char *e = getenv("VLS_SPLINE_STREAM");
+  return e ? atoi(e) != 0 : (int64_t)r.nR * r.nJ >= kStreamColumns;
+}
+
+bool kick_streams(const Run &r) {
+  // a point whose delay line was taken away keeps its kicked value in f
+  if (!r.kept || line_shape(r) || r.nChainFlags > r.nChains) return false;
+  return r.kickMode >= 0 ? r.kickMode == 4 : kick_moment(r) && !getenv("VLS_KICK_RSOLVE");
+}
+
+void launch_kick_stream(Run &r, hipStream_t s, Timing *t, double *dKeep) {
+  const MomentArgs ma{r.Ct1, r.dU, r.dR, r.gfac, r.P, r.dM, r.Mx, r.acc, r.mTot, r.mCnt};
+  time_begin(t, s, "kick_solve");
+  hipLaunchKernelGGL(k_kick_vsolve_moment<true>, dim3((r.nR + 62) / 63 * r.nJ), dim3(64),
+                     (size_t)(r.nU + 2 * r.nR) * sizeof(double), s, r.f, r.kept, r.nR, r.nU, r.nJ,
+                     (int64_t)((r.nU - 1) / kSegRows) * r.nR, 0, r.tv, ma);
+  time_mark(t, s, "kick_solve");
+  time_begin(t, s, "kick_eval");
+  launch_kick_up(r, r.c, dKeep, s);
+  time_mark(t, s, "kick_eval");
+}
+
+void launch_spline_from_kick(Run &r, hipStream_t s, Timing *t) {
+  time_begin(t, s, "spline_r");
+  launch_spline_r(r, r.c, r.f, s);
+  time_mark(t, s, "spline_r");
+  time_begin(t, s, "spline_v");
+  launch_spline_v(r, r.f, s);
+  time_mark(t, s, "spline_v");
+}
+
 void launch_spline_kick(Run &r, hipStream_t s, Timing *t, bool moment, double *dKeep) {
   if (moment && kick_moment(r)) {
     // the column splines into c, or where the adjoint keeps them
@@ -2705,7 +2633,7 @@ void launch_spline_kick(Run &r, hipStream_t s, Timing *t, bool moment, double *d
       hipLaunchKernelGGL(ls->kickMoment, grid, dim3(64), 2 * (size_t)r.nR * sizeof(double), s, r.f, d,
                          r.nR, r.nJ, r.cs, 0, r.tv, ma);
     else
-      hipLaunchKernelGGL(k_kick_vsolve_moment, grid, dim3(64), (size_t)(r.nU + 2 * r.nR) * sizeof(double),
+      hipLaunchKernelGGL(k_kick_vsolve_moment<false>, grid, dim3(64), (size_t)(r.nU + 2 * r.nR) * sizeof(double),
                          s, r.f, d, r.nR, r.nU, r.nJ, r.cs, 0, r.tv, ma);
     time_mark(t, s, "kick_solve");
     time_begin(t, s, "kick_eval");
@@ -2793,7 +2721,8 @@ std::string describe(const Run &r, const Sched &c, bool cached) {
     sp = c.streamR ? std::string("r-solve streaming") : "r-solve LDS tile of " + std::to_string(c.TR) + " rows";
     sp += c.streamV ? ", v-solve streaming" : ", v-solve LDS tile of " + std::to_string(c.TC) + " columns";
   }
-  static const char *const kKick[] = {"two-kernel", "fused", "moment-fused", "r-solve-folded"};
+  static const char *const kKick[] = {"two-kernel", "fused", "moment-fused", "r-solve-folded",
+                                     "streaming"};
   snprintf(buf, sizeof buf,
            "%dx%dx%d: %s, %s kick (spline %.1f us, moment, kick and r-solve %.1f us%s)",
            r.nR, r.nU, r.nJ, sp.c_str(), kKick[c.kickMode], c.splineUs, c.kickUs,
@@ -2826,7 +2755,7 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
       probe.LS = lsCands[k];
       probe.TR = probe.LS > 64 ? 64 : probe.LS;
     }
-    const double us = time_us(s, [&] { launch_spline_r(probe, r.f, s); });
+    const double us = time_us(s, [&] { launch_spline_r(probe, r.f, r.c, s); });
     if (us < bestR) {
       bestR = us;
       best.streamR = probe.streamR;
@@ -2872,17 +2801,22 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
       return time_us(s, [&] {
         if (mode == 3) {
           launch_kick_rsolve(r, s, nullptr);
+        } else if (mode == 4) {
+          launch_kick_stream(r, s, nullptr, nullptr);
+          launch_spline_r(r, r.c, r.f, s);
         } else {
           launch_spline_kick(r, s, nullptr, true);
-          launch_spline_r(r, r.f, s);
+          launch_spline_r(r, r.f, r.c, s);
         }
       });
     };
     best.kickMode = 0;
     best.kickUs = time_kick(0);
     if (kick_moment_possible(r)) {
-      for (int mode : {2, 3}) {
+      for (int mode : {2, 3, 4}) {
         if (mode == 3 && (!r.fRows || best.lineMode != 1)) continue;
+        r.kickMode = mode;
+        if (mode == 4 && !kick_streams(r)) continue;
         const double us = time_kick(mode);
         if (us < best.kickUs) {
           best.kickMode = mode;
@@ -2922,7 +2856,10 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
           launch_spline(r, r.f, s, nullptr);
           launch_drift(r, s);
         }
-        if (kick_in_rsolve(r)) {
+        if (kick_streams(r)) {
+          launch_kick_stream(r, s, nullptr, nullptr);
+          launch_spline_from_kick(r, s, nullptr);
+        } else if (kick_in_rsolve(r)) {
           launch_kick_rsolve(r, s, nullptr);
           launch_spline_v_timed(r, s, nullptr);
         } else {
