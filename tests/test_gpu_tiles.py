@@ -1,0 +1,63 @@
+"""The solves and the kick by line tiles in LDS (grids whose slices fit neither
+in a CU's LDS nor in the register kernels) at the sizes where they can go
+wrong, bit for bit against the oracle: lines shorter than the pivots' head,
+around the rows held in registers and past them, the fewest lines a tile may
+have, short last tiles, one and two species.  No tolerance: the operations and
+their order are the oracle's."""
+import numpy as np
+import pytest
+
+from tests.configs import UDF_2SPECIES_DELAYED, UDF_C1, UDF_STRONG_KICK
+
+pytestmark = pytest.mark.gpu
+
+V = pytest.importorskip("vlasolve_amd")
+from oracle import oracle as O  # noqa: E402
+
+# cells of r, v and j (r and v lines have one node more)
+GRIDS = [(3, 3, 2), (14, 15, 4), (15, 16, 9), (22, 24, 6), (30, 31, 5), (63, 40, 7), (94, 95, 3),
+         (102, 103, 3), (110, 112, 2), (150, 131, 2), (131, 257, 2), (257, 130, 2), (340, 60, 2),
+         (20, 619, 2), (619, 20, 2), (640, 20, 2)]
+CASES = {"linking": UDF_C1, "no linking": UDF_C1, "strong kick": UDF_STRONG_KICK,
+         "two species": UDF_2SPECIES_DELAYED}
+
+
+@pytest.mark.parametrize("pr,pu,pj", GRIDS)
+@pytest.mark.parametrize("case", list(CASES))
+def test_line_tiles_bit_exact(monkeypatch, pr, pu, pj, case):
+    monkeypatch.setenv("VLS_NO_SLICE_STEP", "1")
+    cfg = dict(CASES[case], **{"grid.Pres": pr, "grid.Ures": [pu, pj],
+                               "solver.noLinking": int(case == "no linking")})
+    label = f"line tiles {pr + 1} x {pu + 1} x {pj} {case}"
+    print("case " + label, flush=True)
+    gpu, orc = V.Solver(cfg), O.Oracle(cfg, nthreads=0)
+    for k in (1, 2):
+        gpu.step(k)
+        orc.step(k)
+        assert np.array_equal(gpu.f(), orc.f()), label
+    for a, b in zip(gpu.moments(), orc.last_moments()):
+        assert np.array_equal(a, b), label
+
+
+def test_line_tiles_recorded(monkeypatch):
+    """The coefficients, a recorded run's state and its gradient against the
+    streaming kernels (the gradient's sums in LDS have no fixed order: 1e-12
+    of its largest, 5 steps of sums of some tens of terms)."""
+    cfg = dict(UDF_C1, **{"grid.Pres": 40, "grid.Ures": [34, 9]})
+    print("case line tiles recorded", flush=True)
+    monkeypatch.setenv("VLS_NO_SLICE_STEP", "1")
+    seen, grads = [], []
+    for stream in (None, "1"):
+        if stream:
+            monkeypatch.setenv("VLS_SPLINE_STREAM", stream)
+        s = V.Solver(cfg)
+        ctx = s.context
+        s.step(4)
+        got = [s.f(), ctx.coef(0, 3, s.nU, s.nR), *ctx.get_chains()]
+        ctx.record(5, 2)
+        got += [s.f(), *ctx.get_chains()]
+        grads.append(ctx.adjoint(dL_df=np.cos(np.arange(s.f().size)))[0])
+        seen.append(got)
+    for k, (a, b) in enumerate(zip(*seen)):
+        assert np.array_equal(a, b), k
+    assert np.abs(grads[0] - grads[1]).max() <= 1e-12 * np.abs(grads[1]).max()

@@ -732,6 +732,8 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
         VLS_HIP_CHECK(hipStreamSynchronize(s));  // u, rd, rl go out of scope
       }
       vls::configure_slice(maxLds);
+      r.pivots = pivots;
+      vls::choose_line_tiles(r);
       if (pivots && vls::slice_shape(r, maxLds)) {
         // one allocation: the group sums, the counters and the kicked f
         const size_t nG = vls::slice_group_doubles(r);

@@ -64,11 +64,12 @@ struct Run {
   int TR = 32, LS = 0;  // r-sweep tile: rows per block, odd LDS row stride (>= TR)
   int TC = 32;          // v-sweep tile: columns per block
   bool streamR = false, streamV = false;  // streaming solvers for long lines
+  bool tileR = false, tileV = false, tileK = false;  // solves, kick by line tiles (vls_slice.hip)
   // schedule choices (vls_autotune): -1 from the shape and the environment;
   // lineMode 0 / 1: LDS-tiled or streaming solvers / register lines (shapes
-  // that have them); kickMode 0 / 1 / 2 / 3 / 4: two-kernel / fused kick / the
+  // that have them); kickMode 0 / 1 / 2 / 3 / 4 / 5: two-kernel / fused kick / the
   // moment fused into the kick's column splines / that, and the kick's
-  // evaluation folded into the drift's r-solve / streaming
+  // evaluation folded into the drift's r-solve / streaming / column tiles
   int lineMode = -1, kickMode = -1;
   // a step in two launches (vls_slice.hip), for the shapes that have sliceG: -1
   // unless the environment forces one of the other schedules, 0 / 1 tuned
@@ -92,6 +93,7 @@ struct Run {
   // moment
   double *P = nullptr;      // [nJ][nR] per-slice partials
   double *dM = nullptr, *Mx = nullptr, *acc = nullptr, *mTot = nullptr;
+  bool pivots = false;  // the axes have the pivots that vls_slice.hip has as literals
   int cus = 256;  // the compute units the run may count on (an ensemble's runs share them)
   // slice step: the kicked f where several blocks share a slice, their group
   // sums of the moment and their counters (zero between launches)
@@ -243,6 +245,15 @@ bool launch_slice_partials(Run &r, const double *f, double *P, hipStream_t s);
 void launch_slice_start(Run &r, hipStream_t s);
 void launch_slice_kick(Run &r, hipStream_t s, double *dKeep);
 void launch_slice_drift(Run &r, hipStream_t s, bool last);
+// the kick of the plane r.f by column tiles in LDS, in place, with the
+// acceleration of the last launch_moment; dKeep as above
+void launch_kick_tile(Run &r, hipStream_t s, double *dKeep);
+// tileR, tileV, tileK by the run's sizes
+void choose_line_tiles(Run &r);
+// the r-solves (rows; src in f's layout) or v-solves (src in c's layout, dst
+// itself allowed) by tiles of lines in LDS; whether the run's lines fit
+bool line_tile_shape(const Run &r, bool rows);
+void launch_line_tile(const Run &r, bool rows, const double *src, double *dst, hipStream_t s);
 void mark_chains(Run &r, hipStream_t s);  // attach the delay lines to their points
 void launch_stats(Run &r, hipStream_t s);
 // rho[nR], phi[nR] (device) from the moment and enclosed mass of the last launch_moment

@@ -2475,6 +2475,8 @@ static void launch_spline_r(Run &r, const double *src, double *dst, hipStream_t 
   if (const LineShape *ls = line_shape(r)) {
     hipLaunchKernelGGL(ls->rows, dim3((r.nU + 63) / 64, r.nJ), dim3(64), 0, s, src, dst, r.nR,
                        r.nU, r.nJ, r.cs, 0, r.tr);
+  } else if (r.tileR) {
+    launch_line_tile(r, true, src, dst, s);
   } else if (r.streamR) {
     launch_stream_r(r, src, dst, s);
   } else {
@@ -2490,6 +2492,8 @@ static void launch_spline_v(Run &r, const double *rowsIn, hipStream_t s) {
   if (const LineShape *ls = line_shape(r)) {
     hipLaunchKernelGGL(ls->cols, dim3((r.nR + 2 + 63) / 64 * r.nJ), dim3(64), 0, s, rowsIn, r.c,
                        r.nR, r.nU, r.nJ, r.cs, 0, r.tv);
+  } else if (r.tileV) {
+    launch_line_tile(r, false, rowsIn ? rowsIn : r.c, r.c, s);
   } else if (r.streamV) {
     launch_stream_v(r, rowsIn ? rowsIn : r.c, r.c, s);
   } else {
@@ -2579,11 +2583,11 @@ void launch_spline_v_timed(Run &r, hipStream_t s, Timing *t) {
 // there to f's buffer and the v-solves back to c.  5 passes over memory
 // where the column splines written out and read back take 7, against longer
 // chains per column, so it wants columns enough to fill the SIMDs: moment and
-// kick of 513x513x256 take 420 us for 870, of 321x321x200 182 for 249, of
-// 385x385x128 208 for 234, but of 321x321x100 161 for 146 and of 201x201x200,
-// whose lines fit in registers, 111 for 70.  The order of evaluation counts
-// on U_Val rising.
-constexpr int64_t kStreamColumns = 40960;
+// kick of 513x513x256 take 420 us for 870, of 321x321x200 184 for 249 (by
+// column tiles in LDS 214), of 385x385x128 208 for 234 (220), but of
+// 321x321x128 166 by tiles 139 and of 201x201x200, whose lines fit in
+// registers, 111 for 70.  The order of evaluation counts on U_Val rising.
+constexpr int64_t kStreamColumns = 49152;
 
 bool kick_stream_shape(const Run &r) {
   if (r.nS > 1 || !(r.hinv_v > 0) || r.nU > 8192) return false;
@@ -2593,6 +2597,13 @@ bool kick_stream_shape(const Run &r) {
     if (!(r.hU[u] > (u ? r.hU[u - 1] : -HUGE_VAL))) return false;
   const char *e = getenv("VLS_SPLINE_STREAM");
   return e ? atoi(e) != 0 : (int64_t)r.nR * r.nJ >= kStreamColumns;
+}
+
+// The kick by column tiles in LDS (vls_slice.hip; kickMode 5), after the
+// moment in a launch of its own
+static bool kick_tiles(const Run &r) {
+  if (!r.tileK || line_shape(r)) return false;
+  return r.kickMode >= 0 ? r.kickMode == 5 : kick_moment(r) || r.nS > 1;
 }
 
 bool kick_streams(const Run &r) {
@@ -2623,6 +2634,17 @@ void launch_spline_from_kick(Run &r, hipStream_t s, Timing *t) {
 }
 
 void launch_spline_kick(Run &r, hipStream_t s, Timing *t, bool moment, double *dKeep) {
+  if (kick_tiles(r)) {
+    if (moment) {
+      time_begin(t, s, "moment");
+      launch_moment(r, s);
+      time_mark(t, s, "moment");
+    }
+    time_begin(t, s, "kick");
+    launch_kick_tile(r, s, dKeep);
+    time_mark(t, s, "kick");
+    return;
+  }
   if (moment && kick_moment(r)) {
     // the column splines into c, or where the adjoint keeps them
     double *d = dKeep ? dKeep : r.c;
@@ -2668,7 +2690,7 @@ void launch_spline_kick(Run &r, hipStream_t s, Timing *t, bool moment, double *d
 namespace {
 struct Sched {
   int lineMode, kickMode, TR, LS, TC;
-  bool streamR, streamV;
+  bool streamR, streamV, tileR, tileV;
   double splineUs, kickUs;
   bool slice = false;              // a step in two launches
   double stepUs = 0, sliceUs = 0;  // a step of the kernels per phase, and of the slice step
@@ -2684,6 +2706,8 @@ void apply_sched(Run &r, const Sched &c) {
   r.TC = c.TC;
   r.streamR = c.streamR;
   r.streamV = c.streamV;
+  r.tileR = c.tileR;
+  r.tileV = c.tileV;
   r.sliceMode = c.slice ? 1 : 0;
 }
 
@@ -2718,11 +2742,15 @@ std::string describe(const Run &r, const Sched &c, bool cached) {
   if (c.lineMode == 1) {
     sp = "register lines";
   } else {
-    sp = c.streamR ? std::string("r-solve streaming") : "r-solve LDS tile of " + std::to_string(c.TR) + " rows";
-    sp += c.streamV ? ", v-solve streaming" : ", v-solve LDS tile of " + std::to_string(c.TC) + " columns";
+    sp = c.tileR     ? std::string("r-solve LDS tiles")
+         : c.streamR ? std::string("r-solve streaming")
+                     : "r-solve LDS tile of " + std::to_string(c.TR) + " rows";
+    sp += c.tileV     ? ", v-solve LDS tiles"
+          : c.streamV ? ", v-solve streaming"
+                      : ", v-solve LDS tile of " + std::to_string(c.TC) + " columns";
   }
   static const char *const kKick[] = {"two-kernel", "fused", "moment-fused", "r-solve-folded",
-                                     "streaming"};
+                                     "streaming", "column-tile"};
   snprintf(buf, sizeof buf,
            "%dx%dx%d: %s, %s kick (spline %.1f us, moment, kick and r-solve %.1f us%s)",
            r.nR, r.nU, r.nJ, sp.c_str(), kKick[c.kickMode], c.splineUs, c.kickUs,
@@ -2743,9 +2771,10 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
   }
   // the drift's spline: register lines where the shape has them, else the
   // best LDS-tiled or streaming solver for each direction
-  Sched best{0, 0, r.TR, r.LS, r.TC, r.streamR, r.streamV, 1e30, 0};
+  Sched best{0, 0, r.TR, r.LS, r.TC, r.streamR, r.streamV, false, false, 1e30, 0};
   Run &probe = r;  // tried in place; the best schedule is applied at the end
   probe.lineMode = 0;
+  probe.tileR = probe.tileV = false;
   double bestR = 1e30, bestV = 1e30;
   std::vector<int> lsCands = {7, 15, 31, 63, 65};
   for (int k = -1; k < (int)lsCands.size(); k++) {
@@ -2763,6 +2792,14 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
       best.TR = probe.TR;
     }
   }
+  if (line_tile_shape(r, true)) {
+    probe.tileR = true;
+    const double us = time_us(s, [&] { launch_spline_r(probe, r.f, r.c, s); });
+    if (us < bestR) {
+      bestR = us;
+      best.tileR = true;
+    }
+  }
   for (int tc : {-1, 8, 16, 32, 64}) {
     if (tc > 0 && (size_t)tc * (r.nU + 2) * sizeof(double) > (size_t)maxLds) continue;
     probe.streamV = tc < 0;
@@ -2772,6 +2809,14 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
       bestV = us;
       best.streamV = probe.streamV;
       best.TC = probe.TC;
+    }
+  }
+  if (line_tile_shape(r, false)) {
+    probe.tileV = true;
+    const double us = time_us(s, [&] { launch_spline_v(probe, nullptr, s); });
+    if (us < bestV) {
+      bestV = us;
+      best.tileV = true;
     }
   }
   best.splineUs = bestR + bestV;
@@ -2812,6 +2857,13 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
     };
     best.kickMode = 0;
     best.kickUs = time_kick(0);
+    if (r.tileK && best.lineMode == 0) {
+      const double us = time_kick(5);
+      if (us < best.kickUs) {
+        best.kickMode = 5;
+        best.kickUs = us;
+      }
+    }
     if (kick_moment_possible(r)) {
       for (int mode : {2, 3, 4}) {
         if (mode == 3 && (!r.fRows || best.lineMode != 1)) continue;

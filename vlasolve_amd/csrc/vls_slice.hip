@@ -227,7 +227,7 @@ __device__ __forceinline__ void lds_line(double *p, int st, int L, const LineTab
 struct KickArgs {
   const double *src;   // f [nS][nJ][nU][nR]
   double *dst;         // the kicked f (may be src)
-  const double *P;     // moment partials [nJ][nR] of f
+  const double *P;     // moment partials [nJ][nR] of f (null: acc holds the acceleration)
   double *dKeep;       // the column splines [j][m][r], slice stride cs (null: not kept)
   const double *gfac, *U_Val;
   double *dM, *Mx, *acc, *mTot;
@@ -246,8 +246,8 @@ struct KickArgs {
 // block has a CU for itself (twice the waves in the evaluation), else 256 (two
 // blocks on a CU, two solves side by side).
 
-inline size_t kick_lds(int nR, int nU, int nJ, int W) {
-  const size_t nC = (nJ + kJC - 1) / kJC;
+inline size_t kick_lds(int nR, int nU, int nJ, int W, bool sums) {
+  const size_t nC = sums ? (nJ + kJC - 1) / kJC : 0;
   return ((size_t)W * (nU + 3) + nU + nR + nC * nR + 1) * sizeof(double) + sizeof(LineTab);
 }
 
@@ -309,7 +309,7 @@ template <int kTK>
 __global__ void __launch_bounds__(kTK) k_kick_tile(KickArgs a) {
   extern __shared__ double lds[];
   const int nR = a.nR, nU = a.nU, nJ = a.nJ, W = a.W;
-  const int nC = (nJ + kJC - 1) / kJC;
+  const int nC = a.P ? (nJ + kJC - 1) / kJC : 0;
   double *D = lds, *Us = D + W * (nU + 3), *accs = Us + nU;
   double *Sc = accs + nR;
   LineTab *hv = (LineTab *)(Sc + nC * nR);
@@ -329,7 +329,7 @@ __global__ void __launch_bounds__(kTK) k_kick_tile(KickArgs a) {
     *ready = 0;
   }
   for (int u = t; u < nU; u += kTK) Us[u] = a.U_Val[u];
-  for (int r = t; r < nR; r += kTK) accs[r] = a.gfac[r];
+  for (int r = t; r < nR; r += kTK) accs[r] = a.P ? a.gfac[r] : a.acc[r];
   for (int i = t; i < W; i += kTK) D[(nU + 2) * W + i] = 0.0;  // read with weight 0
 
   for (int s = 0; s < a.nS; s++) {
@@ -355,7 +355,7 @@ __global__ void __launch_bounds__(kTK) k_kick_tile(KickArgs a) {
     __syncthreads();
     if (w == 0) {
       if (lane < W) lds_line(D + lane, W, nU, *hv);
-    } else if (s == 0) {
+    } else if (a.P && s == 0) {
       // chunk sums of the partials (k_moment_chunks), a thread per (chunk, r)
 #pragma unroll 1
       for (int i = t - 64; i < nC * nR; i += kTK - 64) {
@@ -840,6 +840,86 @@ int kick_width(const Run &r) {
   return (r.nR + nT - 1) / nT;
 }
 
+// ---------------------------------------------------------------- line tiles
+struct TileArgs {
+  const double *src;
+  double *dst;
+  ThomasAxis ax;
+  int nR, nU, W, nT, pitch;
+  unsigned mulIn, mulOut;  // i / (elements of a row in, out) == __umulhi(i, mul)
+  int64_t cs;
+};
+
+// The r-solves (kRows: lines are rows of f) and v-solves (columns of the
+// padded rows, in place allowed) of a tile of a slice's lines in LDS, for the
+// drift's spline of grids whose slices don't fit in a CU's LDS and whose lines
+// don't fit in registers.  One of the block's two waves solves (222 registers:
+// eight waves a CU); the loads and stores of the other blocks on the CU run
+// beside it.  Blocks of 128 threads and 52 KB took 16 and 26 us where 256 and
+// 80 KB took 15 and 25 at 129x257x96, and 25 and 21 for 23 and 29 at
+// 257x129x128.
+template <bool kRows>
+__global__ void __launch_bounds__(128) k_line_tile(TileArgs a) {
+  extern __shared__ double lds[];
+  constexpr int kTL = 128, kB = 16;
+  const int t = threadIdx.x, W = a.W, nR = a.nR, nU = a.nU, S = nR + 2;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int j = tile / a.nT, l0 = (tile - j * a.nT) * W;
+  const int wid = min(W, (kRows ? nU : S) - l0), ps = a.pitch;
+  double *D = lds;
+  LineTab *tab = (LineTab *)(D + (kRows ? W * ps : (nU + 2) * W));
+  if (t == 0) line_tab(tab, a.ax);
+  if constexpr (kRows) {
+    const double *src = a.src + ((size_t)j * nU + l0) * nR;
+    const int n = wid * nR;
+#pragma unroll 1
+    for (int b = t; b < n; b += kB * kTL) {
+      double v[kB];
+#pragma unroll
+      for (int q = 0; q < kB; q++) v[q] = src[min(b + q * kTL, n - 1)];
+#pragma unroll
+      for (int q = 0; q < kB; q++) {
+        const int e = b + q * kTL;
+        if (e < n) D[1 + e + (int)__umulhi((unsigned)e, a.mulIn) * (ps - nR)] = v[q];
+      }
+    }
+  } else {
+    const double *src = a.src + (size_t)j * a.cs + S + l0;
+    const int n = nU * W;
+#pragma unroll 1
+    for (int b = t; b < n; b += kB * kTL) {
+      double v[kB];
+#pragma unroll
+      for (int q = 0; q < kB; q++) {
+        const int e = min(b + q * kTL, n - 1);
+        const int u = __umulhi((unsigned)e, a.mulIn), c = e - u * W;
+        v[q] = src[(size_t)u * S + min(c, wid - 1)];
+      }
+#pragma unroll
+      for (int q = 0; q < kB; q++)
+        if (b + q * kTL < n) D[W + b + q * kTL] = v[q];
+    }
+  }
+  __syncthreads();
+  if (t < wid) lds_line(kRows ? D + t * ps : D + t, kRows ? 1 : W, kRows ? nR : nU, *tab);
+  __syncthreads();
+  if constexpr (kRows) {
+    double *dst = a.dst + (size_t)j * a.cs + (size_t)(l0 + 1) * S;
+    const int n = wid * S;
+#pragma unroll 4
+    for (int e = t; e < n; e += kTL)
+      dst[e] = D[e + (int)__umulhi((unsigned)e, a.mulOut) * (ps - S)];
+  } else {
+    double *dst = a.dst + (size_t)j * a.cs + l0;
+    const int n = (nU + 2) * W;
+#pragma unroll 4
+    for (int e = t; e < n; e += kTL) {
+      const int u = __umulhi((unsigned)e, a.mulOut), c = e - u * W;
+      if (c < wid) dst[(size_t)u * S + c] = D[e];
+    }
+  }
+}
+
 }  // namespace
 
 // Whether the set-up's table holds the pivots that lds_line has as literals.
@@ -854,7 +934,7 @@ bool slice_pivots(const ThomasAxis &ax, const double *u, const double *rd, const
 
 bool slice_shape(const Run &r, int maxLdsPerBlock) {
   return maxLdsPerBlock >= kMaxLds && slice_lds(r.nR, r.nU, r.maxLines) <= (size_t)kMaxLds &&
-         kick_lds(r.nR, r.nU, r.nJ, kick_width(r)) <= (size_t)kMaxLds;
+         kick_lds(r.nR, r.nU, r.nJ, kick_width(r), true) <= (size_t)kMaxLds;
 }
 
 size_t slice_group_doubles(const Run &r) { return (size_t)r.nJ * ((r.nU + 14) / 16) * r.nR; }
@@ -862,7 +942,8 @@ bool slice_shared(const Run &r) { return slice_parts(r) > 1; }
 
 void configure_slice(int maxLdsPerBlock) {
   for (const void *fn : {(const void *)k_kick_tile<256>, (const void *)k_kick_tile<512>,
-                         (const void *)k_slice_drift, (const void *)k_slice_moment})
+                         (const void *)k_slice_drift, (const void *)k_slice_moment,
+                         (const void *)k_line_tile<true>, (const void *)k_line_tile<false>})
     VLS_HIP_CHECK(
         hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxLdsPerBlock));
 }
@@ -907,21 +988,15 @@ void launch_slice_start(Run &r, hipStream_t s) {
   launch_slice_partials(r, r.f, r.P, s);
 }
 
-void launch_slice_kick(Run &r, hipStream_t s, double *dKeep) {
+static KickArgs kick_args(Run &r, int W) {
   KickArgs k{};
-  k.src = r.sp.no_linking ? kicked(r) : r.f;
-  k.dst = kicked(r);
-  k.P = r.P;
-  k.dKeep = dKeep;
+  k.src = k.dst = r.f;
   k.gfac = r.gfac;
   k.U_Val = r.U_Val;
   k.dM = r.dM;
   k.Mx = r.Mx;
   k.acc = r.acc;
   k.mTot = r.mTot;
-  k.head = r.nChains ? r.ch_head : nullptr;
-  k.len = r.ch_len;
-  k.nChains = r.nChains;
   k.nVal = r.nVal;
   k.cs = r.cs;
   k.Ulo = r.Ulo;
@@ -933,14 +1008,104 @@ void launch_slice_kick(Run &r, hipStream_t s, double *dKeep) {
   k.nU = r.nU;
   k.nJ = r.nJ;
   k.nS = r.nS;
-  k.W = kick_width(r);
-  k.nT = (r.nR + k.W - 1) / k.W;
-  k.mulW = magic(k.W);
+  k.W = W;
+  k.nT = (r.nR + W - 1) / W;
+  k.mulW = magic(W);
   k.mulR = magic(r.nR);
+  return k;
+}
+
+void launch_slice_kick(Run &r, hipStream_t s, double *dKeep) {
+  KickArgs k = kick_args(r, kick_width(r));
+  if (r.sp.no_linking) k.src = kicked(r);
+  k.dst = kicked(r);
+  k.P = r.P;
+  k.dKeep = dKeep;
+  k.head = r.nChains ? r.ch_head : nullptr;
+  k.len = r.ch_len;
+  k.nChains = r.nChains;
   k.roll = r.sp.no_linking ? 2 : 1;
   const bool wide = r.nJ * k.nT <= r.cus;
   hipLaunchKernelGGL(wide ? k_kick_tile<512> : k_kick_tile<256>, dim3(r.nJ * k.nT),
-                     dim3(wide ? 512 : 256), kick_lds(r.nR, r.nU, r.nJ, k.W), s, k);
+                     dim3(wide ? 512 : 256), kick_lds(r.nR, r.nU, r.nJ, k.W, true), s, k);
+}
+
+// Lines per tile of `lines` lines of L rows, in equal tiles of at most kb
+// KiB (other: bytes of them not taken by lines), or of 16 lines if two such
+// tiles fit on a CU (0: they don't).
+static int tile_lines(int L, int lines, size_t other, int kb) {
+  const size_t line = (size_t)((L + 3) | 1) * sizeof(double);
+  const size_t room = (size_t)kb * 1024 - 512 - other, most = (size_t)kMaxLds / 2 - 512;
+  const int W = (int)std::min<size_t>(64, std::max<size_t>(room / line, 16));
+  if (W * line + other > most) return 0;
+  const int nT = (lines + W - 1) / W;
+  return (lines + nT - 1) / nT;
+}
+constexpr int kLineKB = 52, kKickKB = 80;  // three and two blocks on a CU
+
+static int line_tile_width(const Run &r, bool rows) {
+  return tile_lines(rows ? r.nR : r.nU, rows ? r.nU : r.nR + 2, 64, kLineKB);
+}
+static size_t kick_tile_other(const Run &r) {
+  return (r.nU + (size_t)r.nR + 1) * sizeof(double) + sizeof(LineTab);
+}
+
+bool line_tile_shape(const Run &r, bool rows) {
+  return r.pivots && line_tile_width(r, rows) > 0;
+}
+
+// Which of the solves and the kick of a run without register lines go by
+// tiles (the axes have the pivots above).  A tile's time is a line's chain and the CU holds 160 KB of lines,
+// where the streaming solves have every line in flight but wait for memory
+// every segment: tiles win while there are few lines.
+//   r: always where 20 rows fit in a tile, else up to four blocks a CU
+//      (stream, tile in us: 129x257x96 38, 15; 257x129x128 60, 24;
+//      321x321x200 190, 129; 401x401x30 79, 61; but 385x385x128 138, 144 and
+//      481x481x40 101, 105)
+//   v: the blocks in one round, three a CU (37, 26; 28, 21; but 301x301x64
+//      45, 57 and 321x321x100 53, 86: the streaming columns come in rows of
+//      512 bytes)
+//   kick: always, unless it streams (with the moment, for the column splines
+//      and the evaluation: 129x257x96 89, 52; 257x129x128 71, 58; 211x181x64
+//      70, 44; 321x321x128 166 streaming, 139; kick_stream_shape)
+void choose_line_tiles(Run &r) {
+  if (!r.pivots) return;
+  for (const char *e : {"VLS_NO_REGISTER_LINES", "VLS_SPLINE_STREAM", "VLS_TILE_R", "VLS_TILE_V"})
+    if (getenv(e)) return;
+  const int wr = line_tile_width(r, true), wv = line_tile_width(r, false);
+  auto blocks = [&](int lines, int w) { return (int64_t)(lines + w - 1) / w * r.nJ; };
+  r.tileR = wr > 0 && ((r.nR + 4) * sizeof(double) * 20 <= kLineKB * 1024 ||
+                       blocks(r.nU, wr) <= 4 * 256);
+  r.tileV = wv > 0 && blocks(r.nR + 2, wv) <= 3 * 256;
+  r.tileK = !r.kept && tile_lines(r.nU, r.nR, kick_tile_other(r), kKickKB) > 0;
+}
+
+void launch_line_tile(const Run &r, bool rows, const double *src, double *dst, hipStream_t s) {
+  TileArgs a{};
+  a.src = src;
+  a.dst = dst;
+  a.ax = rows ? r.tr : r.tv;
+  a.nR = r.nR;
+  a.nU = r.nU;
+  a.cs = r.cs;
+  const int lines = rows ? r.nU : r.nR + 2;
+  a.W = line_tile_width(r, rows);
+  a.nT = (lines + a.W - 1) / a.W;
+  a.pitch = (r.nR + 2) | 1;
+  a.mulIn = magic(rows ? r.nR : a.W);
+  a.mulOut = magic(rows ? r.nR + 2 : a.W);
+  const size_t lds = (rows ? (size_t)a.W * a.pitch : (size_t)a.W * (r.nU + 2)) * sizeof(double) +
+                     sizeof(LineTab);
+  hipLaunchKernelGGL(rows ? k_line_tile<true> : k_line_tile<false>, dim3(a.nT * r.nJ), dim3(128),
+                     lds, s, a);
+}
+
+void launch_kick_tile(Run &r, hipStream_t s, double *dKeep) {
+  KickArgs k = kick_args(r, tile_lines(r.nU, r.nR, kick_tile_other(r), kKickKB));
+  k.nS = 1;  // the plane r.f
+  k.dKeep = dKeep;
+  hipLaunchKernelGGL(k_kick_tile<256>, dim3(r.nJ * k.nT), dim3(256),
+                     kick_lds(r.nR, r.nU, r.nJ, k.W, false), s, k);
 }
 
 void launch_slice_drift(Run &r, hipStream_t s, bool last) {
