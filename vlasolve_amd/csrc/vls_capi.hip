@@ -97,11 +97,13 @@ void h2d(T *dst, const T *src, size_t n, hipStream_t s) {
 // 100, a 25-step gradient at 201x201x200 (an upload, a download) from 24.1 to
 // 19.8.  The pinned
 // memory (16 MiB) is shared by the process's contexts: made by the first large
-// transfer, held by one transfer at a time (others take the runtime's path
+// download or upload of 64 MiB (making it takes 4 ms: the uploads of a
+// smaller context's set-up are faster without), held by one transfer at a time (others take the runtime's path
 // meanwhile) and given back with the last context.
 struct Staging {
   static constexpr int kThreads = 8;
   static constexpr size_t kPiece = (size_t)1 << 20, kMin = (size_t)2 << 20;
+  static constexpr size_t kMakeIn = (size_t)64 << 20;
   std::mutex use;      // one transfer at a time
   std::mutex mu;       // guards the two below
   char *pin = nullptr;
@@ -119,9 +121,10 @@ struct Staging {
       pin = nullptr;
     }
   }
-  char *memory() {  // with `use` held
+  // with `use` held; make: if there is none yet
+  char *memory(bool make) {
     std::lock_guard<std::mutex> l(mu);
-    if (!pin && hipHostMalloc((void **)&pin, kThreads * 2 * kPiece, hipHostMallocPortable) !=
+    if (!pin && make && hipHostMalloc((void **)&pin, kThreads * 2 * kPiece, hipHostMallocPortable) !=
                     hipSuccess) {
       (void)hipGetLastError();  // no pinned memory: the runtime's path
       pin = nullptr;
@@ -132,7 +135,7 @@ struct Staging {
   // bytes between dev and host on stream s, complete on return
   void copy(void *dev, void *host, size_t bytes, bool out, int device, hipStream_t s) {
     std::unique_lock<std::mutex> u(use, std::try_to_lock);
-    char *p = bytes >= kMin && u.owns_lock() ? memory() : nullptr;
+    char *p = bytes >= kMin && u.owns_lock() ? memory(out || bytes >= kMakeIn) : nullptr;
     if (!p) {
       if (u.owns_lock()) u.unlock();
       VLS_HIP_CHECK(out ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s)
@@ -687,28 +690,28 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
       r.kickScratch = getenv("VLS_KICK_SCRATCH") != nullptr;
       if (streams) r.kept = dalloc<double>(r, vls::kept_doubles(r));
       r.feet = dalloc<double>(r, 2 * r.nVal);
-      r.P = dalloc<double>(r, (size_t)r.nJ * r.nR);
-      r.dM = dalloc<double>(r, r.nR);
-      r.Mx = dalloc<double>(r, r.nR);
-      r.acc = dalloc<double>(r, r.nR);
-      r.mTot = dalloc<double>(r, 1);
       r.mCnt = dalloc<unsigned>(r, vls::moment_counters(r));
       VLS_HIP_CHECK(hipMemsetAsync(r.mCnt, 0, vls::moment_counters(r) * sizeof(unsigned), s));
-      r.rhoPhi = dalloc<double>(r, 2 * (size_t)r.nR);
-      r.st_part = dalloc<double>(r, 7 * (size_t)r.nJ * r.nR);
-      r.st_q = dalloc<double>(r, 6 * (size_t)r.nJ + r.nR);
-      r.st_out = dalloc<double>(r, 14);
+      // the small arrays share an allocation (50 us each on their own)
+      const size_t nR = r.nR, nU = r.nU, nJ = r.nJ;
+      const std::pair<double **, size_t> small[] = {
+          {&r.P, nJ * nR},    {&r.dM, nR},    {&r.Mx, nR},      {&r.acc, nR},
+          {&r.mTot, 1},       {&r.rhoPhi, 2 * nR},              {&r.st_part, 7 * nJ * nR},
+          {&r.st_q, 6 * nJ + nR},             {&r.st_out, 14},  {&r.R_Val, nR},
+          {&r.U_Val, nU},     {&r.J_Val, nJ}, {&r.dR, nR},      {&r.dU, nU},
+          {&r.Ct1, nJ},       {&r.gfac, nR}};
+      auto padded = [](size_t n) { return (n + 31) / 32 * 32; };
+      size_t total = 0;
+      for (const auto &x : small) total += padded(x.second);
+      double *at = dalloc<double>(r, total);
+      for (const auto &x : small) {
+        *x.first = at;
+        at += padded(x.second);
+      }
       // tables
       std::vector<double> Ct1(r.nJ), gfac(r.nR);
       for (int j = 0; j < r.nJ; j++) Ct1[j] = 8 * M_PI * M_PI * G.J_Val[j] * G.dJ[j];
       for (int i = 0; i < r.nR; i++) gfac[i] = r.sp.G / (G.R_Val[i] * G.R_Val[i]) * r.sp.dt;
-      r.R_Val = dalloc<double>(r, r.nR);
-      r.U_Val = dalloc<double>(r, r.nU);
-      r.J_Val = dalloc<double>(r, r.nJ);
-      r.dR = dalloc<double>(r, r.nR);
-      r.dU = dalloc<double>(r, r.nU);
-      r.Ct1 = dalloc<double>(r, r.nJ);
-      r.gfac = dalloc<double>(r, r.nR);
       h2d(r.R_Val, G.R_Val, r.nR, s);
       h2d(r.U_Val, G.U_Val, r.nU, s);
       h2d(r.J_Val, G.J_Val, r.nJ, s);
@@ -819,12 +822,13 @@ int vls_set_drift(vls_ctx *ctx, int run, const double *xr, const double *xu, con
     // the drift kernel reads the point's kind from xr (-1 outside, -2 delay
     // line) and a delay-line point's chain index from xu (-1: none yet)
     std::vector<double> xf(xr, xr + r.nVal), uf(xu, xu + r.nVal);
+    int64_t lines = 0;
     for (int64_t i = 0; i < r.nVal; i++) {
       if (flag[i] == VLS_FOOT_OUT) xf[i] = -1.0;
-      if (flag[i] == VLS_FOOT_CHAIN) xf[i] = -2.0, uf[i] = -1.0;
+      if (flag[i] == VLS_FOOT_CHAIN) xf[i] = -2.0, uf[i] = -1.0, lines++;
     }
     r.hflag.assign(flag, flag + r.nVal);
-    r.nChainFlags = std::count(flag, flag + r.nVal, (uint8_t)VLS_FOOT_CHAIN);
+    r.nChainFlags = lines;
     hipStream_t s = ctx->c.stream;
     std::vector<double> ft(2 * r.nVal);
     for (int64_t i = 0; i < r.nVal; i++) ft[2 * i] = xf[i], ft[2 * i + 1] = uf[i];
