@@ -39,12 +39,14 @@ def test_line_tiles_bit_exact(monkeypatch, pr, pu, pj, case):
         assert np.array_equal(a, b), label
 
 
-def test_line_tiles_recorded(monkeypatch):
+@pytest.mark.parametrize("pr,pu,pj", [(3, 3, 3), (14, 15, 4), (15, 17, 5), (24, 23, 6), (31, 25, 5),
+                                      (40, 34, 9), (150, 131, 3), (64, 64, 4)])
+def test_line_tiles_recorded(monkeypatch, pr, pu, pj):
     """The coefficients, a recorded run's state and its gradient against the
-    streaming kernels (the gradient's sums in LDS have no fixed order: 1e-12
+    streaming kernels, at the edges of the adjoint's chunks too (the gradient's sums in LDS have no fixed order: 1e-12
     of its largest, 5 steps of sums of some tens of terms)."""
-    cfg = dict(UDF_C1, **{"grid.Pres": 40, "grid.Ures": [34, 9]})
-    print("case line tiles recorded", flush=True)
+    cfg = dict(UDF_C1, **{"grid.Pres": pr, "grid.Ures": [pu, pj]})
+    print(f"case line tiles recorded {pr + 1} x {pu + 1} x {pj}", flush=True)
     monkeypatch.setenv("VLS_NO_SLICE_STEP", "1")
     seen, grads = [], []
     for stream in (None, "1"):
@@ -53,7 +55,7 @@ def test_line_tiles_recorded(monkeypatch):
         s = V.Solver(cfg)
         ctx = s.context
         s.step(4)
-        got = [s.f(), ctx.coef(0, 3, s.nU, s.nR), *ctx.get_chains()]
+        got = [s.f(), ctx.coef(0, 2, s.nU, s.nR), *ctx.get_chains()]
         ctx.record(5, 2)
         got += [s.f(), *ctx.get_chains()]
         grads.append(ctx.adjoint(dL_df=np.cos(np.arange(s.f().size)))[0])

@@ -935,16 +935,20 @@ void launch_adj_drift(Run &r, const double *fb, double *cb, double *ringb, const
 }
 
 void launch_adj_spline(Run &r, double *cb, double *out, hipStream_t s) {
-  if (const AdjShape *a = adj_shape(r)) {
-    hipLaunchKernelGGL(a->v, dim3((r.nR + 2 + 63) / 64 * r.nJ), dim3(64), 0, s, cb, r.cs, 0, r.tv);
-    hipLaunchKernelGGL(a->r, dim3((r.nU + 63) / 64, r.nJ), dim3(64), 0, s, cb, out, r.nU, r.cs, 0,
-                       r.tr);
-    return;
-  }
-  hipLaunchKernelGGL(k_adj_v, dim3((r.nR + 2 + 63) / 64 * r.nJ), dim3(64), 0, s, cb, r.nR + 2, r.cs,
-                     r.tv);
-  hipLaunchKernelGGL(k_adj_r, dim3((r.nU + 63) / 64, r.nJ), dim3(64), 0, s, cb, out, r.nR, r.nU,
-                     r.cs, r.tr);
+  const AdjShape *a = adj_shape(r);
+  const dim3 gv((r.nR + 2 + 63) / 64 * r.nJ), gr((r.nU + 63) / 64, r.nJ);
+  if (a)
+    hipLaunchKernelGGL(a->v, gv, dim3(64), 0, s, cb, r.cs, 0, r.tv);
+  else if (adj_line_tile(r, false))
+    launch_adj_line_tile(r, false, cb, nullptr, s);
+  else
+    hipLaunchKernelGGL(k_adj_v, gv, dim3(64), 0, s, cb, r.nR + 2, r.cs, r.tv);
+  if (adj_line_tile(r, true))
+    launch_adj_line_tile(r, true, cb, out, s);
+  else if (a)
+    hipLaunchKernelGGL(a->r, gr, dim3(64), 0, s, cb, out, r.nU, r.cs, 0, r.tr);
+  else
+    hipLaunchKernelGGL(k_adj_r, gr, dim3(64), 0, s, cb, out, r.nR, r.nU, r.cs, r.tr);
 }
 
 void launch_adj_kick(Run &r, const double *fsb, const double *cK, const double *accK, double *cb,

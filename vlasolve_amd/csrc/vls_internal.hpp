@@ -93,6 +93,7 @@ struct Run {
   // moment
   double *P = nullptr;      // [nJ][nR] per-slice partials
   double *dM = nullptr, *Mx = nullptr, *acc = nullptr, *mTot = nullptr;
+  bool lineTiles = false;  // lines may go by tiles (the pivots, and no schedule forced)
   bool pivots = false;  // the axes have the pivots that vls_slice.hip has as literals
   int cus = 256;  // the compute units the run may count on (an ensemble's runs share them)
   // slice step: the kicked f where several blocks share a slice, their group
@@ -248,6 +249,10 @@ void launch_slice_drift(Run &r, hipStream_t s, bool last);
 // the kick of the plane r.f by column tiles in LDS, in place, with the
 // acceleration of the last launch_moment; dKeep as above
 void launch_kick_tile(Run &r, hipStream_t s, double *dKeep);
+// the line adjoints of the drift's spline by tiles: rows of cb to out (f's
+// layout), or its columns in place
+bool adj_line_tile(const Run &r, bool rows);
+void launch_adj_line_tile(const Run &r, bool rows, double *cb, double *out, hipStream_t s);
 // tileR, tileV, tileK by the run's sizes
 void choose_line_tiles(Run &r);
 // the r-solves (rows; src in f's layout) or v-solves (src in c's layout, dst

@@ -920,6 +920,173 @@ __global__ void __launch_bounds__(128) k_line_tile(TileArgs a) {
   }
 }
 
+// ---------------------------------------------------------------- adjoint
+// The line adjoints of the drift's spline (the sweeps of k_adj_v and k_adj_r,
+// vls_adjoint.hip: c1 -= A01 c0, c2 -= A02 c0, c[t] -= u[t-1] c[t-1] going up,
+// then the last row, the scaling by 1/d and the carry c16 c[k] going down) by
+// tiles of lines in LDS: the streaming kernels take the line through memory
+// twice each way.  Same operations, same order.  A block's first wave
+// sweeps (a chain of 1 and 3 dependent operations, a DS read and a write a row).
+struct AdjTileArgs {
+  double *cb;   // padded coefficients' adjoints; columns: in place
+  double *out;  // rows: f's layout
+  ThomasAxis ax;
+  int nR, nU, W, nT, pitch;
+  unsigned mulIn, mulOut;
+  int64_t cs;
+};
+
+// A line in LDS, in place: p[k st], k = 0..M-1.  Chunks of kQ rows, read a
+// chunk ahead.
+__device__ __forceinline__ void lds_line_adjoint(double *p, int st, const ThomasAxis &ax) {
+  const int M = ax.M;
+  constexpr int kQ = 8, kH = kHead + 2;  // rows 0 .. kHead + 1 take the pivots of the head
+  st = __builtin_amdgcn_readfirstlane(st);
+  asm volatile("" : "+s"(st));
+  const double uS = kPivU[kHead + 1], rdS = kPivRd[kHead + 1];
+  double h[kH];
+#pragma unroll
+  for (int t = 0; t < kH; t++) h[t] = p[min(t, M - 1) * st];
+  double prev = 0.0;
+#pragma unroll
+  for (int t = 0; t < kH; t++) {
+    if (t < M) {
+      if (t == 1) h[t] = fma(-ax.A01, h[0], h[t]);
+      if (t == 2) h[t] = fma(-ax.A02, h[0], h[t]);
+      if (t >= 2) h[t] = fma(-kPivU[t - 1], prev, h[t]);
+      prev = h[t];
+      p[t * st] = prev;
+    }
+  }
+  double a[kQ];
+  double *sp = p + kH * st;
+  int t = kH;
+  if (t + kQ <= M) {
+#pragma unroll
+    for (int q = 0; q < kQ; q++) a[q] = sp[q * st];
+#pragma unroll 1
+    for (; t + 2 * kQ <= M; t += kQ) {
+      double b[kQ];
+#pragma unroll
+      for (int q = 0; q < kQ; q++) b[q] = a[q];
+#pragma unroll
+      for (int q = 0; q < kQ; q++) a[q] = sp[(kQ + q) * st];
+#pragma unroll
+      for (int q = 0; q < kQ; q++) {
+        prev = fma(-uS, prev, b[q]);
+        *sp = prev;
+        sp += st;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kQ; q++) {
+      prev = fma(-uS, prev, a[q]);
+      *sp = prev;
+      sp += st;
+    }
+    t += kQ;
+  }
+  for (; t < M; t++) {
+    prev = fma(-uS, prev, *sp);
+    *sp = prev;
+    sp += st;
+  }
+  const double tt = prev * ax.rq;  // prev = c[M-1]
+  double carry = 0.0;
+  auto down = [&](double v) {
+    v *= rdS;
+    carry = ax.c16 * v;
+    *sp = v;
+    sp -= st;
+  };
+  sp = p + (M - 2) * st;
+  int k = M - 2;
+  if (k > kHead) {
+    down(fma(-ax.p, tt, *sp - carry));
+    k--;
+  }
+  if (k > kHead && k == M - 3) {
+    down(fma(-ax.hi2, tt, *sp - carry));
+    k--;
+  }
+  if (k - kQ >= kHead) {
+#pragma unroll
+    for (int q = 0; q < kQ; q++) a[q] = sp[-q * st];
+#pragma unroll 1
+    for (; k - 2 * kQ >= kHead; k -= kQ) {
+      double b[kQ];
+#pragma unroll
+      for (int q = 0; q < kQ; q++) b[q] = a[q];
+#pragma unroll
+      for (int q = 0; q < kQ; q++) a[q] = sp[-(kQ + q) * st];
+#pragma unroll
+      for (int q = 0; q < kQ; q++) down(b[q] - carry);
+    }
+#pragma unroll
+    for (int q = 0; q < kQ; q++) down(a[q] - carry);
+    k -= kQ;
+  }
+  for (; k > kHead; k--) down(*sp - carry);
+#pragma unroll
+  for (int m = kHead; m >= 1; m--) {
+    if (m <= M - 2) {
+      double v = h[m] - carry;
+      if (m == M - 2) v = fma(-ax.p, tt, v);
+      if (m == M - 3) v = fma(-ax.hi2, tt, v);
+      v *= kPivRd[m];
+      carry = ax.c16 * v;
+      p[m * st] = v;
+    }
+  }
+}
+
+template <bool kRows>
+__global__ void __launch_bounds__(128) k_adj_line_tile(AdjTileArgs a) {
+  extern __shared__ double D[];
+  constexpr int kTL = 128, kB = 16;
+  const int t = threadIdx.x, W = a.W, nR = a.nR, nU = a.nU, S = nR + 2;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int j = tile / a.nT, l0 = (tile - j * a.nT) * W;
+  const int wid = min(W, (kRows ? nU : S) - l0), ps = a.pitch;
+  double *src = a.cb + (size_t)j * a.cs + (kRows ? (size_t)(l0 + 1) * S : l0);
+  const int n = kRows ? wid * S : (nU + 2) * W;
+#pragma unroll 1
+  for (int b = t; b < n; b += kB * kTL) {
+    double v[kB];
+#pragma unroll
+    for (int q = 0; q < kB; q++) {
+      const int e = min(b + q * kTL, n - 1);
+      if constexpr (kRows) {
+        v[q] = src[e];
+      } else {
+        const int m = __umulhi((unsigned)e, a.mulIn), c = e - m * W;
+        v[q] = src[(size_t)m * S + min(c, wid - 1)];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kB; q++) {
+      const int e = b + q * kTL;
+      if (e < n) D[kRows ? e + (int)__umulhi((unsigned)e, a.mulIn) * (ps - S) : e] = v[q];
+    }
+  }
+  __syncthreads();
+  if (t < wid) lds_line_adjoint(kRows ? D + t * ps : D + t, kRows ? 1 : W, a.ax);
+  __syncthreads();
+  if constexpr (kRows) {
+    double *dst = a.out + ((size_t)j * nU + l0) * nR;
+#pragma unroll 4
+    for (int e = t; e < wid * nR; e += kTL)
+      dst[e] = D[1 + e + (int)__umulhi((unsigned)e, a.mulOut) * (ps - nR)];
+  } else {
+    // rows 1 .. nU: the r-direction takes no others
+#pragma unroll 4
+    for (int e = t; e < nU * W; e += kTL) {
+      const int u = __umulhi((unsigned)e, a.mulOut), c = e - u * W;
+      if (c < wid) src[(size_t)(u + 1) * S + c] = D[W + e];
+    }
+  }
+}
+
 }  // namespace
 
 // Whether the set-up's table holds the pivots that lds_line has as literals.
@@ -943,7 +1110,9 @@ bool slice_shared(const Run &r) { return slice_parts(r) > 1; }
 void configure_slice(int maxLdsPerBlock) {
   for (const void *fn : {(const void *)k_kick_tile<256>, (const void *)k_kick_tile<512>,
                          (const void *)k_slice_drift, (const void *)k_slice_moment,
-                         (const void *)k_line_tile<true>, (const void *)k_line_tile<false>})
+                         (const void *)k_line_tile<true>, (const void *)k_line_tile<false>,
+                         (const void *)k_adj_line_tile<true>,
+                         (const void *)k_adj_line_tile<false>})
     VLS_HIP_CHECK(
         hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxLdsPerBlock));
 }
@@ -1072,6 +1241,7 @@ void choose_line_tiles(Run &r) {
   if (!r.pivots) return;
   for (const char *e : {"VLS_NO_REGISTER_LINES", "VLS_SPLINE_STREAM", "VLS_TILE_R", "VLS_TILE_V"})
     if (getenv(e)) return;
+  r.lineTiles = true;
   const int wr = line_tile_width(r, true), wv = line_tile_width(r, false);
   auto blocks = [&](int lines, int w) { return (int64_t)(lines + w - 1) / w * r.nJ; };
   r.tileR = wr > 0 && ((r.nR + 4) * sizeof(double) * 20 <= kLineKB * 1024 ||
@@ -1098,6 +1268,41 @@ void launch_line_tile(const Run &r, bool rows, const double *src, double *dst, h
                      sizeof(LineTab);
   hipLaunchKernelGGL(rows ? k_line_tile<true> : k_line_tile<false>, dim3(a.nT * r.nJ), dim3(128),
                      lds, s, a);
+}
+
+constexpr int kAdjKB = 40;  // four blocks on a CU (of 26 KB: 5% slower)
+static int adj_tile_width(const Run &r, bool rows) {
+  return tile_lines(rows ? r.nR : r.nU, rows ? r.nU : r.nR + 2, 0, kAdjKB);
+}
+
+// The blocks of the tiles in one round: us of the streaming sweeps and of the
+// tiles, r: 40 and 16 on average over runs of 151x132x96, 211x181x64,
+// 132x258x70 and 97x65x48, v: 31 and 20; at 201x201x200 (1800 blocks) 73 and 47,
+// 52 and 51, but the walk after it then takes 27 more.  On register shapes
+// the columns are faster there (129x129x64: 9 us against 17), the rows here
+// (18 against 14).
+bool adj_line_tile(const Run &r, bool rows) {
+  const int w = r.lineTiles ? adj_tile_width(r, rows) : 0, lines = rows ? r.nU : r.nR + 2;
+  return w > 0 && (int64_t)(lines + w - 1) / w * r.nJ <= 4 * 256;
+}
+
+void launch_adj_line_tile(const Run &r, bool rows, double *cb, double *out, hipStream_t s) {
+  AdjTileArgs a{};
+  a.cb = cb;
+  a.out = out;
+  a.ax = rows ? r.tr : r.tv;
+  a.nR = r.nR;
+  a.nU = r.nU;
+  a.cs = r.cs;
+  const int lines = rows ? r.nU : r.nR + 2;
+  a.W = adj_tile_width(r, rows);
+  a.nT = (lines + a.W - 1) / a.W;
+  a.pitch = (r.nR + 2) | 1;
+  a.mulIn = magic(rows ? r.nR + 2 : a.W);
+  a.mulOut = magic(rows ? r.nR : a.W);
+  const size_t lds = (size_t)a.W * (rows ? a.pitch : r.nU + 2) * sizeof(double);
+  hipLaunchKernelGGL(rows ? k_adj_line_tile<true> : k_adj_line_tile<false>, dim3(a.nT * r.nJ),
+                     dim3(128), lds, s, a);
 }
 
 void launch_kick_tile(Run &r, hipStream_t s, double *dKeep) {
