@@ -156,9 +156,9 @@ int vls_set_timing(vls_ctx *ctx, int on);
 int vls_kernel_times(vls_ctx *ctx, const char **names, double *ms, int *n);
 /* Schedule tuner: times the run's line-solve schedules on its current data
  * and keeps the fastest -- register lines (shapes that have them), or the
- * LDS-tiled solvers with the tile size chosen from a set of candidates, or
- * the streaming solvers, for each direction -- then the fused or two-kernel
- * kick on a copy of f.  run = -1 tunes every run of the context.  Every
+ * LDS-tiled solvers with the tile size chosen from a set of candidates, line
+ * tiles or the streaming solvers, for each direction -- then the kick's
+ * schedules on a copy of f, then whole steps against the slice step.  run = -1 tunes every run of the context.  Every
  * schedule runs the same operations in the same order: the choice changes
  * the time of a step, never its bits.  Choices are cached per grid shape for
  * the life of the process; desc (may be NULL) receives one line per run
@@ -167,7 +167,8 @@ int vls_kernel_times(vls_ctx *ctx, const char **names, double *ms, int *n);
 int vls_autotune(vls_ctx *ctx, int run, char *desc, int descLen);
 
 /* Restrict the timing to one kernel ("kick_line", "drift", "spline_r",
- * "spline_v", "moment", "kick"): an event before and after each of its
+ * "spline_v", "moment", "kick", "kick_solve", "kick_eval", "slice_start",
+ * "slice_kick", "slice_drift"): an event before and after each of its
  * launches only, so that the other kernels run as without timing; NULL
  * times every kernel again.  No counterpart in the reference. */
 int vls_set_timing_kernel(vls_ctx *ctx, const char *kernel);

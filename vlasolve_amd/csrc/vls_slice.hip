@@ -30,6 +30,8 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <mutex>
+#include <set>
 
 #include "vls_device.hpp"
 #include "vls_div.hpp"
@@ -1108,6 +1110,13 @@ size_t slice_group_doubles(const Run &r) { return (size_t)r.nJ * ((r.nU + 14) / 
 bool slice_shared(const Run &r) { return slice_parts(r) > 1; }
 
 void configure_slice(int maxLdsPerBlock) {
+  // once per device: a tenth of a small context's creation otherwise
+  static std::mutex mu;
+  static std::set<int> done;
+  int device = 0;
+  VLS_HIP_CHECK(hipGetDevice(&device));
+  std::lock_guard<std::mutex> lock(mu);
+  if (done.count(device)) return;
   for (const void *fn : {(const void *)k_kick_tile<256>, (const void *)k_kick_tile<512>,
                          (const void *)k_slice_drift, (const void *)k_slice_moment,
                          (const void *)k_line_tile<true>, (const void *)k_line_tile<false>,
@@ -1115,6 +1124,7 @@ void configure_slice(int maxLdsPerBlock) {
                          (const void *)k_adj_line_tile<false>})
     VLS_HIP_CHECK(
         hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxLdsPerBlock));
+  done.insert(device);
 }
 
 bool slice_fits(const Run &r) {
