@@ -9,8 +9,9 @@
 // elimination from the kept y before it in registers and substitutes back:
 // two reads and one write.  The repeated operations are the same, so are the
 // bits.  At 513x513x256, whose planes of 0.54 GB come from HBM, the v-solves
-// take 342 to 374 us for 477 and the r-solves 496 to 509 for 646 (with
-// segments of 256 instead of 128 bytes of a row as well).  Columns take
+// take 342 to 374 us for 477 and the r-solves 496 to 516 for 646 (637 with
+// segments of 16 columns: rows start off the 128-byte lines, and a segment's
+// first and last line are fetched twice).  Columns take
 // segments of 16 rows: of 32, the two copies of a segment do not fit in the
 // 168 registers that leave three waves a SIMD.
 #pragma clang fp contract(off)
