@@ -124,7 +124,7 @@ int vls_synchronize(vls_ctx *ctx);
 /* Ensembles (nRuns > 1): by default vls_step captures one step of all runs
  * as a HIP graph, each run on a stream of its own so that runs of different
  * sizes execute concurrently, and replays it once per step (the graph is
- * rebuilt after vls_set_chains).  on = 0 steps the runs one after the other
+ * rebuilt after vls_set_drift, vls_set_chains and vls_autotune).  on = 0 steps the runs one after the other
  * on the context stream.  No counterpart in the reference, which runs one
  * model per process. */
 int vls_set_graph(vls_ctx *ctx, int on);

@@ -1,0 +1,86 @@
+"""Foot tables changed between steps: every schedule, and the captured step of
+an ensemble, gives the bits of the kernels per phase.  No tolerance: the
+schedules run the same operations."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from tests.configs import UDF_C1
+
+pytestmark = pytest.mark.gpu
+
+V = pytest.importorskip("vlasolve_amd")
+
+OUT, CHAIN = 1, 2
+NO_LINES = {"VLS_NO_SLICE_STEP": "1", "VLS_NO_REGISTER_LINES": "1"}
+PHASES = dict(NO_LINES, VLS_SPLINE_STREAM="0")
+SCHEDULES = {"slice": {}, "streams": dict(NO_LINES, VLS_SPLINE_STREAM="1")}
+
+
+def _cfg(pr=40, pu=34, pj=9):
+    return dict(UDF_C1, **{"grid.Pres": pr, "grid.Ures": [pu, pj]})
+
+
+def _p(a, t=C.c_double):
+    return a.ctypes.data_as(C.POINTER(t))
+
+
+def _feet(shape, seed, chains=()):
+    """A foot table inside the domain, a tenth of it outside the grid, the
+    given points on delay lines."""
+    rng = np.random.default_rng(seed)
+    nJ, nU, nR = shape
+    n = nJ * nU * nR
+    xr, xu = rng.uniform(0, nR - 1, n), rng.uniform(0, nU - 1, n)
+    flag = np.where(rng.random(n) < 0.1, OUT, 0).astype(np.uint8)
+    flag[list(chains)] = CHAIN
+    return xr, xu, flag
+
+
+def _set_drift(ctx, run, xr, xu, flag):
+    V._check(V.lib().vls_set_drift(ctx._h, run, _p(xr), _p(xu), _p(flag, C.c_uint8)))
+
+
+def _points(shape, n, seed, taken=()):
+    rng = np.random.default_rng(seed)
+    free = np.setdiff1d(np.arange(int(np.prod(shape))), np.asarray(taken, np.int64))
+    return np.sort(rng.choice(free, n, replace=False))
+
+
+def _under(monkeypatch, env, fn):
+    with monkeypatch.context() as m:
+        for k, v in env.items():
+            m.setenv(k, v)
+        return fn()
+
+
+def _same(a, b):
+    for k, (x, y) in enumerate(zip(a, b)):
+        assert np.array_equal(x, y), (k, np.flatnonzero(np.asarray(x) != np.asarray(y))[:5])
+
+
+@pytest.mark.parametrize("schedule", list(SCHEDULES))
+def test_captured_step_follows_new_feet(monkeypatch, schedule):
+    """An ensemble whose foot table gets delay-line points without lines
+    between two calls: the points keep their kicked value, as in the same
+    steps without the captured graph."""
+    cfgs = [_cfg(), _cfg(33, 30, 6)]
+    print(f"case captured step, new feet, {schedule}", flush=True)
+
+    def run(graph):
+        e = V.Ensemble(cfgs)
+        e.set_graph(graph)
+        ctx = e.context
+        shapes = [e.f(k).shape for k in range(2)]
+        for k, shape in enumerate(shapes):
+            ctx.clear_chains(k)
+            _set_drift(ctx, k, *_feet(shape, k))
+        e.step(2)
+        for k, shape in enumerate(shapes):
+            _set_drift(ctx, k, *_feet(shape, k, _points(shape, 400, 7 + k)))
+        e.step(3)
+        return [e.f(0), e.f(1)]
+
+    want = _under(monkeypatch, PHASES, lambda: run(False))
+    _same(_under(monkeypatch, SCHEDULES[schedule], lambda: run(True)), want)

@@ -827,9 +827,13 @@ int vls_set_drift(vls_ctx *ctx, int run, const double *xr, const double *xu, con
       if (flag[i] == VLS_FOOT_OUT) xf[i] = -1.0;
       if (flag[i] == VLS_FOOT_CHAIN) xf[i] = -2.0, uf[i] = -1.0, lines++;
     }
+    hipStream_t s = ctx->c.stream;
+    // a captured step holds launches chosen by the flags (kick_streams, the
+    // slice step's pass over delay-line points without a line)
+    VLS_HIP_CHECK(hipStreamSynchronize(s));
+    drop_graph(ctx->c);
     r.hflag.assign(flag, flag + r.nVal);
     r.nChainFlags = lines;
-    hipStream_t s = ctx->c.stream;
     std::vector<double> ft(2 * r.nVal);
     for (int64_t i = 0; i < r.nVal; i++) ft[2 * i] = xf[i], ft[2 * i + 1] = uf[i];
     copy_in(ctx->c, r.feet, ft.data(), 2 * r.nVal * sizeof(double), s);
