@@ -1,6 +1,6 @@
-"""Foot tables changed between steps: every schedule, and the captured step of
-an ensemble, gives the bits of the kernels per phase.  No tolerance: the
-schedules run the same operations."""
+"""Foot tables and delay lines changed between steps: every schedule,
+and the captured step of an ensemble, gives the bits of the kernels per phase.
+No tolerance: the schedules run the same operations."""
 import ctypes as C
 
 import numpy as np
@@ -40,6 +40,20 @@ def _feet(shape, seed, chains=()):
 
 def _set_drift(ctx, run, xr, xu, flag):
     V._check(V.lib().vls_set_drift(ctx._h, run, _p(xr), _p(xu), _p(flag, C.c_uint8)))
+
+
+def _set_chains(ctx, run, points, shape, seed):
+    rng = np.random.default_rng(seed)
+    nJ, nU, nR = shape
+    n = len(points)
+    length = rng.integers(2, 6, n).astype(np.int32)
+    head = (rng.integers(0, 6, n) % length).astype(np.int32)
+    bxr, bxu = rng.uniform(0, nR - 1, n), rng.uniform(0, nU - 1, n)
+    out = np.zeros(n, np.uint8)
+    vals = rng.random(int(length.sum()))
+    V._check(V.lib().vls_set_chains(ctx._h, run, n, _p(np.asarray(points, np.int64), C.c_int64),
+                                    _p(length, C.c_int32), _p(head, C.c_int32), _p(bxr), _p(bxu),
+                                    _p(out, C.c_uint8), _p(vals)))
 
 
 def _points(shape, n, seed, taken=()):
@@ -84,3 +98,26 @@ def test_captured_step_follows_new_feet(monkeypatch, schedule):
 
     want = _under(monkeypatch, PHASES, lambda: run(False))
     _same(_under(monkeypatch, SCHEDULES[schedule], lambda: run(True)), want)
+
+
+@pytest.mark.parametrize("schedule", list(SCHEDULES))
+def test_moved_delay_line_points(monkeypatch, schedule):
+    """Lines attached to one set of points and a later foot table whose
+    delay-line points are others, as many as there are lines or fewer: the
+    points without a line keep their kicked value."""
+    print(f"case moved delay-line points, {schedule}", flush=True)
+
+    def run():
+        s = V.Solver(_cfg())
+        ctx, shape = s.context, s.shape
+        ctx.clear_chains()
+        lines = _points(shape, 60, 1)
+        _set_drift(ctx, 0, *_feet(shape, 2, lines))
+        _set_chains(ctx, 0, lines, shape, 3)
+        s.step(2)
+        _set_drift(ctx, 0, *_feet(shape, 4, _points(shape, 50, 5, lines)))
+        s.step(3)
+        return [s.f(), *ctx.get_chains()]
+
+    want = _under(monkeypatch, PHASES, run)
+    _same(_under(monkeypatch, SCHEDULES[schedule], run), want)

@@ -82,6 +82,15 @@ bool foot_in_domain(double xr, double xu, const vls::Run &r) {
   return a >= 0 && a <= r.nR - 1 && b >= 0 && b <= r.nU - 1;
 }
 
+// Points that the foot table puts on a delay line but that have none: the
+// two may be set in either order, so the lines' points need not be the flagged
+// ones, and as many lines as flags do not mean that every flag has its line.
+void count_loose(vls::Run &r) {
+  r.nLoose = r.nChainFlags;
+  if (r.nLoose == 0) return;
+  for (int64_t p : r.hch_point) r.nLoose -= r.hflag[p] == VLS_FOOT_CHAIN;
+}
+
 template <class T>
 void h2d(T *dst, const T *src, size_t n, hipStream_t s) {
   if (n) VLS_HIP_CHECK(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyHostToDevice, s));
@@ -834,6 +843,7 @@ int vls_set_drift(vls_ctx *ctx, int run, const double *xr, const double *xu, con
     drop_graph(ctx->c);
     r.hflag.assign(flag, flag + r.nVal);
     r.nChainFlags = lines;
+    count_loose(r);
     std::vector<double> ft(2 * r.nVal);
     for (int64_t i = 0; i < r.nVal; i++) ft[2 * i] = xf[i], ft[2 * i + 1] = uf[i];
     copy_in(ctx->c, r.feet, ft.data(), 2 * r.nVal * sizeof(double), s);
@@ -890,6 +900,7 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
     r.nChains = nChains;
     r.nCells = cells;
     r.hch_point.assign(point, point + nChains);
+    count_loose(r);
     r.hch_xr.assign(back_xr, back_xr + nChains);
     r.hch_xu.assign(back_xu, back_xu + nChains);
     r.hch_out.assign(back_out, back_out + nChains);

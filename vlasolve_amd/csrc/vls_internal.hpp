@@ -90,6 +90,7 @@ struct Run {
   double *feet = nullptr;  // [nVal][2]
   std::vector<uint8_t> hflag;  // host copy of the VLS_FOOT_* kinds
   int64_t nChainFlags = 0;     // points of kind VLS_FOOT_CHAIN
+  int64_t nLoose = 0;          // those that have no delay line
   // moment
   double *P = nullptr;      // [nJ][nR] per-slice partials
   double *dM = nullptr, *Mx = nullptr, *acc = nullptr, *mTot = nullptr;

@@ -2608,7 +2608,7 @@ static bool kick_tiles(const Run &r) {
 
 bool kick_streams(const Run &r) {
   // a point whose delay line was taken away keeps its kicked value in f
-  if (!r.kept || line_shape(r) || r.nChainFlags > r.nChains) return false;
+  if (!r.kept || line_shape(r) || r.nLoose > 0) return false;
   return r.kickMode >= 0 ? r.kickMode == 4 : kick_moment(r) && !getenv("VLS_KICK_RSOLVE");
 }
 

@@ -821,7 +821,7 @@ SliceArgs slice_args(Run &r) {
   a.cnt = r.sliceCnt;
   const int nG = (r.nU - 1 + 15) / 16, parts = slice_parts(r);
   a.maxLines = r.maxLines;
-  a.loose = r.nChainFlags > r.nChains;
+  a.loose = r.nLoose > 0;
   a.gPart = (nG + parts - 1) / parts;
   a.parts = (nG + a.gPart - 1) / a.gPart;
   return a;
