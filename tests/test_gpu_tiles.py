@@ -63,3 +63,20 @@ def test_line_tiles_recorded(monkeypatch, pr, pu, pj):
     for k, (a, b) in enumerate(zip(*seen)):
         assert np.array_equal(a, b), k
     assert np.abs(grads[0] - grads[1]).max() <= 1e-12 * np.abs(grads[1]).max()
+
+
+@pytest.mark.parametrize("pj", [1, 3])
+def test_row_adjoints_of_register_shapes(monkeypatch, pj):
+    """The rows of a register shape by tiles in LDS: the gradient has the bits
+    of the register kernels (VLS_TILE_R leaves the tiles out)."""
+    cfg = dict(UDF_C1, **{"grid.Pres": 128, "grid.Ures": [128, pj]})
+    print(f"case row adjoints of a register shape, 129 x 129 x {pj}", flush=True)
+    grads = []
+    for tile in (None, "63"):
+        if tile:
+            monkeypatch.setenv("VLS_TILE_R", tile)
+        s = V.Solver(cfg)
+        s.context.record(4, 2)
+        grads.append(s.context.adjoint(dL_df=np.cos(np.arange(s.f().size))))
+    for a, b in zip(*grads):
+        assert np.array_equal(a, b), np.abs(a - b).max()

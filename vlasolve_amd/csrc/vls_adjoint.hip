@@ -940,13 +940,13 @@ void launch_adj_spline(Run &r, double *cb, double *out, hipStream_t s) {
   if (a)
     hipLaunchKernelGGL(a->v, gv, dim3(64), 0, s, cb, r.cs, 0, r.tv);
   else if (adj_line_tile(r, false))
-    launch_adj_line_tile(r, false, cb, nullptr, s);
+    launch_adj_line_tile(r, false, false, cb, nullptr, s);
   else
     hipLaunchKernelGGL(k_adj_v, gv, dim3(64), 0, s, cb, r.nR + 2, r.cs, r.tv);
   // short rows are faster in registers (65x65x32: a reverse step 49 us, by
   // tiles 50.5; 129x129x64: rows 18, by tiles 14)
   if (!(a && r.nR <= 65) && adj_line_tile(r, true))
-    launch_adj_line_tile(r, true, cb, out, s);
+    launch_adj_line_tile(r, true, a != nullptr, cb, out, s);
   else if (a)
     hipLaunchKernelGGL(a->r, gr, dim3(64), 0, s, cb, out, r.nU, r.cs, 0, r.tr);
   else

@@ -251,9 +251,11 @@ void launch_slice_drift(Run &r, hipStream_t s, bool last);
 // acceleration of the last launch_moment; dKeep as above
 void launch_kick_tile(Run &r, hipStream_t s, double *dKeep);
 // the line adjoints of the drift's spline by tiles: rows of cb to out (f's
-// layout), or its columns in place
+// layout), or its columns in place; fused (rows): with the rounding of the
+// register line adjoints
 bool adj_line_tile(const Run &r, bool rows);
-void launch_adj_line_tile(const Run &r, bool rows, double *cb, double *out, hipStream_t s);
+void launch_adj_line_tile(const Run &r, bool rows, bool fused, double *cb, double *out,
+                          hipStream_t s);
 // tileR, tileV, tileK by the run's sizes
 void choose_line_tiles(Run &r);
 // the r-solves (rows; src in f's layout) or v-solves (src in c's layout, dst

@@ -927,8 +927,12 @@ __global__ void __launch_bounds__(128) k_line_tile(TileArgs a) {
 // vls_adjoint.hip: c1 -= A01 c0, c2 -= A02 c0, c[t] -= u[t-1] c[t-1] going up,
 // then the last row, the scaling by 1/d and the carry c16 c[k] going down) by
 // tiles of lines in LDS: the streaming kernels take the line through memory
-// twice each way.  Same operations, same order.  A block's first wave
-// sweeps (a chain of 1 and 3 dependent operations, a DS read and a write a row).
+// twice each way.  Same operations, same order: on grids without register
+// line adjoints those of the streaming sweeps (adj_down: the carry c16 c[k]
+// rounded, then subtracted), on the others those of the register kernels
+// (kFused, k_adj_rows: an fma of c16, after the last row's terms).  A block's
+// first wave sweeps (a chain of 1 dependent operation up and 3, fused 2, down,
+// a DS read and a write a row).
 struct AdjTileArgs {
   double *cb;   // padded coefficients' adjoints; columns: in place
   double *out;  // rows: f's layout
@@ -940,6 +944,7 @@ struct AdjTileArgs {
 
 // A line in LDS, in place: p[k st], k = 0..M-1.  Chunks of kQ rows, read a
 // chunk ahead.
+template <bool kFused>
 __device__ __forceinline__ void lds_line_adjoint(double *p, int st, const ThomasAxis &ax) {
   const int M = ax.M;
   constexpr int kQ = 8, kH = kHead + 2;  // rows 0 .. kHead + 1 take the pivots of the head
@@ -994,21 +999,34 @@ __device__ __forceinline__ void lds_line_adjoint(double *p, int st, const Thomas
     sp += st;
   }
   const double tt = prev * ax.rq;  // prev = c[M-1]
+  // element k from its value x of the ascending sweep; the carry is c[k + 1],
+  // or c16 times that.  last: the last row's coefficient in rows M-2 and M-3.
   double carry = 0.0;
-  auto down = [&](double v) {
-    v *= rdS;
+  auto down = [&](double x, double rd) {
+    double v = kFused ? fma(-ax.c16, carry, x) : x - carry;
+    v *= rd;
+    carry = kFused ? v : ax.c16 * v;
+    return v;
+  };
+  auto down_last = [&](double x, double last, double rd) {
+    if constexpr (kFused) return down(fma(-last, tt, x), rd);
+    double v = fma(-last, tt, x - carry);
+    v *= rd;
     carry = ax.c16 * v;
+    return v;
+  };
+  auto put = [&](double v) {
     *sp = v;
     sp -= st;
   };
   sp = p + (M - 2) * st;
   int k = M - 2;
   if (k > kHead) {
-    down(fma(-ax.p, tt, *sp - carry));
+    put(down_last(*sp, ax.p, rdS));
     k--;
   }
   if (k > kHead && k == M - 3) {
-    down(fma(-ax.hi2, tt, *sp - carry));
+    put(down_last(*sp, ax.hi2, rdS));
     k--;
   }
   if (k - kQ >= kHead) {
@@ -1022,27 +1040,22 @@ __device__ __forceinline__ void lds_line_adjoint(double *p, int st, const Thomas
 #pragma unroll
       for (int q = 0; q < kQ; q++) a[q] = sp[-(kQ + q) * st];
 #pragma unroll
-      for (int q = 0; q < kQ; q++) down(b[q] - carry);
+      for (int q = 0; q < kQ; q++) put(down(b[q], rdS));
     }
 #pragma unroll
-    for (int q = 0; q < kQ; q++) down(a[q] - carry);
+    for (int q = 0; q < kQ; q++) put(down(a[q], rdS));
     k -= kQ;
   }
-  for (; k > kHead; k--) down(*sp - carry);
+  for (; k > kHead; k--) put(down(*sp, rdS));
 #pragma unroll
   for (int m = kHead; m >= 1; m--) {
-    if (m <= M - 2) {
-      double v = h[m] - carry;
-      if (m == M - 2) v = fma(-ax.p, tt, v);
-      if (m == M - 3) v = fma(-ax.hi2, tt, v);
-      v *= kPivRd[m];
-      carry = ax.c16 * v;
-      p[m * st] = v;
-    }
+    if (m <= M - 2)
+      p[m * st] = m >= M - 3 ? down_last(h[m], m == M - 2 ? ax.p : ax.hi2, kPivRd[m])
+                             : down(h[m], kPivRd[m]);
   }
 }
 
-template <bool kRows>
+template <bool kRows, bool kFused>
 __global__ void __launch_bounds__(128) k_adj_line_tile(AdjTileArgs a) {
   extern __shared__ double D[];
   constexpr int kTL = 128, kB = 16;
@@ -1072,7 +1085,7 @@ __global__ void __launch_bounds__(128) k_adj_line_tile(AdjTileArgs a) {
     }
   }
   __syncthreads();
-  if (t < wid) lds_line_adjoint(kRows ? D + t * ps : D + t, kRows ? 1 : W, a.ax);
+  if (t < wid) lds_line_adjoint<kFused>(kRows ? D + t * ps : D + t, kRows ? 1 : W, a.ax);
   __syncthreads();
   if constexpr (kRows) {
     double *dst = a.out + ((size_t)j * nU + l0) * nR;
@@ -1120,8 +1133,9 @@ void configure_slice(int maxLdsPerBlock) {
   for (const void *fn : {(const void *)k_kick_tile<256>, (const void *)k_kick_tile<512>,
                          (const void *)k_slice_drift, (const void *)k_slice_moment,
                          (const void *)k_line_tile<true>, (const void *)k_line_tile<false>,
-                         (const void *)k_adj_line_tile<true>,
-                         (const void *)k_adj_line_tile<false>})
+                         (const void *)k_adj_line_tile<true, false>,
+                         (const void *)k_adj_line_tile<true, true>,
+                         (const void *)k_adj_line_tile<false, false>})
     VLS_HIP_CHECK(
         hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxLdsPerBlock));
   done.insert(device);
@@ -1296,7 +1310,8 @@ bool adj_line_tile(const Run &r, bool rows) {
   return w > 0 && (int64_t)(lines + w - 1) / w * r.nJ <= 4 * 256;
 }
 
-void launch_adj_line_tile(const Run &r, bool rows, double *cb, double *out, hipStream_t s) {
+void launch_adj_line_tile(const Run &r, bool rows, bool fused, double *cb, double *out,
+                          hipStream_t s) {
   AdjTileArgs a{};
   a.cb = cb;
   a.out = out;
@@ -1311,8 +1326,10 @@ void launch_adj_line_tile(const Run &r, bool rows, double *cb, double *out, hipS
   a.mulIn = magic(rows ? r.nR + 2 : a.W);
   a.mulOut = magic(rows ? r.nR : a.W);
   const size_t lds = (size_t)a.W * (rows ? a.pitch : r.nU + 2) * sizeof(double);
-  hipLaunchKernelGGL(rows ? k_adj_line_tile<true> : k_adj_line_tile<false>, dim3(a.nT * r.nJ),
-                     dim3(128), lds, s, a);
+  void (*fn)(AdjTileArgs) = k_adj_line_tile<false, false>;
+  if (rows) fn = k_adj_line_tile<true, false>;
+  if (rows && fused) fn = k_adj_line_tile<true, true>;
+  hipLaunchKernelGGL(fn, dim3(a.nT * r.nJ), dim3(128), lds, s, a);
 }
 
 void launch_kick_tile(Run &r, hipStream_t s, double *dKeep) {
