@@ -72,3 +72,27 @@ def test_slice_step_against_kernels_per_phase(monkeypatch):
         seen.append(got)
     for k, (a, b) in enumerate(zip(*seen)):
         assert np.array_equal(a, b), k
+
+
+@pytest.mark.parametrize("grid,by_slice", [
+    ((64, 64, 256), True), ((64, 64, 257), False), ((32, 32, 1024), False),
+    ((128, 32, 170), True), ((128, 32, 171), False), ((40, 35, 320), True), ((40, 35, 321), False),
+    ((139, 32, 213), True), ((139, 32, 214), False), ((299, 24, 102), True), ((299, 24, 103), False)])
+def test_slice_step_is_for_slices_that_fill_the_chip_once(grid, by_slice):
+    """The grids that go by slice, at both sides of the bounds on the slices
+    and on the kick's blocks (register lines and others)."""
+    pr, pu, pj = grid
+    print(f"case schedule of {pr + 1} x {pu + 1} x {pj}", flush=True)
+    s = V.Solver(dict(UDF_C1, **{"grid.Pres": pr, "grid.Ures": [pu, pj]}))
+    ctx = s.context
+    ctx.set_timing(True)
+    ctx.step(1)
+    names = {n for n, _ in ctx.kernel_times()}
+    assert ("slice_kick" in names) == by_slice, names
+
+
+@pytest.mark.parametrize("pr,pu,pj", [(12, 13, 300), (16, 16, 600)])
+def test_more_slices_than_cus_bit_exact(monkeypatch, pr, pu, pj):
+    monkeypatch.setenv("VLS_SLICE_STEP", "1")
+    _run(dict(UDF_C1, **{"grid.Pres": pr, "grid.Ures": [pu, pj]}),
+         f"slice step {pr + 1} x {pu + 1} x {pj}")

@@ -72,7 +72,7 @@ struct Run {
   // evaluation folded into the drift's r-solve / streaming / column tiles
   int lineMode = -1, kickMode = -1;
   // a step in two launches (vls_slice.hip), for the shapes that have sliceG: -1
-  // unless the environment forces one of the other schedules, 0 / 1 tuned
+  // from the shape (slice_pays) and the environment, 0 / 1 tuned
   int sliceMode = -1;
   vls_solver_params sp{};
   double start_v = 0, hinv_v = 0, Ulo = 0, Uhi = 0;
@@ -241,6 +241,8 @@ size_t slice_group_doubles(const Run &r);
 void configure_slice(int maxLdsPerBlock);
 bool slice_fits(const Run &r);    // the run's buffers are there and its delay lines fit too
 bool slice_on(const Run &r);
+// whether the run's lines have register kernels
+bool register_lines(const Run &r);
 // the moment partials P [nJ][nR] of f (the run's shape and species), a block
 // per slice; false if a slice's group sums don't fit in LDS
 bool launch_slice_partials(Run &r, const double *f, double *P, hipStream_t s);

@@ -2465,6 +2465,8 @@ static const LineShape *line_shape(const Run &r) {
   return &it->second;
 }
 
+bool register_lines(const Run &r) { return line_shape(r) != nullptr; }
+
 bool kick_rsolve_shape(const Run &r) {
   return r.nS == 1 && row_shape(r.nR) && col_shape(r.nU);
 }
