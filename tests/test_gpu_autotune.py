@@ -6,7 +6,7 @@ choices are cached per shape."""
 import numpy as np
 import pytest
 
-from tests.configs import HERNQUIST_SMALL, UDF_C1, UDF_ODD, UDF_TINY
+from tests.configs import HERNQUIST_SMALL, UDF_2SPECIES_DELAYED, UDF_C1, UDF_ODD, UDF_TINY
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +31,17 @@ def test_tuned_schedules_give_the_same_bits():
     # a second tuning of the same shapes comes from the cache
     again = V.Ensemble(CFGS[:1])
     assert "cached" in again.autotune()
+
+
+@pytest.mark.parametrize("pr,pu,pj", [(24, 20, 12), (64, 64, 6), (150, 131, 3)])
+def test_two_species(pr, pu, pj):
+    """Runs of two species, whose moment reads both planes of f: by slice,
+    register lines, and lines too long for either."""
+    cfg = dict(UDF_2SPECIES_DELAYED, **{"grid.Pres": pr, "grid.Ures": [pu, pj]})
+    print(f"case autotune of two species, {pr + 1} x {pu + 1} x {pj}", flush=True)
+    ref, s = V.Solver(cfg), V.Solver(cfg)
+    print("  " + s.context.autotune(), flush=True)
+    ref.step(3)
+    s.step(3)
+    assert np.array_equal(s.f(), ref.f())
+    assert all(np.array_equal(a, b) for a, b in zip(s.context.get_chains(), ref.context.get_chains()))

@@ -2831,20 +2831,24 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
     }
   }
   // the moment, the kick and the drift's r-solve (which the kick can be
-  // folded into), on a copy of f (the kick works in place)
+  // folded into), on a copy of f (the kick works in place), all its species:
+  // the moment reads every plane
   apply_sched(r, best);
   launch_moment(r, s);
   double *f0 = r.f, *tmp = nullptr;
   // as large as f's buffer, which the kick folded into the r-solve writes
-  const size_t fDoubles = r.fRows ? std::max<size_t>(r.nVal, (size_t)r.nJ * r.cs) : r.nVal;
+  const size_t values = (size_t)r.nVal * r.nS;
+  const size_t fDoubles = r.fRows ? std::max<size_t>(values, (size_t)r.nJ * r.cs) : values;
   VLS_HIP_CHECK(hipMalloc(&tmp, fDoubles * sizeof(double)));
+  auto copy_f = [&] {
+    VLS_HIP_CHECK(hipMemcpyAsync(tmp, f0, values * sizeof(double), hipMemcpyDeviceToDevice, s));
+  };
   r.f = tmp;
   const int64_t chains = r.nChains;
   try {
     auto time_kick = [&](int mode) {
       r.kickMode = mode;
-      VLS_HIP_CHECK(hipMemcpyAsync(tmp, f0, (size_t)r.nVal * sizeof(double),
-                                   hipMemcpyDeviceToDevice, s));
+      copy_f();
       return time_us(s, [&] {
         if (mode == 3) {
           launch_kick_rsolve(r, s, nullptr);
@@ -2900,10 +2904,6 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
       // whole steps on the copy of f, the delay lines left out of the drift
       r.nChains = 0;
       apply_sched(r, best);
-      auto copy_f = [&] {
-        VLS_HIP_CHECK(hipMemcpyAsync(tmp, f0, (size_t)r.nVal * sizeof(double),
-                                     hipMemcpyDeviceToDevice, s));
-      };
       copy_f();
       best.stepUs = time_us(s, [&] {
         if (r.sp.no_linking) {
