@@ -45,3 +45,22 @@ def test_two_species(pr, pu, pj):
     s.step(3)
     assert np.array_equal(s.f(), ref.f())
     assert all(np.array_equal(a, b) for a, b in zip(s.context.get_chains(), ref.context.get_chains()))
+
+
+def test_choices_are_kept_apart():
+    """A choice made for two species, without linking or for a run that has the
+    GPU for itself is not taken for the same grid under other conditions."""
+    grid = {"grid.Pres": 28, "grid.Ures": [26, 10]}
+    runs = [dict(UDF_2SPECIES_DELAYED, **grid), dict(UDF_C1, **grid),
+            dict(UDF_C1, **grid, **{"solver.noLinking": 1})]
+    print("case autotune of one grid under several conditions", flush=True)
+    for again in (False, True):
+        for cfg in runs:
+            desc = V.Solver(cfg).context.autotune()
+            print("  " + desc, flush=True)
+            assert ("cached" in desc) == again and " 0.0 us" not in desc
+    # runs that share the GPU go by slice where the sizes say so, whatever one
+    # of them alone was timed at
+    desc = V.Ensemble(runs[1:2] * 3).autotune()
+    print("  " + desc, flush=True)
+    assert desc.count("slice step (by its sizes") == 3

@@ -240,6 +240,7 @@ bool slice_shared(const Run &r);  // several blocks take a slice
 size_t slice_group_doubles(const Run &r);
 void configure_slice(int maxLdsPerBlock);
 bool slice_fits(const Run &r);    // the run's buffers are there and its delay lines fit too
+bool slice_pays(const Run &r);    // and the sizes are those it is faster for
 bool slice_on(const Run &r);
 // whether the run's lines have register kernels
 bool register_lines(const Run &r);

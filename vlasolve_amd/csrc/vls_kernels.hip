@@ -2696,9 +2696,13 @@ struct Sched {
   double splineUs, kickUs;
   bool slice = false;              // a step in two launches
   double stepUs = 0, sliceUs = 0;  // a step of the kernels per phase, and of the slice step
+                                   // (0: not timed)
 };
+// What a choice depends on: the grid, the LDS, the species, the linking and
+// whether the streaming kick is open to the run.
+using TuneKey = std::tuple<int, int, int, int, int, bool, bool>;
 std::mutex g_tuneMu;
-std::map<std::tuple<int, int, int, int>, Sched> g_tuned;
+std::map<TuneKey, Sched> g_tuned;
 
 void apply_sched(Run &r, const Sched &c) {
   r.lineMode = c.lineMode;
@@ -2737,8 +2741,13 @@ std::string describe(const Run &r, const Sched &c, bool cached) {
   char buf[256];
   std::string sp;
   if (c.slice) {
-    snprintf(buf, sizeof buf, "%dx%dx%d: slice step (%.1f us a step, kernels per phase %.1f us%s)",
-             r.nR, r.nU, r.nJ, c.sliceUs, c.stepUs, cached ? ", cached" : "");
+    if (c.sliceUs > 0)
+      snprintf(buf, sizeof buf,
+               "%dx%dx%d: slice step (%.1f us a step, kernels per phase %.1f us%s)", r.nR, r.nU,
+               r.nJ, c.sliceUs, c.stepUs, cached ? ", cached" : "");
+    else
+      snprintf(buf, sizeof buf, "%dx%dx%d: slice step (by its sizes, not timed%s)", r.nR, r.nU,
+               r.nJ, cached ? ", cached" : "");
     return buf;
   }
   if (c.lineMode == 1) {
@@ -2762,13 +2771,26 @@ std::string describe(const Run &r, const Sched &c, bool cached) {
 }  // namespace
 
 std::string autotune(Run &r, hipStream_t s, int maxLds) {
-  const auto key = std::make_tuple(r.nR, r.nU, r.nJ, maxLds);
+  const TuneKey key{r.nR, r.nU, r.nJ, maxLds, r.nS, r.sp.no_linking != 0, r.kept && r.nLoose == 0};
+  // Whether to step by slice is timed for one species and a run that has the
+  // GPU for itself; otherwise the sizes say (slice_pays).  The copy of f below
+  // has no delay lines of several species to step with, and a run that shares
+  // the GPU has its blocks laid out for its share: alone on an idle GPU the
+  // slice step looks slower than it is (32 runs of 65 to 257 points: 1270 us
+  // a step by the sizes, 1310 by such times).
+  const bool timeSlice = r.nS == 1 && r.cus == 256 && slice_fits(r);
+  auto slice_by_size = [&](Sched &c) {
+    c.slice = slice_fits(r) && slice_pays(r);
+    c.stepUs = c.sliceUs = 0;
+  };
   {
     std::lock_guard<std::mutex> lock(g_tuneMu);
     auto it = g_tuned.find(key);
     if (it != g_tuned.end()) {
-      apply_sched(r, it->second);
-      return describe(r, it->second, true);
+      Sched c = it->second;
+      if (!timeSlice || c.sliceUs == 0) slice_by_size(c);
+      apply_sched(r, c);
+      return describe(r, c, true);
     }
   }
   // the drift's spline: register lines where the shape has them, else the
@@ -2898,9 +2920,9 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
         best.kickUs = us;
       }
     }
-    if (slice_fits(r) && r.nS > 1) {
-      best.slice = true;
-    } else if (slice_fits(r)) {
+    if (!timeSlice) {
+      slice_by_size(best);
+    } else {
       // whole steps on the copy of f, the delay lines left out of the drift
       r.nChains = 0;
       apply_sched(r, best);

@@ -1160,7 +1160,7 @@ bool slice_fits(const Run &r) {
 //     300x49x100, 500, 69, 80 but x128, 640, 94, 88; 257x57x256 149, 123);
 //     with a second drift or species past 768 (129x129x256, 768, without
 //     linking 146, 159, two species 184, 205; 97x97x300, two species, 182, 159).
-static bool slice_pays(const Run &r) {
+bool slice_pays(const Run &r) {
   const int W = kick_width(r), nT = (r.nR + W - 1) / W;
   const bool lines = register_lines(r), twice = r.nS > 1 || r.sp.no_linking;
   if (r.nJ > (nT == 1 && !lines ? 320 : 256)) return false;
