@@ -1,6 +1,7 @@
-"""Foot tables and delay lines changed between steps: every schedule,
-and the captured step of an ensemble, gives the bits of the kernels per phase.
-No tolerance: the schedules run the same operations."""
+"""Foot tables and delay lines changed between steps, and feet and back cells
+at the edges of the domain that vls_set_drift and vls_set_chains accept: every
+schedule, and the captured step of an ensemble, gives the bits of the kernels
+per phase.  No tolerance: the schedules run the same operations."""
 import ctypes as C
 
 import numpy as np
@@ -42,13 +43,15 @@ def _set_drift(ctx, run, xr, xu, flag):
     V._check(V.lib().vls_set_drift(ctx._h, run, _p(xr), _p(xu), _p(flag, C.c_uint8)))
 
 
-def _set_chains(ctx, run, points, shape, seed):
+def _set_chains(ctx, run, points, shape, seed, back=None):
     rng = np.random.default_rng(seed)
     nJ, nU, nR = shape
     n = len(points)
     length = rng.integers(2, 6, n).astype(np.int32)
     head = (rng.integers(0, 6, n) % length).astype(np.int32)
     bxr, bxu = rng.uniform(0, nR - 1, n), rng.uniform(0, nU - 1, n)
+    if back is not None:
+        bxr[:], bxu[:] = back
     out = np.zeros(n, np.uint8)
     vals = rng.random(int(length.sum()))
     V._check(V.lib().vls_set_chains(ctx._h, run, n, _p(np.asarray(points, np.int64), C.c_int64),
@@ -121,3 +124,20 @@ def test_moved_delay_line_points(monkeypatch, schedule):
 
     want = _under(monkeypatch, PHASES, run)
     _same(_under(monkeypatch, SCHEDULES[schedule], run), want)
+
+
+def test_back_cell_below_the_first_knot(monkeypatch):
+    """A back cell inside (-1, 0): its integer part is 0, so it is evaluated."""
+    print("case back cell below the first knot", flush=True)
+
+    def run():
+        s = V.Solver(_cfg())
+        ctx, shape = s.context, s.shape
+        lines = _points(shape, 40, 1)
+        _set_drift(ctx, 0, *_feet(shape, 2, lines))
+        ctx.clear_chains()
+        _set_chains(ctx, 0, lines, shape, 3, back=(-0.375, 3.25))
+        s.step(7)
+        return [s.f(), *ctx.get_chains()]
+
+    _same(_under(monkeypatch, {}, run), _under(monkeypatch, PHASES, run))

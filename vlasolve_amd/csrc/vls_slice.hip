@@ -601,7 +601,7 @@ static_assert(40 * kT * sizeof(double) >= 163840, "a slice that fits in LDS fits
 
 // A delay line of the slice while its block waits for the solves.
 struct LineRec {
-  double bxr, bxu, front;  // back foot (bxr < 0: outside), value at the front
+  double bxr, bxu, front;  // back foot (kFootOut: outside), value at the front
   int64_t back;            // index of the slot behind the front in vals
   int il;                  // point in the slice (-1: of another block's rows)
   int pad;
@@ -683,7 +683,7 @@ __global__ void __launch_bounds__(kT) k_slice_drift(SliceArgs a) {
             if (h < 0) h += len;
             const int64_t off = a.ch.off[k];
             LineRec l;
-            l.bxr = a.ch.bout[k] ? -1.0 : a.ch.bxr[k];
+            l.bxr = a.ch.bout[k] ? kFootOut : a.ch.bxr[k];
             l.bxu = a.ch.bxu[k];
             l.front = vals[off + h];
             l.back = off + (h == 0 ? len - 1 : h - 1);
@@ -705,7 +705,7 @@ __global__ void __launch_bounds__(kT) k_slice_drift(SliceArgs a) {
       if (l.il >= uB * nR) {
         halo[l.il - uB * nR] = l.front;
       } else {
-        vals[l.back] = l.bxr < 0.0 ? 0.0 : eval_c(C, ps, l.bxr, l.bxu);
+        vals[l.back] = l.bxr > kFootOut ? eval_c(C, ps, l.bxr, l.bxu) : 0.0;
         fj[l.il] = l.front;
       }
     }
