@@ -141,3 +141,31 @@ def test_back_cell_below_the_first_knot(monkeypatch):
         return [s.f(), *ctx.get_chains()]
 
     _same(_under(monkeypatch, {}, run), _under(monkeypatch, PHASES, run))
+
+
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("where", ["feet", "back cells"])
+def test_past_the_last_knot(monkeypatch, axis, where):
+    """Feet and back cells between the last knot and the next integer: their
+    stencil ends in the first column of the next row, or the first row of the
+    next slice."""
+    print(f"case past the last knot, axis {axis}, {where}", flush=True)
+
+    def run():
+        s = V.Solver(_cfg(39, 34, 9))  # rows of 42 coefficients, an odd pitch in LDS
+        ctx, shape = s.context, s.shape
+        lines = _points(shape, 40, 1)
+        feet = _feet(shape, 2, lines)
+        last = (shape[2] - 1, shape[1] - 1)
+        back = [5.5, 6.5]
+        if where == "feet":
+            feet[axis][::7] = last[axis] + 0.375
+        else:
+            back[axis] = last[axis] + 0.375
+        ctx.clear_chains()
+        _set_drift(ctx, 0, *feet)
+        _set_chains(ctx, 0, lines, shape, 3, back=back)
+        s.step(7)
+        return [s.f(), *ctx.get_chains()]
+
+    _same(_under(monkeypatch, {}, run), _under(monkeypatch, PHASES, run))

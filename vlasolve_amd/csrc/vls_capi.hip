@@ -81,6 +81,11 @@ bool foot_in_domain(double xr, double xu, const vls::Run &r) {
   double a = std::trunc(xr), b = std::trunc(xu);
   return a >= 0 && a <= r.nR - 1 && b >= 0 && b <= r.nU - 1;
 }
+// ... and is past the last knot of an axis, by more than the rounding of a
+// coordinate on it (the coefficients beyond then weigh 1e-27 at most)
+bool past_last_knot(double xr, double xu, const vls::Run &r) {
+  return xr > r.nR - 1 + 1e-9 || xu > r.nU - 1 + 1e-9;
+}
 
 // Points that the foot table puts on a delay line but that have none: the
 // two may be set in either order, so the lines' points need not be the flagged
@@ -821,12 +826,14 @@ int vls_set_drift(vls_ctx *ctx, int run, const double *xr, const double *xu, con
     vls::Run &r = run_of(ctx, run);
     if (!xr || !xu || !flag) throw vls::Error(VLS_ERR_ARG, "null foot table");
     // every evaluated foot must index inside the padded coefficient array
+    bool past = false;
     for (int64_t i = 0; i < r.nVal; i++) {
       if (flag[i] > VLS_FOOT_CHAIN) throw vls::Error(VLS_ERR_ARG, "invalid foot flag");
       if (flag[i] != VLS_FOOT_EVAL) continue;
       if (!foot_in_domain(xr[i], xu[i], r))
         throw vls::Error(VLS_ERR_ARG, "vls_set_drift: foot outside the spline domain at point " +
                                           std::to_string(i));
+      past = past || past_last_knot(xr[i], xu[i], r);
     }
     // the drift kernel reads the point's kind from xr (-1 outside, -2 delay
     // line) and a delay-line point's chain index from xu (-1: none yet)
@@ -843,6 +850,7 @@ int vls_set_drift(vls_ctx *ctx, int run, const double *xr, const double *xu, con
     drop_graph(ctx->c);
     r.hflag.assign(flag, flag + r.nVal);
     r.nChainFlags = lines;
+    r.feetPast = past;
     count_loose(r);
     std::vector<double> ft(2 * r.nVal);
     for (int64_t i = 0; i < r.nVal; i++) ft[2 * i] = xf[i], ft[2 * i + 1] = uf[i];
@@ -869,6 +877,7 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
     std::vector<int64_t> off(nChains);
     std::vector<uint8_t> seen(nChains ? r.nVal : 0, 0);
     int64_t cells = 0;
+    bool past = false;
     for (int64_t k = 0; k < nChains; k++) {
       if (len[k] < 2) throw vls::Error(VLS_ERR_ARG, "chain shorter than 2 cells");
       if (head[k] < 0 || head[k] >= len[k]) throw vls::Error(VLS_ERR_ARG, "chain head out of range");
@@ -878,6 +887,7 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
       if (seen[point[k]]++) throw vls::Error(VLS_ERR_ARG, "two chains attached to one point");
       if (!back_out[k] && !foot_in_domain(back_xr[k], back_xu[k], r))
         throw vls::Error(VLS_ERR_ARG, "chain back cell outside the spline domain");
+      past = past || (!back_out[k] && past_last_knot(back_xr[k], back_xu[k], r));
       off[k] = cells;
       cells += len[k];
     }
@@ -899,6 +909,7 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
     r.adj.tilesValid = false;  // the transposed foot table lists the back cells
     r.nChains = nChains;
     r.nCells = cells;
+    r.backPast = past;
     r.hch_point.assign(point, point + nChains);
     count_loose(r);
     r.hch_xr.assign(back_xr, back_xr + nChains);

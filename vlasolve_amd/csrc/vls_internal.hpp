@@ -89,6 +89,10 @@ struct Run {
   // (xr <= -1 marks points outside the grid or on delay lines)
   double *feet = nullptr;  // [nVal][2]
   std::vector<uint8_t> hflag;  // host copy of the VLS_FOOT_* kinds
+  // feet, back cells between the last knot and the next integer: accepted, and
+  // their stencils reach the next row's or slice's coefficients, which c has in
+  // place and the slices in LDS do not
+  bool feetPast = false, backPast = false;
   int64_t nChainFlags = 0;     // points of kind VLS_FOOT_CHAIN
   int64_t nLoose = 0;          // those that have no delay line
   // moment
@@ -239,7 +243,9 @@ bool slice_pivots(const ThomasAxis &ax, const double *u, const double *rd, const
 bool slice_shared(const Run &r);  // several blocks take a slice
 size_t slice_group_doubles(const Run &r);
 void configure_slice(int maxLdsPerBlock);
-bool slice_fits(const Run &r);    // the run's buffers are there and its delay lines fit too
+// whether the run's buffers are there, its delay lines fit too and its stencils
+// stay in their slice
+bool slice_fits(const Run &r);
 bool slice_pays(const Run &r);    // and the sizes are those it is faster for
 bool slice_on(const Run &r);
 // whether the run's lines have register kernels

@@ -1142,7 +1142,8 @@ void configure_slice(int maxLdsPerBlock) {
 }
 
 bool slice_fits(const Run &r) {
-  return r.sliceG && slice_lds(r.nR, r.nU, r.maxLines) <= (size_t)kMaxLds;
+  return r.sliceG && !r.feetPast && !r.backPast &&
+         slice_lds(r.nR, r.nU, r.maxLines) <= (size_t)kMaxLds;
 }
 
 // Whether a run's steps go by slice unless it is told otherwise.  Every block
