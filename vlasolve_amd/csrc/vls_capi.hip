@@ -101,23 +101,22 @@ void h2d(T *dst, const T *src, size_t n, hipStream_t s) {
   if (n) VLS_HIP_CHECK(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyHostToDevice, s));
 }
 
-// Large transfers between the device and a caller's pageable memory.  The
-// runtime moves those through its own staging one after another with a single
-// host thread: 17 GB/s, and 4 to 9 into memory that has not been touched yet
-// (a new array's page faults).  Here up to kCopyThreads threads each take a
-// part, a piece at a time through two pinned pieces of their own, so that the
-// device's copies, the host's copies and the faults overlap: 201x201x200 from
-// 105 to 101 ms per 500 steps with a download, 513x513x256 from 318 to 284 per
-// 100, a 25-step gradient at 201x201x200 (an upload, a download) from 24.1 to
-// 19.8.  The pinned
-// memory (16 MiB) is shared by the process's contexts: made by the first large
-// download or upload of 64 MiB (making it takes 4 ms: the uploads of a
-// smaller context's set-up are faster without), held by one transfer at a time (others take the runtime's path
-// meanwhile) and given back with the last context.
+// Large downloads into a caller's pageable memory.  The runtime moves those
+// through its own staging one after another with a single host thread: 17.5
+// GB/s, and 10.5 into memory that has not been touched yet (a new array's page
+// faults).  Here up to kThreads threads each take a part, a piece at a time
+// through two pinned pieces of their own, so that the device's copies, the
+// host's copies and the faults overlap: 19 to 31 GB/s from 2 to 257 MiB, new
+// memory or not.  Page-locked memory goes by DMA in one copy (57 GB/s; by
+// pieces 30), and so do uploads from pageable memory, for which the runtime
+// locks the caller's pages (24 to 37 GB/s from 2 to 34 MiB where pieces reached
+// 20 to 27, and 30 either way from 62 MiB on).  The pinned memory (16 MiB) is
+// shared by the process's contexts: made by the first large download, held by
+// one transfer at a time (others take the runtime's path meanwhile) and given
+// back with the last context.
 struct Staging {
   static constexpr int kThreads = 8;
   static constexpr size_t kPiece = (size_t)1 << 20, kMin = (size_t)2 << 20;
-  static constexpr size_t kMakeIn = (size_t)64 << 20;
   std::mutex use;      // one transfer at a time
   std::mutex mu;       // guards the two below
   char *pin = nullptr;
@@ -135,10 +134,10 @@ struct Staging {
       pin = nullptr;
     }
   }
-  // with `use` held; make: if there is none yet
-  char *memory(bool make) {
+  // with `use` held
+  char *memory() {
     std::lock_guard<std::mutex> l(mu);
-    if (!pin && make && hipHostMalloc((void **)&pin, kThreads * 2 * kPiece, hipHostMallocPortable) !=
+    if (!pin && hipHostMalloc((void **)&pin, kThreads * 2 * kPiece, hipHostMallocPortable) !=
                     hipSuccess) {
       (void)hipGetLastError();  // no pinned memory: the runtime's path
       pin = nullptr;
@@ -146,14 +145,23 @@ struct Staging {
     return pin;
   }
 
-  // bytes between dev and host on stream s, complete on return
-  void copy(void *dev, void *host, size_t bytes, bool out, int device, hipStream_t s) {
-    std::unique_lock<std::mutex> u(use, std::try_to_lock);
-    char *p = bytes >= kMin && u.owns_lock() ? memory(out || bytes >= kMakeIn) : nullptr;
+  // memory that the runtime knows: page-locked, managed or a device's
+  static bool known(const void *host) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, host) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+  }
+
+  // bytes of dev to host on stream s, complete on return
+  void copy(const void *dev, void *host, size_t bytes, int device, hipStream_t s) {
+    std::unique_lock<std::mutex> u(use, std::defer_lock);
+    char *p = bytes >= kMin && !known(host) && u.try_lock() ? memory() : nullptr;
     if (!p) {
       if (u.owns_lock()) u.unlock();
-      VLS_HIP_CHECK(out ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s)
-                        : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s));
+      VLS_HIP_CHECK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
       VLS_HIP_CHECK(hipStreamSynchronize(s));
       return;
     }
@@ -168,41 +176,22 @@ struct Staging {
       if (e == hipSuccess && before != device) e = hipSetDevice(device);
       for (int k = 0; k < 2 && e == hipSuccess; k++)
         e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
-      auto at = [&](size_t k) { return (char *)host + k * kPiece; };
       auto len = [&](size_t k) { return std::min(kPiece, bytes - k * kPiece); };
       auto buf = [&](size_t k) { return p + ((size_t)t * 2 + (k & 1)) * kPiece; };
       auto send = [&](size_t k) {
-        char *d = (char *)dev + k * kPiece;
-        e = out ? hipMemcpyAsync(buf(k), d, len(k), hipMemcpyDeviceToHost, s)
-                : hipMemcpyAsync(d, buf(k), len(k), hipMemcpyHostToDevice, s);
+        e = hipMemcpyAsync(buf(k), (const char *)dev + k * kPiece, len(k), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipEventRecord(ev[k & 1], s);
       };
-      size_t sent = from;  // pieces given to the device
-      if (out)
-        for (; sent < to && sent < from + 2 && e == hipSuccess; sent++) send(sent);
+      size_t sent = from;  // pieces asked of the device
+      for (; sent < to && sent < from + 2 && e == hipSuccess; sent++) send(sent);
       for (size_t k = from; k < to && e == hipSuccess; k++) {
-        if (out) {
-          e = hipEventSynchronize(ev[k & 1]);
-          if (e != hipSuccess) break;
-          std::memcpy(at(k), buf(k), len(k));
-          if (sent < to) send(sent++);
-        } else {
-          if (k >= from + 2) e = hipEventSynchronize(ev[k & 1]);
-          if (e != hipSuccess) break;
-          std::memcpy(buf(k), at(k), len(k));
-          send(k);
-          sent++;
-        }
+        e = hipEventSynchronize(ev[k & 1]);
+        if (e != hipSuccess) break;
+        std::memcpy((char *)host + k * kPiece, buf(k), len(k));
+        if (sent < to) send(sent++);
       }
-      // the pinned pieces are free again only when the device is done with them
       for (int k = 0; k < 2; k++)
-        if (ev[k]) {
-          if (sent > from) {
-            const hipError_t w = hipEventSynchronize(ev[k]);
-            if (e == hipSuccess) e = w;
-          }
-          (void)hipEventDestroy(ev[k]);
-        }
+        if (ev[k]) (void)hipEventDestroy(ev[k]);
       if (before != device) (void)hipSetDevice(before);
       err[t] = e;
     };
@@ -218,18 +207,23 @@ struct Staging {
     }
     for (int t = 0; t <= nt - own; t++) work(t);
     for (auto &x : th) x.join();
+    // after an error too: the pinned pieces are free again only when the device
+    // is done with them
+    const hipError_t end = hipStreamSynchronize(s);
     for (hipError_t e : err) VLS_HIP_CHECK(e);
-    VLS_HIP_CHECK(hipStreamSynchronize(s));
+    VLS_HIP_CHECK(end);
   }
 };
 Staging g_staging;
 
 // complete on return
-void copy_in(vls::Context &C, void *dev, const void *host, size_t bytes, hipStream_t s) {
-  if (bytes) g_staging.copy(dev, const_cast<void *>(host), bytes, false, C.device, s);
+void copy_in(void *dev, const void *host, size_t bytes, hipStream_t s) {
+  if (!bytes) return;
+  VLS_HIP_CHECK(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s));
+  VLS_HIP_CHECK(hipStreamSynchronize(s));
 }
 void copy_out(vls::Context &C, void *host, const void *dev, size_t bytes, hipStream_t s) {
-  if (bytes) g_staging.copy(const_cast<void *>(dev), host, bytes, true, C.device, s);
+  if (bytes) g_staging.copy(dev, host, bytes, C.device, s);
 }
 
 template <class T>
@@ -799,9 +793,9 @@ int vls_upload_f(vls_ctx *ctx, int run, const double *f) {
     if (!f) throw vls::Error(VLS_ERR_ARG, "null f");
     if (r.nS > 1) {
       std::vector<double> planes = to_planes(f, r.nVal, r.nS);
-      copy_in(ctx->c, r.f, planes.data(), planes.size() * sizeof(double), ctx->c.stream);
+      copy_in(r.f, planes.data(), planes.size() * sizeof(double), ctx->c.stream);
     } else {
-      copy_in(ctx->c, r.f, f, r.nVal * sizeof(double), ctx->c.stream);
+      copy_in(r.f, f, r.nVal * sizeof(double), ctx->c.stream);
     }
     r.have_f = true;
   });
@@ -854,7 +848,7 @@ int vls_set_drift(vls_ctx *ctx, int run, const double *xr, const double *xu, con
     count_loose(r);
     std::vector<double> ft(2 * r.nVal);
     for (int64_t i = 0; i < r.nVal; i++) ft[2 * i] = xf[i], ft[2 * i + 1] = uf[i];
-    copy_in(ctx->c, r.feet, ft.data(), 2 * r.nVal * sizeof(double), s);
+    copy_in(r.feet, ft.data(), 2 * r.nVal * sizeof(double), s);
     r.hxr.swap(xf);
     r.hxu.swap(uf);
     r.adj.tilesValid = false;  // the adjoint's transposed foot table follows the feet
@@ -954,7 +948,7 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
       // clear the marks of any earlier delay lines, then attach these
       std::vector<double> ft(2 * r.nVal);
       for (int64_t i = 0; i < r.nVal; i++) ft[2 * i] = r.hxr[i], ft[2 * i + 1] = r.hxu[i];
-      copy_in(ctx->c, r.feet, ft.data(), 2 * r.nVal * sizeof(double), s);
+      copy_in(r.feet, ft.data(), 2 * r.nVal * sizeof(double), s);
       vls::mark_chains(r, s);
       VLS_HIP_CHECK(hipStreamSynchronize(s));
     }
@@ -1378,11 +1372,10 @@ void adjoint_check(const vls::Run &r) {
 }
 
 // lambda_N: the loss's derivative in f_N, directly and through M(<r).
-void adjoint_seed(vls::Context &C, vls::Run &r, hipStream_t s, const double *dL_dM,
-                  const double *dL_df) {
+void adjoint_seed(vls::Run &r, hipStream_t s, const double *dL_dM, const double *dL_df) {
   auto &A = r.adj;
   if (dL_df)
-    copy_in(C, A.fb, dL_df, r.nVal * sizeof(double), s);
+    h2d(A.fb, dL_df, r.nVal, s);
   else
     vls::launch_fill(A.fb, (int64_t)r.nVal, 0.0, s);
   if (dL_dM) {
@@ -1483,7 +1476,7 @@ int vls_adjoint(vls_ctx *ctx, int run, const double *dL_dM, const double *dL_df,
     adjoint_check(r);
     if (!grad_f0) throw vls::Error(VLS_ERR_ARG, "null gradient output");
     hipStream_t s = ctx->c.stream;
-    adjoint_seed(ctx->c, r, s, dL_dM, dL_df);
+    adjoint_seed(r, s, dL_dM, dL_df);
     for (int sg = r.adj.nCk - 1; sg >= 0; sg--) adjoint_segment(r, s, sg);
     VLS_HIP_CHECK(hipGetLastError());
     adjoint_end(ctx->c, r, s, grad_f0, grad_vals0);
@@ -1539,7 +1532,7 @@ int vls_adjoint_batch(vls_ctx *ctx, const double *const *dL_dM, const double *co
     }
     fork_runs(C);
     for (int k = 0; k < nRuns; k++)
-      adjoint_seed(C, C.runs[k], C.runStreams[k], dL_dM ? dL_dM[k] : nullptr,
+      adjoint_seed(C.runs[k], C.runStreams[k], dL_dM ? dL_dM[k] : nullptr,
                    dL_df ? dL_df[k] : nullptr);
     for (int sg = nCk - 1; sg >= 0; sg--)
       for (int k = 0; k < nRuns; k++) adjoint_segment(C.runs[k], C.runStreams[k], sg);
