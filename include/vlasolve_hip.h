@@ -185,6 +185,17 @@ int vls_device_info(char *buf, int len);
 int vls_copy_probe(size_t bytes);
 int vls_check_division(const double *b, int nb, int64_t samples, uint64_t seed,
                        int64_t *mismatches);
+/* Host check of the division by a pivot in two operations, fma(a, rh, RN(a rl))
+ * with rh = RN(1/d), rl = RN(1/d - rh).  For each of the nd divisors d:
+ * proven[i] says whether the set-up takes it for correctly rounded for every
+ * numerator (with rl moved by rlUlps units in its last place, which it refuses
+ * unless 0), and mismatches[i] counts the numerators whose quotient differs
+ * from a / d, among `samples` random ones with exponents in [-900, 900] and
+ * the significands nearest to a rounding tie.  Below about 2^-968 (1e-292) the
+ * product a rl is subnormal and the quotient may be one ulp off, as with the
+ * known-divisor division there. */
+int vls_check_pivot_division(const double *d, int nd, int rlUlps, int64_t samples, uint64_t seed,
+                             int *proven, int64_t *mismatches);
 
 /* Sizes of one run: {nR, nU, nJ, number of delay lines, delay-line cells,
  * species}. */

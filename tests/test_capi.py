@@ -123,3 +123,38 @@ def test_two_operation_pivot_division_is_correctly_rounded():
             a = float(A)
             assert float(F(a) * F(rh) + F(a * rl)) == a / d, (d, A)
     assert len(pivots) >= 16 and solved >= 2
+
+
+def test_pivot_division_host_check():
+    """The compiled division by a pivot and the condition that the set-up puts to
+    every pivot: the pivots are proven and divide as IEEE over random numerators
+    and those nearest to a rounding tie; a remainder that is not the rounded one
+    is refused; so are divisors that do divide wrongly."""
+    L = V.lib()
+    P = C.POINTER
+    L.vls_check_pivot_division.argtypes = [P(C.c_double), C.c_int, C.c_int, C.c_int64, C.c_uint64,
+                                           P(C.c_int), P(C.c_int64)]
+
+    def check(divisors, ulps=0, samples=20000):
+        d = np.array(divisors, np.float64)
+        proven, bad = np.full(len(d), -1, np.int32), np.full(len(d), -1, np.int64)
+        assert L.vls_check_pivot_division(d.ctypes.data_as(P(C.c_double)), len(d), ulps, samples, 5,
+                                          proven.ctypes.data_as(P(C.c_int)),
+                                          bad.ctypes.data_as(P(C.c_int64))) == 0
+        return proven, bad
+
+    pivots = sorted({float(x) for x in thomas(513, 60.0)[1][1:514]})
+    assert len(pivots) >= 16
+    proven, bad = check(pivots)
+    assert np.all(proven == 1) and np.all(bad == 0)
+    for ulps in (-1, 1, 1000):
+        assert not np.any(check(pivots, ulps, 0)[0])
+    # divisors in [1, 2): none that is proven divides wrongly, and some that are
+    # not proven do
+    d = np.random.default_rng(1).uniform(1.0, 2.0, 20000)
+    proven, bad = check(d, samples=20)
+    assert np.all(bad[proven == 1] == 0)
+    assert np.count_nonzero(bad) > 50 and 0.95 < proven.mean() < 1.0
+    for odd in (0.0, 5e-324, np.inf, np.nan):
+        assert L.vls_check_pivot_division((C.c_double * 1)(odd), 1, 0, 0, 1, (C.c_int * 1)(),
+                                          (C.c_int64 * 1)()) == 1

@@ -26,7 +26,8 @@ EXPORTS = (
     "vls_moments", "vls_stats", "vls_download_coef", "vls_set_timing", "vls_kernel_times",
     "vlsd_create", "vlsd_destroy", "vlsd_info", "vlsd_step", "vlsd_get_f", "vlsd_stats",
     "vlsd_moments", "vlsd_run", "vlsd_write_restart", "vlsd_snapshot", "vlsd_context",
-    "vlsd_last_error", "vls_thomas_table", "vls_check_division", "vls_device_info",
+    "vlsd_last_error", "vls_thomas_table", "vls_check_division",
+    "vls_check_pivot_division", "vls_device_info",
     "vls_copy_probe", "vlsd_host_create", "vlsd_host_destroy", "vlsd_host_info", "vlsd_host_f",
     "vlsd_host_feet", "vlsd_host_chains", "vls_run_info", "vls_put_chains", "vls_mass_profile",
     "vls_record", "vls_adjoint", "vls_set_graph", "vlsd_ensemble_create", "vlsd_ensemble_destroy",

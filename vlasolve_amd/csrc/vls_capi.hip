@@ -636,6 +636,43 @@ int vls_check_division(const double *b, int nb, int64_t samples, uint64_t seed,
   return VLS_OK;
 }
 
+int vls_check_pivot_division(const double *d, int nd, int rlUlps, int64_t samples, uint64_t seed,
+                             int *proven, int64_t *mismatches) {
+  if (!d || nd < 0 || samples < 0 || !proven || !mismatches) return fail(VLS_ERR_ARG, "bad arguments");
+  uint64_t x = seed ? seed : 0x9E3779B97F4A7C15ull;
+  auto next = [&]() {
+    x ^= x << 13;
+    x ^= x >> 7;
+    x ^= x << 17;
+    return x;
+  };
+  for (int i = 0; i < nd; i++) {
+    if (!std::isnormal(d[i])) return fail(VLS_ERR_ARG, "divisor is zero, subnormal or not finite");
+    const double rh = 1.0 / d[i];
+    double rl = vls::pivot_remainder(d[i], rh);
+    for (int k = 0; k < std::abs(rlUlps); k++) rl = std::nextafter(rl, rlUlps > 0 ? HUGE_VAL : -HUGE_VAL);
+    proven[i] = vls::pivot_division_exact(d[i], rh, rl);
+    int64_t bad = 0;
+    for (int64_t k = 0; k < samples; k++) {
+      const uint64_t r = next(), e = next();
+      double a = std::ldexp(1.0 + (double)(r & ((1ull << 52) - 1)) / 4503599627370496.0,
+                            (int)(e % 1801) - 900);
+      if (r >> 63) a = -a;
+      bad += vls::div_pivot(a, rh, rl) != a / d[i];
+    }
+    uint64_t odd;
+    int t;
+    vls::significand(d[i], odd, t);
+    if (odd != 1)
+      (void)vls::nearest_to_ties(odd, t, [&](double a) {
+        bad += vls::div_pivot(a, rh, rl) != a / d[i];
+        return true;
+      });
+    mismatches[i] = bad;
+  }
+  return VLS_OK;
+}
+
 int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vls_ctx **out) {
   if (!out) return fail(VLS_ERR_ARG, "null output pointer");
   *out = nullptr;

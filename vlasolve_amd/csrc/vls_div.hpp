@@ -44,7 +44,8 @@ VLS_HD inline double div_known(double a, double b, double yb) {
 // first of these distances, at most two significands A with
 // 2^53 A or 2^54 A = +-2^t (mod D); pivot_division_exact solves for them and
 // compares the result with a / d there, which makes the rounding proven for a
-// given d (no intermediate may underflow, as above).  An elimination row is a
+// given d (no intermediate may underflow, as above: a rl is subnormal for a
+// below about 2^-968).  An elimination row is a
 // chain of dependent operations: c16 y, the subtraction, and 2 here against 5
 // of div_known (one FP64 operation: 7 to 9 cycles).  At 129x129x64 k_line_rows
 // went from 15.0 to 13.8 us, k_line from 9.4 to 8.8, the column splines with
@@ -53,17 +54,11 @@ VLS_HD inline double div_pivot(double a, double rh, double rl) { return std::fma
 
 inline double pivot_remainder(double d, double rh) { return std::fma(-d, rh, 1.0) / d; }
 
-// Whether div_pivot(a, rh, rl) is RN(a / d) for every a (host).
-inline bool pivot_division_exact(double d, double rh, double rl) {
-  int e = 0;
-  uint64_t D = (uint64_t)std::ldexp(std::frexp(std::fabs(d), &e), 53), odd = D;
-  int t = 0;
-  while (!(odd & 1)) odd >>= 1, t++;
-  if (odd == 1) return rl == 0.0;  // a power of two: a * rh is exact
-  // 4 |rl d| D bounds the error in units of 1 / (2 D) ulp: below 2^t no
-  // numerator is near enough to a midpoint, below 3 2^t only the first ones
-  if (4.0 * std::fabs(rl * d) * (double)D < std::ldexp(1.0, t)) return true;
-  if (!(4.0 * std::fabs(rl * d) * (double)D < 3.0 * std::ldexp(1.0, t))) return false;
+// Calls fn(a) for the 53-bit significands a whose quotient a / d lies at the
+// first distance from a midpoint; false if fn returned false, or for too many
+// of them (d with few significant bits).  D = 2^t odd is d's significand.
+template <class F>
+inline bool nearest_to_ties(uint64_t odd, int t, F fn) {
   typedef unsigned __int128 u128;
   // inverse of 2^k modulo the odd part of D
   auto inv_pow2 = [&](int k) {
@@ -79,13 +74,36 @@ inline bool pivot_division_exact(double d, double rh, double rl) {
       uint64_t A = a0 >= lo ? a0 : a0 + (lo - a0 + odd - 1) / odd * odd;
       int tried = 0;
       for (; A < hi; A += odd) {
-        if (++tried > 4096) return false;  // d with few significant bits: not proven here
-        const double a = (double)A;
-        if (div_pivot(a, rh, rl) != a / d) return false;
+        if (++tried > 4096) return false;
+        if (!fn((double)A)) return false;
       }
     }
   }
   return true;
+}
+// d's 53-bit significand, its odd part and the power of two in it
+inline uint64_t significand(double d, uint64_t &odd, int &t) {
+  int e = 0;
+  const uint64_t D = (uint64_t)std::ldexp(std::frexp(std::fabs(d), &e), 53);
+  odd = D;
+  t = 0;
+  while (!(odd & 1)) odd >>= 1, t++;
+  return D;
+}
+
+// Whether div_pivot(a, rh, rl) is RN(a / d) for every a (host).  The bounds
+// below are those of rh, rl as the set-up makes them: others are refused.
+inline bool pivot_division_exact(double d, double rh, double rl) {
+  if (!std::isnormal(d) || rh != 1.0 / d || rl != pivot_remainder(d, rh)) return false;
+  uint64_t odd;
+  int t;
+  const uint64_t D = significand(d, odd, t);
+  if (odd == 1) return rl == 0.0;  // a power of two: a * rh is exact
+  // 4 |rl d| D bounds the error in units of 1 / (2 D) ulp: below 2^t no
+  // numerator is near enough to a midpoint, below 3 2^t only the first ones
+  if (4.0 * std::fabs(rl * d) * (double)D < std::ldexp(1.0, t)) return true;
+  if (!(4.0 * std::fabs(rl * d) * (double)D < 3.0 * std::ldexp(1.0, t))) return false;
+  return nearest_to_ties(odd, t, [&](double a) { return div_pivot(a, rh, rl) == a / d; });
 }
 
 }  // namespace vls
