@@ -1714,14 +1714,17 @@ k_stats_sums(const double *__restrict__ part, double *__restrict__ dM, double *_
 // same line again.  The serial sums run on values that the block has brought
 // into LDS (x: nR doubles, and 6 nJ where staged), and the shells' terms of the potential
 // energy, a division each, are formed by all threads between its two chains.
+// xg: x in memory instead, for more radii than the 160 KB of LDS have room for.
+constexpr int kStatsRadii = 16000;
+template <bool kGlobal>
 __global__ void __launch_bounds__(256)
 k_stats_line(const double *__restrict__ dM, const double *__restrict__ q,
              const double *__restrict__ R_Val, double G, double *__restrict__ out, int nR, int nJ,
-             int nS, int staged) {
-  extern __shared__ double x[];
+             int nS, int staged, double *xg) {
+  extern __shared__ double xl[];
   __shared__ double tot[6], mass, pot;
   const int t = threadIdx.x;
-  double *xq = x + nR;
+  double *x = kGlobal ? xg : xl, *xq = kGlobal ? xl : xl + nR;
   for (int r = t; r < nR; r += 256) x[r] = dM[r];
   if (staged)
     for (int i = t; i < 6 * nJ; i += 256) xq[i] = q[i];
@@ -3028,9 +3031,12 @@ void launch_stats(Run &r, hipStream_t s) {
   hipLaunchKernelGGL(k_stats_sums, dim3(nQ + (r.nR + 63) / 64), dim3(256), 0, s, r.st_part, dM,
                      r.st_q, r.nR, r.nJ, nQ);
   const bool staged = 6 * (size_t)r.nJ * sizeof(double) <= 32768;
-  hipLaunchKernelGGL(k_stats_line, dim3(1), dim3(256),
-                     (r.nR + (staged ? 6 * (size_t)r.nJ : 0)) * sizeof(double), s, dM, r.st_q,
-                     r.R_Val, r.sp.G, r.st_out, r.nR, r.nJ, r.nS, staged ? 1 : 0);
+  // (the partials have been added up: their first nR doubles are free)
+  const bool global = r.nR > kStatsRadii;
+  hipLaunchKernelGGL(global ? k_stats_line<true> : k_stats_line<false>, dim3(1), dim3(256),
+                     ((global ? 0 : r.nR) + (staged ? 6 * (size_t)r.nJ : 0)) * sizeof(double), s,
+                     dM, r.st_q, r.R_Val, r.sp.G, r.st_out, r.nR, r.nJ, r.nS, staged ? 1 : 0,
+                     r.st_part);
 }
 
 }  // namespace vls
