@@ -928,14 +928,10 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
     VLS_HIP_CHECK(hipStreamSynchronize(s));
     drop_graph(ctx->c);
     dfree(r, r.ch_point);
-    dfree(r, r.ch_off);
     dfree(r, r.ch_len);
-    dfree(r, r.ch_head);
     dfree(r, r.ch_xr);
-    dfree(r, r.ch_xu);
     dfree(r, r.ch_out);
     dfree(r, r.ch_vals);
-    dfree(r, r.ch_start);
     r.adj.recorded = false;
     r.adj.tilesValid = false;  // the transposed foot table lists the back cells
     r.nChains = nChains;
@@ -946,12 +942,15 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
     r.hch_xr.assign(back_xr, back_xr + nChains);
     r.hch_xu.assign(back_xu, back_xu + nChains);
     r.hch_out.assign(back_out, back_out + nChains);
-    r.ch_point = dalloc<int64_t>(r, nChains);
-    r.ch_off = dalloc<int64_t>(r, nChains);
-    r.ch_len = dalloc<int32_t>(r, nChains);
-    r.ch_head = dalloc<int32_t>(r, nChains);
-    r.ch_xr = dalloc<double>(r, nChains);
-    r.ch_xu = dalloc<double>(r, nChains);
+    // the tables of a type share an allocation (50 us each on their own)
+    r.ch_point = dalloc<int64_t>(r, 2 * nChains);
+    r.ch_off = r.ch_point + nChains;
+    r.ch_len = dalloc<int32_t>(r, 3 * nChains + r.nJ + 1);
+    r.ch_head = r.ch_len + nChains;
+    r.ch_order = r.ch_head + nChains;
+    r.ch_start = r.ch_order + nChains;
+    r.ch_xr = dalloc<double>(r, 2 * nChains);
+    r.ch_xu = r.ch_xr + nChains;
     r.ch_out = dalloc<uint8_t>(r, nChains);
     r.ch_vals = dalloc<double>(r, cells * r.nS);
     h2d(r.ch_point, point, nChains, s);
@@ -969,11 +968,8 @@ int vls_set_chains(vls_ctx *ctx, int run, int64_t nChains, const int64_t *point,
     for (int j = 0; j < r.nJ; j++) start[j + 1] += start[j];
     std::vector<int32_t> at(start.begin(), start.end() - 1);
     for (int64_t k = 0; k < nChains; k++) order[at[point[k] / nSlice]++] = (int32_t)k;
-    r.ch_start = dalloc<int32_t>(r, r.nJ + 1 + nChains);
-    r.ch_order = r.ch_start + r.nJ + 1;
-    start.insert(start.end(), order.begin(), order.end());
+    h2d(r.ch_order, order.data(), order.size(), s);
     h2d(r.ch_start, start.data(), start.size(), s);
-    VLS_HIP_CHECK(hipStreamSynchronize(s));  // start goes out of scope
     if (r.nS > 1) {
       std::vector<double> planes = to_planes(vals, cells, r.nS);
       h2d(r.ch_vals, planes.data(), planes.size(), s);
