@@ -5,7 +5,8 @@ with downloads (synchronisations) between them, and with the graph off."""
 import numpy as np
 import pytest
 
-from tests.configs import UDF_TINY, UDF_ODD, HERNQUIST_SMALL, PLDF_SMALL
+from tests.configs import (HERNQUIST_SMALL, PLDF_SMALL, UDF_2SPECIES_DELAYED, UDF_C1, UDF_NOLINK,
+                           UDF_ODD, UDF_TINY)
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +40,22 @@ def test_ensemble_runs_match_single_runs(graph):
             fa = alone(cfg, done)
             bad = np.count_nonzero(fe != fa)
             assert bad == 0, f"run {i} after {done} steps: {bad} points differ"
+
+
+def test_calls_of_one_and_more_steps():
+    """The captured first and last steps of a call, with and without linking
+    and species, beside runs whose steps are all alike (one too wide for the
+    slice step): calls of one step, two and several."""
+    cfgs = [UDF_NOLINK, UDF_2SPECIES_DELAYED, UDF_C1,
+            dict(UDF_C1, **{"grid.Pres": 150, "grid.Ures": [131, 3]})]
+    print(f"case ensemble of {len(cfgs)}, calls of 1, 1, 2 and 4 steps", flush=True)
+    e = V.Ensemble(cfgs)
+    ones = [V.Solver(cfg) for cfg in cfgs]
+    ctx = e.context
+    for k in (1, 1, 2, 4, 1):
+        e.step(k)
+        for i, s in enumerate(ones):
+            s.step(k)
+            f = ctx.download_f(i, s.shape)
+            assert np.array_equal(f, s.f()), (i, k)
+            assert all(np.array_equal(a, b) for a, b in zip(ctx.get_chains(i), s.context.get_chains()))

@@ -389,8 +389,9 @@ void build_ensemble_graph(vls::Context &C, int which) {
     for (int k = 0; k < n; k++) {
       VLS_HIP_CHECK(hipStreamWaitEvent(C.runStreams[k], C.forkEv, 0));
       if (vls::slice_on(C.runs[k])) {
+        if (which & vls::Context::kFirst) vls::launch_slice_start(C.runs[k], C.runStreams[k]);
         vls::launch_slice_kick(C.runs[k], C.runStreams[k], nullptr);
-        vls::launch_slice_drift(C.runs[k], C.runStreams[k], which == 1);
+        vls::launch_slice_drift(C.runs[k], C.runStreams[k], which & vls::Context::kLast);
       } else
         step_once(C.runs[k], C.runStreams[k], nullptr);
       VLS_HIP_CHECK(hipEventRecord(C.joinEv[k], C.runStreams[k]));
@@ -1027,13 +1028,11 @@ int vls_step(vls_ctx *ctx, int nSteps) {
     if (C.runs.size() > 1 && C.graphOn && !t->on) {
       // an ensemble: the runs advance concurrently, one graph launch a step
       bool slices = false;
-      for (auto &r : C.runs)
-        if (nSteps > 0 && vls::slice_on(r)) {
-          vls::launch_slice_start(r, s);
-          slices = true;
-        }
+      for (auto &r : C.runs) slices = slices || vls::slice_on(r);
       for (int n = 0; n < nSteps; n++) {
-        const int which = slices && n + 1 == nSteps;
+        int which = 0;
+        if (slices && n == 0) which |= vls::Context::kFirst;
+        if (slices && n + 1 == nSteps) which |= vls::Context::kLast;
         if (!C.graph[which]) build_ensemble_graph(C, which);
         VLS_HIP_CHECK(hipGraphLaunch(C.graph[which], s));
       }
