@@ -76,7 +76,8 @@ def test_slice_step_against_kernels_per_phase(monkeypatch):
 
 @pytest.mark.parametrize("grid,by_slice", [
     ((64, 64, 256), True), ((64, 64, 257), False), ((32, 32, 1024), False),
-    ((128, 32, 170), True), ((128, 32, 171), False), ((40, 35, 320), True), ((40, 35, 321), False),
+    ((128, 32, 170), True), ((128, 32, 171), False), ((40, 35, 512), True), ((40, 35, 513), False),
+    ((32, 48, 512), True), ((48, 32, 256), True), ((48, 32, 257), False),
     ((139, 32, 213), True), ((139, 32, 214), False), ((299, 24, 102), True), ((299, 24, 103), False)])
 def test_slice_step_is_for_slices_that_fill_the_chip_once(grid, by_slice):
     """The grids that go by slice, at both sides of the bounds on the slices

@@ -174,7 +174,7 @@ struct Context {
   // runs with the slice step (without such runs graph[0] serves for all).  What
   // precedes the first step is captured with it, so that the runs do it side by
   // side: launched one after the other on the context's stream it made calls
-  // of one step slower (4 runs of 65x65x32 130 us a call, captured 95)
+  // of one step slower (4 runs of 65x65x32 130 us a call, captured 86)
   static constexpr int kFirst = 1, kLast = 2;
   hipGraphExec_t graph[4] = {};
   bool graphOn = true;

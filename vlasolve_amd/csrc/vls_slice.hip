@@ -1147,24 +1147,28 @@ bool slice_fits(const Run &r) {
 }
 
 // Whether a run's steps go by slice unless it is told otherwise.  Every block
-// of the kick sums the partials of all slices, and past one round of the
+// of the kick sums the moment partials of all slices, and past a round of the
 // drift (a block fills a CU's registers) or two of the kick (two blocks on a
 // CU) the kernels per phase fill the chip as well.  us a step, by slice and
 // per phase:
 //   slices: 65x65x256 38, 53 and x300 67, 56; x1024 216, 115; 17x17x4096 428,
-//     72; 97x97x256 61, 73; 91x81x320 92, 86; where a tile holds all columns and
-//     the lines have no register kernels a little further: 50x50x320 45, 50;
-//   blocks of the kick: register lines win there (193x65x128, 512 blocks, 59,
-//     65; 129x129x160, 480, 76, 80; x192, 576, 94, 87; 193x65x150, 600, 83,
-//     72), other lines past 640 or where rows are long (150x100x200, 600,
-//     92, 102; 181x81x200, 600, 95, 100; 225x60x192, 768, 97, 93;
-//     300x49x100, 500, 69, 80 but x128, 640, 94, 88; 257x57x256 149, 123);
-//     with a second drift or species past 768 (129x129x256, 768, without
-//     linking 146, 159, two species 184, 205; 97x97x300, two species, 182, 159).
+//     72; 97x97x256 61, 73; 91x81x320 92, 86.  Where a tile of the kick holds
+//     all columns a second round pays too, unless the columns are short and
+//     have register kernels: 50x50x512 51, 61; 33x65x512 46, 51 and x600 71,
+//     56; 49x49x512 50, 54 and x600 77, 59; but 49x33x400 43, 40; 33x33x512
+//     40, 38 (two species 63, 75);
+//   blocks of the kick: register lines win up to 512 (193x65x128, 512, 59, 65;
+//     129x129x160, 480, 76, 80; x192, 576, 94, 87; 193x65x150, 600, 83, 72),
+//     others to 640 unless rows are long (150x100x200, 600, 92, 102;
+//     181x81x200, 600, 95, 100; 225x60x192, 768, 97, 93; 300x49x100, 500, 69,
+//     80 but x128, 640, 94, 88; 257x57x256 149, 123); with a second drift or
+//     species to 768 (129x129x256, 768, without linking 146, 159, two
+//     species 184, 205).
 bool slice_pays(const Run &r) {
   const int W = kick_width(r), nT = (r.nR + W - 1) / W;
   const bool lines = register_lines(r), twice = r.nS > 1 || r.sp.no_linking;
-  if (r.nJ > (nT == 1 && !lines ? 320 : 256)) return false;
+  const bool rounds = nT == 1 && (!lines || r.nU >= 49 || r.nS > 1);
+  if (r.nJ > (rounds ? 512 : 256)) return false;
   return r.nJ * nT <= (twice ? 768 : lines || nT > 3 ? 512 : 640);
 }
 
