@@ -158,11 +158,14 @@ int vls_kernel_times(vls_ctx *ctx, const char **names, double *ms, int *n);
  * and keeps the fastest -- register lines (shapes that have them), or the
  * LDS-tiled solvers with the tile size chosen from a set of candidates, line
  * tiles or the streaming solvers, for each direction -- then the kick's
- * schedules on a copy of f, then whole steps against the slice step.  run = -1 tunes every run of the context.  Every
- * schedule runs the same operations in the same order: the choice changes
- * the time of a step, never its bits.  Choices are cached per grid shape for
- * the life of the process; desc (may be NULL) receives one line per run
- * describing them with the measured times.  No counterpart in the reference,
+ * schedules on a copy of f, then whole steps against the slice step (for one
+ * species and a run that has the GPU for itself; otherwise the sizes decide).
+ * run = -1 tunes every run of the context.  Every schedule runs the same
+ * operations in the same order: the choice changes the time of a step, never
+ * its bits.  Choices are cached for the life of the process, per grid shape,
+ * species, linking and whether the streaming kick is open to the run; desc
+ * (may be NULL) receives one line per run describing them with the measured
+ * times.  No counterpart in the reference,
  * which runs one model per process with a fixed schedule. */
 int vls_autotune(vls_ctx *ctx, int run, char *desc, int descLen);
 

@@ -944,7 +944,10 @@ void launch_adj_spline(Run &r, double *cb, double *out, hipStream_t s) {
   else
     hipLaunchKernelGGL(k_adj_v, gv, dim3(64), 0, s, cb, r.nR + 2, r.cs, r.tv);
   // short rows are faster in registers (65x65x32: a reverse step 49 us, by
-  // tiles 50.5; 129x129x64: rows 18, by tiles 14)
+  // tiles 50.5).  The one longer shape with register kernels, 129x129, is
+  // faster by tiles for any number of slices (a reverse step with its share
+  // of the transfers, registers and tiles: x16 74, 69 us; x64 95, 90; x128
+  // 135, 132; x256 207, 204)
   if (!(a && r.nR <= 65) && adj_line_tile(r, true))
     launch_adj_line_tile(r, true, a != nullptr, cb, out, s);
   else if (a)

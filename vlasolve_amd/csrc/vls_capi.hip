@@ -718,7 +718,7 @@ int vls_create(const vls_geometry *g, const vls_solver_params *sp, int nRuns, vl
       r.hU.assign(G.U_Val, G.U_Val + r.nU);
       r.Ulo = G.U_Val[0];
       r.Uhi = G.U_Val[r.nU - 1];
-      r.cus = (int)(256 * (int64_t)r.nJ / slices);
+      r.cus = (int)(vls::kCUs * (int64_t)r.nJ / slices);
       vls::configure_tiles(r, maxLds);
       // the kick folded into the r-solve and the streaming kick leave the solved
       // rows (c's layout) in f's buffer between the kick and the drift

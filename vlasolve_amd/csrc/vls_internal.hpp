@@ -12,6 +12,9 @@
 
 namespace vls {
 
+// Compute units of an MI355X, which the rules of the schedules count on.
+constexpr int kCUs = 256;
+
 // Data-independent part of the natural cubic B-spline Thomas solve along one
 // axis (localSpline::create_1D with BT_NATURAL at both ends,
 // src/localSpline.hxx:953-1182).  The reference rebuilds these numbers in
@@ -100,7 +103,7 @@ struct Run {
   double *dM = nullptr, *Mx = nullptr, *acc = nullptr, *mTot = nullptr;
   bool lineTiles = false;  // lines may go by tiles (the pivots, and no schedule forced)
   bool pivots = false;  // the axes have the pivots that vls_slice.hip has as literals
-  int cus = 256;  // the compute units the run may count on (an ensemble's runs share them)
+  int cus = kCUs;  // the compute units the run may count on (an ensemble's runs share them)
   // slice step: the kicked f where several blocks share a slice, their group
   // sums of the moment and their counters (zero between launches)
   double *sliceF = nullptr, *sliceG = nullptr;

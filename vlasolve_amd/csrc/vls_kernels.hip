@@ -1681,7 +1681,7 @@ k_stats_sums(const double *__restrict__ part, double *__restrict__ dM, double *_
     if (w == 0 && s0 + lane < nSum) q[s0 + lane] = s;
     return;
   }
-  // the chunks' sums, up to 64 chunks at a time, then their serial sum
+  // the chunks' sums, up to 16 chunks at a time, then their serial sum
   const int r = (blockIdx.x - nQ) * 64 + lane, rc = min(r, nR - 1);
   const int nC = (nJ + kJC - 1) / kJC;
   double *S = &L[0][0];  // [16][64]
@@ -2491,8 +2491,7 @@ static void launch_spline_r(Run &r, const double *src, double *dst, hipStream_t 
   }
 }
 
-// rowsIn: the r-solved rows in c's layout (null: in c, solved in place;
-// otherwise register lines only)
+// rowsIn: the r-solved rows in c's layout (null: in c, solved in place)
 static void launch_spline_v(Run &r, const double *rowsIn, hipStream_t s) {
   if (const LineShape *ls = line_shape(r)) {
     hipLaunchKernelGGL(ls->cols, dim3((r.nR + 2 + 63) / 64 * r.nJ), dim3(64), 0, s, rowsIn, r.c,
@@ -2781,7 +2780,7 @@ std::string autotune(Run &r, hipStream_t s, int maxLds) {
   // the GPU has its blocks laid out for its share: alone on an idle GPU the
   // slice step looks slower than it is (32 runs of 65 to 257 points: 1270 us
   // a step by the sizes, 1310 by such times).
-  const bool timeSlice = r.nS == 1 && r.cus == 256 && slice_fits(r);
+  const bool timeSlice = r.nS == 1 && r.cus == kCUs && slice_fits(r);
   auto slice_by_size = [&](Sched &c) {
     c.slice = slice_fits(r) && slice_pays(r);
     c.stepUs = c.sliceUs = 0;

@@ -1168,8 +1168,8 @@ bool slice_pays(const Run &r) {
   const int W = kick_width(r), nT = (r.nR + W - 1) / W;
   const bool lines = register_lines(r), twice = r.nS > 1 || r.sp.no_linking;
   const bool rounds = nT == 1 && (!lines || r.nU >= 49 || r.nS > 1);
-  if (r.nJ > (rounds ? 512 : 256)) return false;
-  return r.nJ * nT <= (twice ? 768 : lines || nT > 3 ? 512 : 640);
+  if (r.nJ > (rounds ? 2 : 1) * kCUs) return false;
+  return r.nJ * nT <= (twice ? 3 * kCUs : lines || nT > 3 ? 2 * kCUs : 5 * kCUs / 2);
 }
 
 bool slice_on(const Run &r) {
@@ -1296,8 +1296,8 @@ void choose_line_tiles(Run &r) {
   const int wr = line_tile_width(r, true), wv = line_tile_width(r, false);
   auto blocks = [&](int lines, int w) { return (int64_t)(lines + w - 1) / w * r.nJ; };
   r.tileR = wr > 0 && ((r.nR + 4) * sizeof(double) * 20 <= kLineKB * 1024 ||
-                       blocks(r.nU, wr) <= 4 * 256);
-  r.tileV = wv > 0 && blocks(r.nR + 2, wv) <= 3 * 256;
+                       blocks(r.nU, wr) <= 4 * kCUs);
+  r.tileV = wv > 0 && blocks(r.nR + 2, wv) <= 3 * kCUs;
   r.tileK = !r.kept && tile_lines(r.nU, r.nR, kick_tile_other(r), kKickKB) > 0;
 }
 
@@ -1334,7 +1334,7 @@ static int adj_tile_width(const Run &r, bool rows) {
 // (18 against 14).
 bool adj_line_tile(const Run &r, bool rows) {
   const int w = r.lineTiles ? adj_tile_width(r, rows) : 0, lines = rows ? r.nU : r.nR + 2;
-  return w > 0 && (int64_t)(lines + w - 1) / w * r.nJ <= 4 * 256;
+  return w > 0 && (int64_t)(lines + w - 1) / w * r.nJ <= 4 * kCUs;
 }
 
 void launch_adj_line_tile(const Run &r, bool rows, bool fused, double *cb, double *out,
